@@ -14,7 +14,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libfem_amd.so")
 SOURCES = ["fem_host.cpp", "fem_device.hip", "plate_fused.hip", "adjoint.hip", "batch.hip", "bar_owner.hip",
-           "separate.hip", "plate_blocks.hip", "plate_corners.hip", "plate_lanes.hip", "solve.hip",
+           "separate.hip", "plate_blocks.hip", "plate_corners.hip", "plate_lanes.hip", "plate_frames.hip", "solve.hip",
            "forces.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("FEM_AMD_ARCH", "gfx950")

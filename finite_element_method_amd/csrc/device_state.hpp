@@ -50,6 +50,12 @@ struct Device {
   // the three values go to the kernel as arguments
   bool pl_uniform = false;
   double pl_mat[3] = {0.0, 0.0, 0.0};
+  // maps of plates in frames of their own (generic path of plate-only meshes);
+  // pn_waves == 0: the generic path sums element contributions
+  int pn_waves = 0;
+  uint32_t *pn_eid = nullptr, *pn_nodes = nullptr, *pn_wave = nullptr, *pn_lanes = nullptr;
+  double* pn_geo = nullptr;   // per wave element slot: local coordinates, parameters, frame
+  bool pn_geo_dirty = false;  // coordinates, frames or parameters changed since pn_geo was filled
   // bar owner maps
   uint32_t* bo_bid[2] = {nullptr, nullptr};
   uint64_t* bo_bmask = nullptr;

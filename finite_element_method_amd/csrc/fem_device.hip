@@ -8,10 +8,13 @@
 //   row_ptr  6N + 1 int64, col_idx nnz int32, val nnz double  (CSR)
 //
 // Value paths (both deterministic, no atomics; every CSR slot is written once):
-//   generic      : items (element, node pair) write their structural entries
-//                  into a contribution buffer; slots then sum their
-//                  contributions in element-insertion order (a sorted,
-//                  segmented reduction through a precomputed slot map).
+//   generic      : meshes of plates only, with frames of their own: one lane
+//                  per owned node-pair block (plate_frames.hip).  Mixed
+//                  meshes and those past its limits: items (element, node
+//                  pair) write their structural entries into a contribution
+//                  buffer; slots then sum their contributions in
+//                  element-insertion order (a sorted, segmented reduction
+//                  through a precomputed slot map).
 //   plate_fused  : one workgroup per patch of owned nodes; element kinematics
 //                  are staged in LDS and each owned CSR row block is summed in
 //                  registers and written once (see plate_fused_kernel).
@@ -64,6 +67,7 @@ void destroy_device(Device* d) {
   f(d->sep_v); f(d->sep_flag); f(d->sep_pos); f(d->sep_key); f(d->sep_cnt); f(d->sep_off); f(d->sep_aa); f(d->sep_bb);
   f(d->sep_rp); f(d->sep_sum); f(d->sep_ci); f(d->sep_dpos);
   f(d->pb_hdr); f(d->pb_conn); f(d->pb_eid); f(d->pb_blk);
+  f(d->pn_eid); f(d->pn_nodes); f(d->pn_wave); f(d->pn_lanes); f(d->pn_geo);
   f(d->pl_nodes); f(d->pl_lanes); f(d->pl_lane_set); f(d->pl_geo);
   for (int k = 0; k < 6; ++k) f(d->sol_vec[k]);
   f(d->sol_rr); f(d->sol_rb); f(d->sol_part); f(d->sol_s); f(d->sol_diag); f(d->sol_inv); f(d->sol_flag);
@@ -181,7 +185,7 @@ std::string replace_params(Device* d, int type, const double* src, double* host_
   if (!n) return "";
   hipStream_t s = static_cast<hipStream_t>(stream);
   HIP_TRY(hipMemcpyAsync(d->params[type], src, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-  if (type == PLATE) d->pl_geo_dirty = true;
+  if (type == PLATE) d->pl_geo_dirty = d->pn_geo_dirty = true;
   else d->bo_slot_dirty = true;
   HIP_TRY(hipStreamSynchronize(s));
   HIP_TRY(hipMemcpy(host_copy, d->params[type], n * sizeof(double), hipMemcpyDeviceToHost));
@@ -193,7 +197,7 @@ std::string replace_nodes(Device* d, const double* src, double* host_copy, void*
   if (!n) return "";
   hipStream_t s = static_cast<hipStream_t>(stream);
   HIP_TRY(hipMemcpyAsync(d->xyz, src, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-  d->pl_geo_dirty = true;
+  d->pl_geo_dirty = d->pn_geo_dirty = true;
   d->bo_slot_dirty = true;
   HIP_TRY(hipStreamSynchronize(s));
   HIP_TRY(hipMemcpy(host_copy, d->xyz, n * sizeof(double), hipMemcpyDeviceToHost));
@@ -335,6 +339,7 @@ __global__ void slot_gather_kernel(const int64_t* __restrict__ slot_ptr, const u
 }
 
 std::string upload_generic(Device* d, const GenericMaps& g) {
+  d->pn_waves = 0;
   auto e = dupload(d->class_mask, g.class_mask.data(), g.class_mask.size());
   if (!e.empty()) return e;
   e = dupload(d->class_off, g.class_off.data(), g.class_off.size());
@@ -356,6 +361,7 @@ std::string upload_generic(Device* d, const GenericMaps& g) {
 void set_generic_block(Device* d, int threads) { d->gen_block = threads; }
 
 std::string assemble_generic(Device* d, double* val, void* stream, bool timed) {
+  if (d->pn_waves) return assemble_plate_frames(d, val, stream, timed);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const unsigned bs = unsigned(d->gen_block);
   if (timed) HIP_TRY(hipEventRecord(d->ev0, s));

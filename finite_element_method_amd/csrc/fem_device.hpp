@@ -131,6 +131,29 @@ std::string upload_plate_lane_maps(Device* d, const PlateLaneMaps& pm);
 std::string set_plate_lane_material(Device* d, bool uniform, const double mat[3]);
 std::string assemble_plate_lanes(Device* d, double* val, void* stream, bool timed = true);
 
+// Plates with frames of their own (plate_frames.hip): meshes of plates only in
+// which every node is in at most PN_ITEMS elements and the values span 32-bit
+// byte offsets.  One wave per patch of owned nodes, one lane per node-pair block.
+constexpr int PN_NODES = 16;           // owned nodes of a wave patch
+constexpr int PN_ELEMS = 16;           // elements touching a wave patch
+constexpr int PN_ITEMS = 8;            // contributions of a block
+constexpr int PN_STAGE_VALUES = 2320;  // staged values: 64 blocks of 36 and a parity pad per run
+struct PlateFrameMaps {
+  int n_waves = 0;
+  std::vector<uint32_t> seid;   // per wave PN_ELEMS element ids in insertion order (0xFFFFFFFF: unused)
+  // per wave PN_NODES x 2: CSR position of row 6a of owned node s, staging
+  // position (12 bits) | values of its six rows << 12
+  std::vector<uint32_t> nodes;
+  std::vector<uint32_t> waves;  // per wave x 2: its set in `lanes`, elements | nodes << 8 | trips << 16
+  // distinct descriptor sets, 64 lanes x 8 words: up to eight items of 8 bits
+  // (wave element | p << 4 | q << 6, insertion order); the block's structural
+  // mask (36 bits) | items << 36; six 16-bit staging positions of the block's
+  // rows; pad
+  std::vector<uint32_t> lanes;
+};
+std::string upload_plate_frame_maps(Device* d, const PlateFrameMaps& pm);
+std::string assemble_plate_frames(Device* d, double* val, void* stream, bool timed);
+
 // Corner-lane fused plate path (plate_corners.hip): same preconditions as the
 // maps above, every node in at most four elements, every off-diagonal node
 // pair in at most two, and each element corner sharing at most two of its
