@@ -99,7 +99,9 @@ struct Device {
   uint32_t *sol_flag = nullptr, *sol_bid = nullptr;
   int32_t* sol_starts = nullptr;
   uint8_t* sol_tmp = nullptr;
-  size_t sol_cap[16] = {};
+  uint32_t* sol_slice[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // K_aa's slices: rows, pairs, lowest columns, sizes, offsets
+  uint8_t* sol_slice_data = nullptr;                                       // and entries
+  size_t sol_cap[22] = {};
   int64_t sol_na = 0, sol_nb = 0;
   bool sol_done = false;
   double sol_ms = 0.0;

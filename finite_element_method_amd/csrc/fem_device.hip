@@ -72,6 +72,8 @@ void destroy_device(Device* d) {
   for (int k = 0; k < 6; ++k) f(d->sol_vec[k]);
   f(d->sol_rr); f(d->sol_rb); f(d->sol_part); f(d->sol_s); f(d->sol_diag); f(d->sol_inv); f(d->sol_flag);
   f(d->sol_bid); f(d->sol_starts); f(d->sol_tmp); f(d->u_glob);
+  for (int k = 0; k < 5; ++k) f(d->sol_slice[k]);
+  f(d->sol_slice_data);
   if (d->sol_host) { (void)hipHostFree(d->sol_host); d->sol_host = nullptr; }
   for (hipEvent_t ev : {d->ev0, d->ev1, d->ev2, d->ev3, d->ev4, d->ev5})
     if (ev) hipEventDestroy(ev);

@@ -119,6 +119,268 @@ __global__ void sv_spmv_it(const int64_t* __restrict__ rp, const int32_t* __rest
   if (lig == 0) ap[r] = acc;
 }
 
+// ---- K_aa in slices, for the update loop
+//
+// The CSR product above moves 12 bytes per entry and spends its memory
+// instructions on rows of 9 to 27 entries split over four lanes.  A solve that
+// goes on after its first update copies K_aa once into slices of 64 rows, a lane
+// per row:
+//   * every value load of a wave is 1 KiB of consecutive bytes;
+//   * a column takes 16 bits from the slice's lowest column while the slice spans
+//     under 2^16 columns, 32 bits otherwise;
+//   * rows are sorted by length within windows of SL_WINDOW rows, so that the
+//     lanes of a slice end together (a plate's rows of 18, 27 and 1 entries
+//     alternate).
+// A row's entries go to four partial sums, combined as sv_spmv_it_quad's four
+// lanes combine theirs, entry for entry: the product has the same bits, and the
+// rows' order in the slices does not show.
+//
+// Slice s, at its offset of 256-byte units: `pairs` x 64 value pairs (16 bytes a
+// lane), then `pairs` x 64 column pairs (4 bytes a lane, or 8).
+//
+// Bound: the entries' stream, 10.3 bytes per entry with the padding; on the
+// 512 x 512 plate (31 M entries) 78 us per product, 4.1 TB/s, against 106 us for
+// the CSR product; without the gathers of p it would take 62-68 us.  Measured and
+// left out: rows with equal columns sharing a lane (fewer columns and gathers,
+// but each gather then spans 64 nodes: 188 us), one 16-byte gather for two
+// neighbouring columns (87 us), an XCD-contiguous order of the slices (no change).
+constexpr int SL_WINDOW = 1024;  // rows sorted together, by one workgroup
+// The copy costs about two CSR products and a fixed 50 us.  From 10 M entries
+// on a solve of 20 updates gains it back (17 M entries: 2.04 vs 2.11 ms, 50
+// updates 4.47 vs 4.88; 7.7 M entries: 1.22 vs 1.16 ms, 50 updates 2.66 vs 2.64).
+constexpr int64_t SL_MIN_NNZ = 10000000;    // K_aa entries
+constexpr int SL_MIN_UPDATES = 16;          // updates asked for
+constexpr uint32_t SL_NONE = 0xFFFFFFFFu;   // no row in this lane
+constexpr uint32_t SL_UNITS16 = 5, SL_UNITS32 = 6;  // 256-byte units of a pair of 64 lanes
+
+__device__ inline uint32_t wave_min(uint32_t v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = min(v, uint32_t(__shfl_xor(int(v), o)));
+  return v;
+}
+__device__ inline uint32_t wave_max(uint32_t v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = max(v, uint32_t(__shfl_xor(int(v), o)));
+  return v;
+}
+
+// one workgroup per window: rows in order of (length, index); per slice its
+// pairs | wide << 31, lowest column and size in units.  Lengths are below 2^22
+// (the pattern's rows are bounded by 65535 plus a block).
+__global__ __launch_bounds__(512) void sv_slice_rows(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
+                                                     int64_t n, uint32_t* __restrict__ rows,
+                                                     uint32_t* __restrict__ pairs, uint32_t* __restrict__ cbase,
+                                                     uint32_t* __restrict__ units, int64_t n_slices) {
+  __shared__ uint32_t key[SL_WINDOW];
+  const int64_t w0 = int64_t(blockIdx.x) * SL_WINDOW;
+  for (int i = threadIdx.x; i < SL_WINDOW; i += 512) {
+    const int64_t r = w0 + i;
+    key[i] = r < n ? uint32_t(rp[r + 1] - rp[r]) << 10 | uint32_t(i) : SL_NONE;
+  }
+  __syncthreads();
+  for (int k = 2; k <= SL_WINDOW; k <<= 1)  // bitonic sort, ascending
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int t = threadIdx.x; t < SL_WINDOW / 2; t += 512) {
+        const int i = 2 * t - (t & (j - 1)), o = i + j;
+        const uint32_t a = key[i], b = key[o];
+        if ((a > b) == ((i & k) == 0)) {
+          key[i] = b;
+          key[o] = a;
+        }
+      }
+      __syncthreads();
+    }
+  const int lane = threadIdx.x & 63;
+  for (int q = threadIdx.x >> 6; q < SL_WINDOW / 64; q += 8) {
+    const int64_t s = int64_t(blockIdx.x) * (SL_WINDOW / 64) + q;
+    const uint32_t kk = key[64 * q + lane];
+    const bool on = kk != SL_NONE;
+    const int64_t r = w0 + int64_t(kk & (SL_WINDOW - 1));
+    const uint32_t len = on ? kk >> 10 : 0u;
+    uint32_t lo = SL_NONE, hi = 0u;
+    if (len) {  // columns ascend within a row
+      const int64_t b = rp[r];
+      lo = uint32_t(ci[b]);
+      hi = uint32_t(ci[b + len - 1]);
+    }
+    lo = wave_min(lo);
+    hi = wave_max(hi);
+    const uint32_t np = (wave_max(len) + 1u) >> 1;
+    if (s >= n_slices) continue;
+    rows[64 * s + lane] = on ? uint32_t(r) : SL_NONE;
+    if (lane == 0) {
+      const bool wide = np && hi - lo > 0xFFFFu;
+      pairs[s] = np | uint32_t(wide) << 31;
+      cbase[s] = np ? lo : 0u;
+      units[s] = np * (wide ? SL_UNITS32 : SL_UNITS16);
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) units[n_slices] = 0u;  // totals slot of the scan
+}
+
+// One wave per slice.  16 entries of each of 64 rows at a time go through LDS:
+// four lanes read a row's 16 entries together (range-checked 16-byte loads: what
+// lies past a row or the array is loaded but not kept), then each lane writes
+// the pairs of its own row, so that reads and writes both cover consecutive
+// bytes.  Unused places hold value 0 and the slice's lowest column.
+constexpr int SL_TILE = 17;
+__device__ inline void sl_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__global__ __launch_bounds__(256) void sv_slice_fill(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
+                                                     const double* __restrict__ v, const uint32_t* __restrict__ rows,
+                                                     const uint32_t* __restrict__ pairs,
+                                                     const uint32_t* __restrict__ cbase,
+                                                     const uint32_t* __restrict__ offset, int64_t n_slices,
+                                                     unsigned char* __restrict__ data, uint32_t v_bytes) {
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  __shared__ double tile_v[4][64 * SL_TILE];
+  __shared__ uint32_t tile_c[4][64 * SL_TILE];
+  const int64_t s = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (s >= n_slices) return;
+  const uint32_t pw = pairs[s], np = pw & 0x7FFFFFFFu, cb = cbase[s], r = rows[64 * s + lane];
+  const bool wide = pw >> 31;
+  double* tv = tile_v[threadIdx.x >> 6];
+  uint32_t* tc = tile_c[threadIdx.x >> 6];
+  const uint32_t first = r == SL_NONE ? 0u : uint32_t(rp[r]);  // positions are below 2^29
+  const uint32_t len = r == SL_NONE ? 0u : uint32_t(rp[r + 1]) - first;
+  double2* dv = reinterpret_cast<double2*>(data + size_t(offset[s]) * 256);
+  uint32_t* dc = reinterpret_cast<uint32_t*>(dv + 64 * size_t(np));
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(v), 0, int(v_bytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(ci), 0, int(v_bytes / 2u), 0x00020000);
+  for (uint32_t j0 = 0; j0 < np; j0 += 8) {
+    double2 x0[4], x1[4];
+    u32x4 cc[4];
+    uint32_t left[4];  // entries of the row from the lane's first on
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {  // 16 rows, one per four lanes
+      const int src = 16 * pass + (lane >> 2);
+      const uint32_t sl = uint32_t(__shfl(int(len), src)), e = 2 * j0 + 4 * (lane & 3);
+      const uint32_t at = uint32_t(__shfl(int(first), src)) + e;
+      left[pass] = e < sl ? sl - e : 0u;
+      x0[pass] = x1[pass] = make_double2(0.0, 0.0);
+      cc[pass] = u32x4{0u, 0u, 0u, 0u};
+      if (left[pass]) {
+        x0[pass] = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rv, 8u * at, 0, 0));
+        x1[pass] = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rv, 8u * at + 16u, 0, 0));
+        cc[pass] = __builtin_amdgcn_raw_buffer_load_b128(rc, 4u * at, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {
+      const int o = SL_TILE * (16 * pass + (lane >> 2)) + 4 * (lane & 3);
+      const uint32_t n = left[pass];
+      tv[o] = n > 0 ? x0[pass].x : 0.0;
+      tv[o + 1] = n > 1 ? x0[pass].y : 0.0;
+      tv[o + 2] = n > 2 ? x1[pass].x : 0.0;
+      tv[o + 3] = n > 3 ? x1[pass].y : 0.0;
+      tc[o] = n > 0 ? cc[pass].x - cb : 0u;
+      tc[o + 1] = n > 1 ? cc[pass].y - cb : 0u;
+      tc[o + 2] = n > 2 ? cc[pass].z - cb : 0u;
+      tc[o + 3] = n > 3 ? cc[pass].w - cb : 0u;
+    }
+    sl_lds_sync();
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j)
+      if (j0 + j < np) {
+        const double* t = tv + SL_TILE * lane + 2 * j;
+        const uint32_t c0 = tc[SL_TILE * lane + 2 * j], c1 = tc[SL_TILE * lane + 2 * j + 1];
+        dv[64 * size_t(j0 + j) + lane] = make_double2(t[0], t[1]);
+        if (wide)
+          reinterpret_cast<uint2*>(dc)[64 * size_t(j0 + j) + lane] = make_uint2(c0, c1);
+        else
+          dc[64 * size_t(j0 + j) + lane] = c0 | c1 << 16;
+      }
+    sl_lds_sync();
+  }
+}
+
+// N column pairs from pair j: all loads first, then pairs 0, 1 into partial sum
+// a and 2, 3 into b.  The entries are read once per product: non-temporal, so
+// that p keeps the caches (88 -> 78 us on the 512 x 512 plate).  Places past a
+// row's end are loaded (value 0) but not summed, so that an infinite or NaN
+// entry of p reaches only the rows that hold its column.
+template <bool WIDE, int N>
+__device__ inline void slice_pairs(const double2* __restrict__ dv, const uint32_t* __restrict__ dc,
+                                   const double* __restrict__ p, uint32_t j, uint32_t len, int lane, double& a,
+                                   double& b) {
+  typedef double sl_d2 __attribute__((ext_vector_type(2)));
+  typedef unsigned int sl_u2 __attribute__((ext_vector_type(2)));
+  sl_d2 w[N];
+  sl_d2 x[N];
+#pragma unroll
+  for (int t = 0; t < N; ++t) {
+    uint32_t c0, c1;
+    if (WIDE) {
+      const sl_u2 c = __builtin_nontemporal_load(reinterpret_cast<const sl_u2*>(dc) + 64 * size_t(j + t) + lane);
+      c0 = c.x;
+      c1 = c.y;
+    } else {
+      const uint32_t c = __builtin_nontemporal_load(dc + 64 * size_t(j + t) + lane);
+      c0 = c & 0xFFFFu;
+      c1 = c >> 16;
+    }
+    w[t] = __builtin_nontemporal_load(reinterpret_cast<const sl_d2*>(dv) + 64 * size_t(j + t) + lane);
+    x[t].x = p[c0];
+    x[t].y = p[c1];
+  }
+#pragma unroll
+  for (int t = 0; t < N; ++t) {
+    double& acc = t < 2 ? a : b;
+    if (2 * (j + t) < len) acc = __builtin_fma(w[t].x, x[t].x, acc);
+    if (2 * (j + t) + 1 < len) acc = __builtin_fma(w[t].y, x[t].y, acc);
+  }
+}
+
+template <bool WIDE>
+__device__ inline double slice_row(const double2* __restrict__ dv, const uint32_t* __restrict__ dc,
+                                   const double* __restrict__ p, uint32_t np, uint32_t len, int lane) {
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+  uint32_t j = 0;
+  // four pairs (two quads of columns) into two partial sums; false after the
+  // last ones.  np is the slice's, so the whole wave takes the same way.
+  auto chunk = [&](double& a, double& b) -> bool {
+    const uint32_t left = np - j;
+    if (left < 4) {
+      if (left == 1) slice_pairs<WIDE, 1>(dv, dc, p, j, len, lane, a, b);
+      if (left == 2) slice_pairs<WIDE, 2>(dv, dc, p, j, len, lane, a, b);
+      if (left == 3) slice_pairs<WIDE, 3>(dv, dc, p, j, len, lane, a, b);
+      return false;
+    }
+    slice_pairs<WIDE, 4>(dv, dc, p, j, len, lane, a, b);
+    j += 4;
+    return true;
+  };
+  while (chunk(a0, a1) && chunk(a2, a3)) {
+  }
+  return (a0 + a2) + (a1 + a3);
+}
+
+__global__ __launch_bounds__(256) void sv_spmv_slices(const unsigned char* __restrict__ data,
+                                                      const int64_t* __restrict__ rp,
+                                                      const uint32_t* __restrict__ rows,
+                                                      const uint32_t* __restrict__ pairs,
+                                                      const uint32_t* __restrict__ cbase,
+                                                      const uint32_t* __restrict__ offset, int64_t n_slices,
+                                                      const double* __restrict__ p, double* __restrict__ ap,
+                                                      const double* s) {
+  if (s[S_DONE] != 0.0) return;
+  const int64_t sl = int64_t(__builtin_amdgcn_readfirstlane(int(blockIdx.x * 4 + (threadIdx.x >> 6))));
+  const int lane = threadIdx.x & 63;
+  if (sl >= n_slices) return;
+  const uint32_t pw = pairs[sl], np = pw & 0x7FFFFFFFu, r = rows[64 * sl + lane];
+  const double2* dv = reinterpret_cast<const double2*>(data + size_t(offset[sl]) * 256);
+  const uint32_t* dc = reinterpret_cast<const uint32_t*>(dv + 64 * size_t(np));
+  const uint32_t len = r == SL_NONE ? 0u : uint32_t(rp[r + 1] - rp[r]);
+  const double* q = p + cbase[sl];
+  const double y = pw >> 31 ? slice_row<true>(dv, dc, q, np, len, lane) : slice_row<false>(dv, dc, q, np, len, lane);
+  if (r != SL_NONE) ap[r] = y;
+}
+
 // block tree sum of per-thread values into part[blockIdx.x]
 __device__ inline void block_sum2(double a, double b, double* part_a, double* part_b) {
   __shared__ double sa[SV_B], sb[SV_B];
@@ -454,10 +716,13 @@ unsigned grid_for(int64_t items, int per_block) { return unsigned(std::max<int64
 // Work buffers of one solve.  get(slot, bytes) returns device memory for a
 // slot; vectors: 0 b, 1 x = u_a, 2 r, 3 z, 4 p, 5 Ap, 6 r_r, 7 r_b; 8 the
 // reduction partials, 9 the scalars, 10 the Jacobi diagonal, 11 block flags,
-// 12 block ids, 13 block starts, 14 scan storage, 15 block inverses.
+// 12 block ids, 13 block starts, 14 scan storage, 15 block inverses; where
+// grows(), also K_aa's slices: 16 rows, 17 pairs, 18 lowest columns, 19 sizes,
+// 20 offsets, 21 entries.
 struct SolveBuffers {
   virtual std::string get(int slot, size_t bytes, void** out) = 0;
-  double* host = nullptr;  // S_COUNT doubles of host memory for the scalar reads
+  virtual bool grows() const { return false; }
+  double* host = nullptr;  // S_COUNT + 1 doubles of host memory for the scalar reads
 };
 
 namespace {
@@ -472,6 +737,48 @@ std::string take(SolveBuffers& bufs, int slot, size_t n, T*& out) {
   auto e = bufs.get(slot, std::max<size_t>(n, 1) * sizeof(T), &p);
   out = static_cast<T*>(p);
   return e;
+}
+
+// K_aa's slices (sv_spmv_slices): rows and sizes first, the entries once the
+// total size has been read
+struct Slices {
+  int64_t n = 0;
+  uint32_t *rows = nullptr, *pairs = nullptr, *cbase = nullptr, *units = nullptr, *offset = nullptr;
+  unsigned char* data = nullptr;
+};
+
+std::string slices_size(SolveBuffers& bufs, const int64_t* rp, const int32_t* ci, int64_t na, hipStream_t s,
+                        Slices& sl) {
+  sl.n = (na + 63) / 64;
+  const size_t un = size_t(sl.n);
+  std::string e;
+  if (!(e = take(bufs, 16, 64 * un, sl.rows)).empty()) return e;
+  if (!(e = take(bufs, 17, un, sl.pairs)).empty()) return e;
+  if (!(e = take(bufs, 18, un, sl.cbase)).empty()) return e;
+  if (!(e = take(bufs, 19, un + 1, sl.units)).empty()) return e;
+  if (!(e = take(bufs, 20, un + 1, sl.offset)).empty()) return e;
+  size_t bytes = 0;
+  HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, sl.units, sl.offset, int(un + 1), s));
+  void* tmp = nullptr;
+  if (!(e = bufs.get(14, std::max<size_t>(bytes, 1), &tmp)).empty()) return e;
+  sv_slice_rows<<<grid_for(na, SL_WINDOW), 512, 0, s>>>(rp, ci, na, sl.rows, sl.pairs, sl.cbase, sl.units, sl.n);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, sl.units, sl.offset, int(un + 1), s));
+  return "";
+}
+
+// false (and no error left behind) when there is no memory for the entries
+bool slices_fill(SolveBuffers& bufs, const int64_t* rp, const int32_t* ci, const double* v, uint32_t v_bytes,
+                 uint32_t units, hipStream_t s, Slices& sl) {
+  void* data = nullptr;
+  if (!bufs.get(21, size_t(units) * 256, &data).empty() || !data) {
+    (void)hipGetLastError();
+    return false;
+  }
+  sl.data = static_cast<unsigned char*>(data);
+  sv_slice_fill<<<grid_for(sl.n, 4), 256, 0, s>>>(rp, ci, v, sl.rows, sl.pairs, sl.cbase, sl.offset, sl.n, sl.data,
+                                                      v_bytes);
+  return hipGetLastError() == hipSuccess;
 }
 
 // the solve proper: b, preconditioner, PCG updates, r_r, into `bufs`
@@ -566,11 +873,17 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
     const bool quad = wide && size_t(d->sep_nnz[0]) * 8 < (size_t(1) << 32);
     const uint32_t v_bytes = quad ? uint32_t(size_t(d->sep_nnz[0]) * 8) : 0u;
     const unsigned spmv_blocks = grid_for(na * (quad ? SPMV_QUAD_LANES : SPMV_LANES), B);
+    Slices sl;
+    bool slice = quad && bufs.grows() && d->sep_nnz[0] >= SL_MIN_NNZ && max_iter >= SL_MIN_UPDATES;
+    uint32_t slice_total = 0;
     int queued = 0, batch = 1;
     for (;;) {
       const int nq = std::min(batch, max_iter - queued);
       for (int q = 0; q < nq; ++q) {
-        if (quad) sv_spmv_it_quad<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, v_bytes);
+        if (sl.data)
+          sv_spmv_slices<<<grid_for(sl.n, 4), 256, 0, s>>>(sl.data, rp[0], sl.rows, sl.pairs, sl.cbase, sl.offset,
+                                                           sl.n, p, ap, sc);
+        else if (quad) sv_spmv_it_quad<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, v_bytes);
         else sv_spmv_it<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc);
         sv_dot_it<<<SV_PARTS, B, 0, s>>>(p, ap, na, sc, pa);
         sv_final<<<1, 1024, 0, s>>>(pa, nullptr, sc, 1, stop, double(max_iter));
@@ -582,10 +895,20 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
         sv_direction<<<SV_PARTS, B, 0, s>>>(z, sc, na, p);
       }
       HIP_TRY(hipGetLastError());
+      const bool first = queued == 0;
       queued += nq;
+      if (slice && first) {
+        slice = slices_size(bufs, rp[0], ci[0], na, s, sl).empty();  // no memory: the solve goes on without
+        if (slice) HIP_TRY(hipMemcpyAsync(host + S_COUNT, sl.offset + sl.n, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        else (void)hipGetLastError();
+      }
       HIP_TRY(hipMemcpyAsync(host, sc, sizeof(double) * S_COUNT, hipMemcpyDeviceToHost, s));
       HIP_TRY(hipStreamSynchronize(s));
       if (host[S_DONE] != 0.0 || queued >= max_iter) break;
+      if (slice && first) {
+        std::memcpy(&slice_total, host + S_COUNT, sizeof(uint32_t));
+        if (!slices_fill(bufs, rp[0], ci[0], v[0], v_bytes, slice_total, s, sl)) sl.data = nullptr;
+      }
       batch = std::min(batch * 2, 64);
     }
     it = int(host[S_ITER]);
@@ -614,6 +937,7 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
 struct ModelBuffers : SolveBuffers {
   Device* d;
   explicit ModelBuffers(Device* dev) : d(dev) {}
+  bool grows() const override { return true; }
   std::string get(int slot, size_t bytes, void** out) override {
     std::string e;
     const size_t n8 = (bytes + 7) / 8, n4 = (bytes + 3) / 4;
@@ -627,7 +951,9 @@ struct ModelBuffers : SolveBuffers {
     else if (slot == 12) { e = dgrow(d->sol_bid, d->sol_cap[12], n4); *out = d->sol_bid; }
     else if (slot == 13) { e = dgrow(d->sol_starts, d->sol_cap[13], n4); *out = d->sol_starts; }
     else if (slot == 14) { e = dgrow(d->sol_tmp, d->sol_cap[14], bytes); *out = d->sol_tmp; }
-    else { e = dgrow(d->sol_inv, d->sol_cap[15], n8); *out = d->sol_inv; }
+    else if (slot == 15) { e = dgrow(d->sol_inv, d->sol_cap[15], n8); *out = d->sol_inv; }
+    else if (slot < 21) { e = dgrow(d->sol_slice[slot - 16], d->sol_cap[slot], n4); *out = d->sol_slice[slot - 16]; }
+    else { e = dgrow(d->sol_slice_data, d->sol_cap[21], bytes); *out = d->sol_slice_data; }
     return e;
   }
 };
@@ -706,7 +1032,7 @@ std::string solve_pcg_static(Device* d, int precond, int max_iter, double rel_to
   bufs.base = static_cast<unsigned char*>(base);
   bufs.u_a = u_a;
   bufs.r_r = r_r;
-  double host[S_COUNT];
+  double host[S_COUNT + 1];
   bufs.host = host;
   return solve_core(d, precond, max_iter, rel_tol, abs_tol, static_cast<hipStream_t>(stream), res, wide, bufs);
 }
