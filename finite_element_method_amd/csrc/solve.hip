@@ -8,9 +8,13 @@
 //
 // PCG is Saad's Algorithm 9.1 with x0 = 0, stopped when
 // ||r||_2 <= max(rel_tol ||b||_2, abs_tol) and counting the x updates.  All
-// reductions use a fixed grid and fixed trees, so a solve is bitwise
-// reproducible.  The scalars (alpha, beta, r.z) stay on the device; the host
-// reads r.r once per iteration for the stopping test.
+// reductions use a grid that depends on n only and fixed trees, so a solve is
+// bitwise reproducible.  The scalars (alpha, beta, r.z) stay on the device.
+//
+// An update is four launches: product, p.Ap, the vector update and the
+// direction.  The last two begin by summing the partial sums of the one before
+// in every workgroup (the same tree, so every workgroup has the same bits),
+// which takes the place of two one-workgroup launches per update.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -28,14 +32,15 @@ namespace femdev {
 namespace {
 
 constexpr int SV_B = 256;         // threads per block of the vector kernels
-constexpr int SV_PARTS = 1024;    // blocks of the reductions (fixed: reproducible sums)
+constexpr int SV_PARTS = 1024;    // most blocks of the reductions
 constexpr int SPMV_LANES = 8;     // lanes per CSR row
 constexpr int BJ_MAX = 6;         // dofs per node block
 
-// scalar slots (device): 0 r.z, 1 p.Ap, 2 alpha, 3 beta, 4 r.r, 5 (r.z)_new, 6 b.b, 7 status,
-// 8 updates done, 9 stop (converged or capped: every later kernel of the loop
-// returns at once), 10 converged
-enum { S_RZ = 0, S_PAP, S_ALPHA, S_BETA, S_RR, S_RZN, S_BB, S_STATUS, S_ITER, S_DONE, S_CONV, S_COUNT };
+// scalar slots (device).  r.z and the stop flag (converged or capped: every
+// later kernel of the loop returns at once) have two slots: update u reads slot
+// u & 1 and its last kernel writes the other, so that no workgroup reads what
+// another of the same launch writes.
+enum { S_RZ = 0, S_DONE = 2, S_RR = 4, S_BB, S_STATUS, S_ITER, S_CONV, S_COUNT };
 constexpr int BJ_PER_WAVE = 10;   // node blocks per wave in the block-Jacobi kernels (6 lanes each)
 
 template <class T>
@@ -76,9 +81,9 @@ __global__ void sv_spmv(const int64_t* __restrict__ rp, const int32_t* __restric
 constexpr int SPMV_QUAD_LANES = 4;
 __global__ void sv_spmv_it_quad(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
                                 const double* __restrict__ v, const double* __restrict__ p, double* __restrict__ ap,
-                                int64_t n, const double* s, uint32_t v_bytes) {
+                                int64_t n, const double* s, int turn, uint32_t v_bytes) {
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-  if (s[S_DONE] != 0.0) return;
+  if (s[S_DONE + turn] != 0.0) return;
   const int64_t r = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / SPMV_QUAD_LANES;
   const int lig = threadIdx.x & (SPMV_QUAD_LANES - 1);
   if (r >= n) return;
@@ -107,8 +112,8 @@ __global__ void sv_spmv_it_quad(const int64_t* __restrict__ rp, const int32_t* _
 // the same with one 8-byte load per lane and value (values beyond 4 GiB)
 __global__ void sv_spmv_it(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
                            const double* __restrict__ v, const double* __restrict__ p, double* __restrict__ ap,
-                           int64_t n, const double* s) {
-  if (s[S_DONE] != 0.0) return;
+                           int64_t n, const double* s, int turn) {
+  if (s[S_DONE + turn] != 0.0) return;
   const int64_t r = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / SPMV_LANES;
   const int lig = threadIdx.x & (SPMV_LANES - 1);
   if (r >= n) return;
@@ -367,8 +372,8 @@ __global__ __launch_bounds__(256) void sv_spmv_slices(const unsigned char* __res
                                                       const uint32_t* __restrict__ cbase,
                                                       const uint32_t* __restrict__ offset, int64_t n_slices,
                                                       const double* __restrict__ p, double* __restrict__ ap,
-                                                      const double* s) {
-  if (s[S_DONE] != 0.0) return;
+                                                      const double* s, int turn) {
+  if (s[S_DONE + turn] != 0.0) return;
   const int64_t sl = int64_t(__builtin_amdgcn_readfirstlane(int(blockIdx.x * 4 + (threadIdx.x >> 6))));
   const int lane = threadIdx.x & 63;
   if (sl >= n_slices) return;
@@ -381,72 +386,72 @@ __global__ __launch_bounds__(256) void sv_spmv_slices(const unsigned char* __res
   if (r != SL_NONE) ap[r] = y;
 }
 
-// block tree sum of per-thread values into part[blockIdx.x]
-__device__ inline void block_sum2(double a, double b, double* part_a, double* part_b) {
-  __shared__ double sa[SV_B], sb[SV_B];
-  sa[threadIdx.x] = a;
-  sb[threadIdx.x] = b;
-  __syncthreads();
-  for (int s = SV_B / 2; s > 0; s >>= 1) {
-    if (int(threadIdx.x) < s) {
-      sa[threadIdx.x] += sa[threadIdx.x + s];
-      sb[threadIdx.x] += sb[threadIdx.x + s];
-    }
-    __syncthreads();
+// sums of two values over the block, in every thread: a butterfly per wave,
+// then the waves in order
+struct Sum2 {
+  double a, b;
+};
+__device__ inline Sum2 block_sum2(double a, double b) {
+  __shared__ Sum2 w[SV_B / 64];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o);
+    b += __shfl_xor(b, o);
   }
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = {a, b};
+  __syncthreads();
+  Sum2 t = w[0];
+#pragma unroll
+  for (int k = 1; k < SV_B / 64; ++k) {
+    t.a += w[k].a;
+    t.b += w[k].b;
+  }
+  __syncthreads();  // w may be written again
+  return t;
+}
+
+// the block's sums into its partials (part_b may be absent)
+__device__ inline void block_partials(double a, double b, double* part_a, double* part_b) {
+  const Sum2 t = block_sum2(a, b);
   if (threadIdx.x == 0) {
-    part_a[blockIdx.x] = sa[0];
-    if (part_b) part_b[blockIdx.x] = sb[0];
+    part_a[blockIdx.x] = t.a;
+    if (part_b) part_b[blockIdx.x] = t.b;
   }
 }
 
-// partials of p.Ap; grid SV_PARTS x SV_B, strided
-__global__ void sv_dot_it(const double* __restrict__ x, const double* __restrict__ y, int64_t n, const double* s,
-                          double* part) {
-  if (s[S_DONE] != 0.0) return;
+// total of the partials of a launch of the same grid, in every thread
+__device__ inline Sum2 total_partials(const double* part_a, const double* part_b) {
+  double a = 0.0, b = 0.0;
+  for (unsigned i = threadIdx.x; i < gridDim.x; i += SV_B) {
+    a += part_a[i];
+    if (part_b) b += part_b[i];
+  }
+  return block_sum2(a, b);
+}
+
+// partials of p.Ap
+__global__ __launch_bounds__(SV_B) void sv_dot_it(const double* __restrict__ x, const double* __restrict__ y, int64_t n,
+                                                  const double* s, int turn, double* part) {
+  if (s[S_DONE + turn] != 0.0) return;
   double a = 0.0;
-  for (int64_t i = int64_t(blockIdx.x) * SV_B + threadIdx.x; i < n; i += int64_t(SV_PARTS) * SV_B)
+  for (int64_t i = int64_t(blockIdx.x) * SV_B + threadIdx.x; i < n; i += int64_t(gridDim.x) * SV_B)
     a = __builtin_fma(x[i], y[i], a);
-  block_sum2(a, 0.0, part, nullptr);
+  block_partials(a, 0.0, part, nullptr);
 }
 
-// final sums of the partials into scalars, then the PCG scalar step:
-// mode 0: s[S_RZ] = a, s[S_BB] = b (start);  mode 1: s[S_PAP] = a, alpha = rz / pAp;
-// mode 2: s[S_RZN] = a, s[S_RR] = b, beta = rzn / rz, rz = rzn
-__global__ void sv_final(const double* __restrict__ part_a, const double* __restrict__ part_b, double* s, int mode,
-                         double stop, double max_iter) {
-  if (mode != 0 && s[S_DONE] != 0.0) return;
-  __shared__ double sa[SV_PARTS], sb[SV_PARTS];
-  for (int i = threadIdx.x; i < SV_PARTS; i += blockDim.x) {
-    sa[i] = part_a[i];
-    sb[i] = part_b ? part_b[i] : 0.0;
+// start: r.z and b.b from the partials of the start kernel (one workgroup)
+__global__ __launch_bounds__(SV_B) void sv_start_scalars(const double* __restrict__ part_a,
+                                                         const double* __restrict__ part_b, int parts, double* s) {
+  double a = 0.0, b = 0.0;
+  for (int i = threadIdx.x; i < parts; i += SV_B) {
+    a += part_a[i];
+    b += part_b[i];
   }
-  __syncthreads();
-  for (int st = SV_PARTS / 2; st > 0; st >>= 1) {
-    for (int i = threadIdx.x; i < st; i += blockDim.x) {
-      sa[i] += sa[i + st];
-      sb[i] += sb[i + st];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x != 0) return;
-  if (mode == 0) {
-    s[S_RZ] = sa[0];
-    s[S_BB] = sb[0];
-    s[S_RR] = sb[0];
-  } else if (mode == 1) {
-    s[S_PAP] = sa[0];
-    s[S_ALPHA] = s[S_RZ] / sa[0];
-  } else {
-    s[S_RZN] = sa[0];
-    s[S_RR] = sb[0];
-    s[S_BETA] = sa[0] / s[S_RZ];
-    s[S_RZ] = sa[0];
-    const double it = s[S_ITER] + 1.0;
-    const bool conv = sqrt(sb[0]) <= stop;
-    s[S_ITER] = it;
-    s[S_CONV] = conv ? 1.0 : 0.0;
-    s[S_DONE] = (conv || it >= max_iter) ? 1.0 : 0.0;
+  const Sum2 t = block_sum2(a, b);
+  if (threadIdx.x == 0) {
+    s[S_RZ] = t.a;
+    s[S_BB] = t.b;
+    s[S_RR] = t.b;
   }
 }
 
@@ -564,7 +569,7 @@ __global__ void sv_start_jacobi(const double* __restrict__ b, const double* __re
                                 double* __restrict__ x, double* __restrict__ r, double* __restrict__ z,
                                 double* __restrict__ p, double* part_a, double* part_b) {
   double ra = 0.0, rb = 0.0;
-  for (int64_t i = int64_t(blockIdx.x) * SV_B + threadIdx.x; i < n; i += int64_t(SV_PARTS) * SV_B) {
+  for (int64_t i = int64_t(blockIdx.x) * SV_B + threadIdx.x; i < n; i += int64_t(gridDim.x) * SV_B) {
     const double bi = b[i], zi = bi / d[i];
     x[i] = 0.0;
     r[i] = bi;
@@ -573,18 +578,18 @@ __global__ void sv_start_jacobi(const double* __restrict__ b, const double* __re
     ra += bi * zi;
     rb += bi * bi;
   }
-  block_sum2(ra, rb, part_a, part_b);
+  block_partials(ra, rb, part_a, part_b);
 }
 
 // update: x += alpha p, r -= alpha Ap, z = r / d; partials of (r, z) and (r, r)
 __global__ void sv_update_jacobi(const double* __restrict__ d, const double* __restrict__ p,
-                                 const double* __restrict__ ap, const double* __restrict__ s, int64_t n,
-                                 double* __restrict__ x, double* __restrict__ r, double* __restrict__ z, double* part_a,
-                                 double* part_b) {
-  if (s[S_DONE] != 0.0) return;
-  const double alpha = s[S_ALPHA];
+                                 const double* __restrict__ ap, const double* __restrict__ s, int turn,
+                                 const double* __restrict__ part_pap, int64_t n, double* __restrict__ x,
+                                 double* __restrict__ r, double* __restrict__ z, double* part_a, double* part_b) {
+  if (s[S_DONE + turn] != 0.0) return;
+  const double alpha = s[S_RZ + turn] / total_partials(part_pap, nullptr).a;
   double ra = 0.0, rb = 0.0;
-  for (int64_t i = int64_t(blockIdx.x) * SV_B + threadIdx.x; i < n; i += int64_t(SV_PARTS) * SV_B) {
+  for (int64_t i = int64_t(blockIdx.x) * SV_B + threadIdx.x; i < n; i += int64_t(gridDim.x) * SV_B) {
     x[i] = __builtin_fma(alpha, p[i], x[i]);
     const double ri = __builtin_fma(-alpha, ap[i], r[i]);
     r[i] = ri;
@@ -593,7 +598,7 @@ __global__ void sv_update_jacobi(const double* __restrict__ d, const double* __r
     ra += ri * zi;
     rb += ri * ri;
   }
-  block_sum2(ra, rb, part_a, part_b);
+  block_partials(ra, rb, part_a, part_b);
 }
 
 // block Jacobi: six lanes per node block (lane = row of the block), ten
@@ -642,7 +647,7 @@ __global__ void sv_start_block(const double* __restrict__ b, const double* __res
                                double* __restrict__ r, double* __restrict__ z, double* __restrict__ p, double* part_a,
                                double* part_b) {
   const int lane = threadIdx.x & 63;
-  const int64_t waves = int64_t(SV_PARTS) * (SV_B / 64);
+  const int64_t waves = int64_t(gridDim.x) * (SV_B / 64);
   double ra = 0.0, rb = 0.0;
   for (int64_t w = int64_t(blockIdx.x) * (SV_B / 64) + (threadIdx.x >> 6); w * BJ_PER_WAVE < nblk; w += waves) {
     const BjLane L = bj_lane(starts, nblk, w, lane);
@@ -662,17 +667,18 @@ __global__ void sv_start_block(const double* __restrict__ b, const double* __res
       rb = __builtin_fma(ri, ri, rb);
     }
   }
-  block_sum2(ra, rb, part_a, part_b);
+  block_partials(ra, rb, part_a, part_b);
 }
 // update: x += alpha p, r -= alpha Ap, z = M^-1 r; partials of (r, z) and (r, r)
 __global__ void sv_update_block(const double* __restrict__ inv, const int32_t* __restrict__ starts, int64_t nblk,
                                 const double* __restrict__ p, const double* __restrict__ ap,
-                                const double* __restrict__ s, double* __restrict__ x, double* __restrict__ r,
-                                double* __restrict__ z, double* part_a, double* part_b) {
-  if (s[S_DONE] != 0.0) return;
-  const double alpha = s[S_ALPHA];
+                                const double* __restrict__ s, int turn, const double* __restrict__ part_pap,
+                                double* __restrict__ x, double* __restrict__ r, double* __restrict__ z, double* part_a,
+                                double* part_b) {
+  if (s[S_DONE + turn] != 0.0) return;
+  const double alpha = s[S_RZ + turn] / total_partials(part_pap, nullptr).a;
   const int lane = threadIdx.x & 63;
-  const int64_t waves = int64_t(SV_PARTS) * (SV_B / 64);
+  const int64_t waves = int64_t(gridDim.x) * (SV_B / 64);
   double ra = 0.0, rb = 0.0;
   for (int64_t w = int64_t(blockIdx.x) * (SV_B / 64) + (threadIdx.x >> 6); w * BJ_PER_WAVE < nblk; w += waves) {
     const BjLane L = bj_lane(starts, nblk, w, lane);
@@ -690,15 +696,31 @@ __global__ void sv_update_block(const double* __restrict__ inv, const int32_t* _
       rb = __builtin_fma(ri, ri, rb);
     }
   }
-  block_sum2(ra, rb, part_a, part_b);
+  block_partials(ra, rb, part_a, part_b);
 }
 
-// p = z + beta p
-__global__ void sv_direction(const double* __restrict__ z, const double* __restrict__ s, int64_t n,
-                             double* __restrict__ p) {
-  if (s[S_DONE] != 0.0) return;
-  const double beta = s[S_BETA];
-  for (int64_t i = int64_t(blockIdx.x) * SV_B + threadIdx.x; i < n; i += int64_t(SV_PARTS) * SV_B)
+// beta and the update's scalars from the partials of (r, z) and (r, r); p = z + beta p
+__global__ __launch_bounds__(SV_B) void sv_direction(const double* __restrict__ z, double* s, int turn,
+                                                     const double* __restrict__ part_a,
+                                                     const double* __restrict__ part_b, double stop, double max_iter,
+                                                     int64_t n, double* __restrict__ p) {
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (s[S_DONE + turn] != 0.0) {
+    if (first) s[S_DONE + (turn ^ 1)] = 1.0;  // the flag goes on to the next update
+    return;
+  }
+  const Sum2 t = total_partials(part_a, part_b);
+  const double beta = t.a / s[S_RZ + turn];
+  if (first) {
+    s[S_RZ + (turn ^ 1)] = t.a;
+    s[S_RR] = t.b;
+    const double it = s[S_ITER] + 1.0;
+    const bool conv = sqrt(t.b) <= stop;
+    s[S_ITER] = it;
+    s[S_CONV] = conv ? 1.0 : 0.0;
+    s[S_DONE + (turn ^ 1)] = (conv || it >= max_iter) ? 1.0 : 0.0;
+  }
+  for (int64_t i = int64_t(blockIdx.x) * SV_B + threadIdx.x; i < n; i += int64_t(gridDim.x) * SV_B)
     p[i] = __builtin_fma(beta, p[i], z[i]);
 }
 
@@ -797,7 +819,9 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
   if (!(e = take(bufs, 8, size_t(2 * SV_PARTS), part)).empty()) return e;
   if (!(e = take(bufs, 9, size_t(S_COUNT), sc)).empty()) return e;
   double *b = vec[0], *x = vec[1], *r = vec[2], *z = vec[3], *p = vec[4], *ap = vec[5], *rr = vec[6], *rb = vec[7];
-  double *pa = part, *pb = part + SV_PARTS;
+  // partials: (r, z), (r, r), and p.Ap in b, which is not read after the start
+  // (it holds n values, at least one per block)
+  double *pa = part, *pb = part + SV_PARTS, *pc = b;
   double* host = bufs.host;
   const int64_t* rp[4];
   const int32_t* ci[4];
@@ -851,13 +875,15 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
       HIP_TRY(hipGetLastError());
     }
   }
-  // start
+  // start.  The reductions' grid: one block per SV_B dofs, at most SV_PARTS (a
+  // function of n, and the same for every launch of the solve)
+  const unsigned parts = unsigned(std::min<int64_t>(SV_PARTS, grid_for(na, SV_B)));
   if (precond == 0)
-    sv_start_jacobi<<<SV_PARTS, B, 0, s>>>(b, diag, na, x, r, z, p, pa, pb);
+    sv_start_jacobi<<<parts, B, 0, s>>>(b, diag, na, x, r, z, p, pa, pb);
   else
-    sv_start_block<<<SV_PARTS, B, 0, s>>>(b, inv, starts, nblk, x, r, z, p, pa, pb);
+    sv_start_block<<<parts, B, 0, s>>>(b, inv, starts, nblk, x, r, z, p, pa, pb);
   HIP_TRY(hipGetLastError());
-  sv_final<<<1, 1024, 0, s>>>(pa, pb, sc, 0, 0.0, 0.0);
+  sv_start_scalars<<<1, B, 0, s>>>(pa, pb, int(parts), sc);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(host, sc, sizeof(double) * S_COUNT, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
@@ -880,19 +906,18 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
     for (;;) {
       const int nq = std::min(batch, max_iter - queued);
       for (int q = 0; q < nq; ++q) {
+        const int turn = (queued + q) & 1;
         if (sl.data)
           sv_spmv_slices<<<grid_for(sl.n, 4), 256, 0, s>>>(sl.data, rp[0], sl.rows, sl.pairs, sl.cbase, sl.offset,
-                                                           sl.n, p, ap, sc);
-        else if (quad) sv_spmv_it_quad<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, v_bytes);
-        else sv_spmv_it<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc);
-        sv_dot_it<<<SV_PARTS, B, 0, s>>>(p, ap, na, sc, pa);
-        sv_final<<<1, 1024, 0, s>>>(pa, nullptr, sc, 1, stop, double(max_iter));
+                                                           sl.n, p, ap, sc, turn);
+        else if (quad) sv_spmv_it_quad<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, turn, v_bytes);
+        else sv_spmv_it<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, turn);
+        sv_dot_it<<<parts, B, 0, s>>>(p, ap, na, sc, turn, pc);
         if (precond == 0)
-          sv_update_jacobi<<<SV_PARTS, B, 0, s>>>(diag, p, ap, sc, na, x, r, z, pa, pb);
+          sv_update_jacobi<<<parts, B, 0, s>>>(diag, p, ap, sc, turn, pc, na, x, r, z, pa, pb);
         else
-          sv_update_block<<<SV_PARTS, B, 0, s>>>(inv, starts, nblk, p, ap, sc, x, r, z, pa, pb);
-        sv_final<<<1, 1024, 0, s>>>(pa, pb, sc, 2, stop, double(max_iter));
-        sv_direction<<<SV_PARTS, B, 0, s>>>(z, sc, na, p);
+          sv_update_block<<<parts, B, 0, s>>>(inv, starts, nblk, p, ap, sc, turn, pc, x, r, z, pa, pb);
+        sv_direction<<<parts, B, 0, s>>>(z, sc, turn, pa, pb, stop, double(max_iter), na, p);
       }
       HIP_TRY(hipGetLastError());
       const bool first = queued == 0;
@@ -904,7 +929,7 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
       }
       HIP_TRY(hipMemcpyAsync(host, sc, sizeof(double) * S_COUNT, hipMemcpyDeviceToHost, s));
       HIP_TRY(hipStreamSynchronize(s));
-      if (host[S_DONE] != 0.0 || queued >= max_iter) break;
+      if (host[S_DONE] != 0.0 || host[S_DONE + 1] != 0.0 || queued >= max_iter) break;
       if (slice && first) {
         std::memcpy(&slice_total, host + S_COUNT, sizeof(uint32_t));
         if (!slices_fill(bufs, rp[0], ci[0], v[0], v_bytes, slice_total, s, sl)) sl.data = nullptr;
