@@ -7,6 +7,8 @@
 
 namespace femdev {
 
+struct UpdateReport;
+
 struct Device {
   hipStream_t stream = nullptr;
   int dev = 0;
@@ -107,6 +109,11 @@ struct Device {
   double sol_ms = 0.0;
   double* u_glob = nullptr;  // global displacements of the last solve (6 per node)
   size_t ucap = 0;
+  // updates in place (fem_device.hip): report words, their copy in pinned host
+  // memory, and the number of the last update
+  uint32_t* upd_words = nullptr;
+  UpdateReport* upd_report = nullptr;
+  uint32_t upd_number = 0;
   // timing
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr, ev3 = nullptr, ev4 = nullptr, ev5 = nullptr;
   bool timed = false, timed_bwd = false;

@@ -268,10 +268,19 @@ std::string run_adjoint(Device* d, int mode, const double* g, double* const dpar
 double last_backward_ms(Device* d);
 
 // Device-to-device replacement of one element type's parameters or of the node
-// coordinates (then synchronous); the host mirrors are refreshed from the
-// device.  The caller reruns run_setup for the frames.
-std::string replace_params(Device* d, int type, const double* src, double* host_copy, void* stream);
-std::string replace_nodes(Device* d, const double* src, double* host_copy, void* stream);
+// coordinates, with the frames that follow from them; synchronous.  The report
+// says for each type whether a frame's code changed (fetch_codes then reads
+// them), and whether the plates' E, nu, k differ from the first plate's.
+struct UpdateReport {
+  uint32_t changed[3] = {0, 0, 0};
+  uint32_t mixed = 0;
+  double plate[4] = {0.0, 0.0, 0.0, 0.0};  // the first plate's parameters
+};
+std::string update_params(Device* d, int type, const double* src, void* stream, UpdateReport& out);
+std::string update_nodes(Device* d, const double* src, void* stream, UpdateReport& out);
+std::string fetch_nodes(Device* d, double* host);
+std::string fetch_params(Device* d, int type, double* host);
+std::string fetch_codes(Device* d, int type, std::vector<uint16_t>& rzero);
 
 double* values(Device* d);
 const int64_t* row_ptr(Device* d);

@@ -89,6 +89,9 @@ struct fem_model {
   std::vector<uint32_t> node_number;
   std::vector<double> xyz;
   std::unordered_map<uint64_t, std::vector<uint32_t>> coord_hash;
+  // an update in place rewrites the device's coordinates or parameters: xyz,
+  // params and coord_hash here are then behind until refresh_host
+  bool xyz_behind = false, hash_behind = false, params_behind[3] = {false, false, false};
   ElementSet set[3];
   std::unordered_map<uint64_t, uint32_t> truss_pairs, beam_pairs;
   std::vector<std::vector<uint32_t>> node_plates;
@@ -174,6 +177,8 @@ void clear_model(fem_model* m, uint32_t nodes_number) {
   m->node_number.clear();
   m->xyz.clear();
   m->coord_hash.clear();
+  m->xyz_behind = m->hash_behind = false;
+  for (bool& b : m->params_behind) b = false;
   for (auto& s : m->set) s = ElementSet();
   m->truss_pairs.clear();
   m->beam_pairs.clear();
@@ -190,6 +195,22 @@ void clear_model(fem_model* m, uint32_t nodes_number) {
   m->bc_dirty = true;
   m->own_vals = false;
   if (m->dev) femdev::invalidate_separation(m->dev);
+}
+
+// the host's coordinates and parameters from the device, if an update left them
+// behind (called wherever the host reads them)
+int refresh_host(fem_model* m) {
+  std::string e;
+  if (m->xyz_behind) {
+    e = femdev::fetch_nodes(m->dev, m->xyz.data());
+    if (e.empty()) m->xyz_behind = false;
+  }
+  for (int t = 0; t < 3 && e.empty(); ++t)
+    if (m->params_behind[t]) {
+      e = femdev::fetch_params(m->dev, t, m->set[t].params.data());
+      if (e.empty()) m->params_behind[t] = false;
+    }
+  return e.empty() ? FEM_OK : fail(m, FEM_ERR_DEVICE, e);
 }
 
 bool node_exists(fem_model* m, uint32_t number) {  // methods_for_node_data_handle.rs:81-86
@@ -1421,6 +1442,10 @@ int ensure_ready(fem_model* m) {
     m->dev = femdev::create_device(err);
     if (!m->dev) return fail(m, FEM_ERR_DEVICE, err);
   }
+  if (m->dirty || !m->pattern_valid) {
+    int rc = refresh_host(m);
+    if (rc) return rc;
+  }
   if (m->dirty) {
     auto e = femdev::upload_nodes(m->dev, m->xyz.data(), m->node_number.size());
     for (int t = 0; t < 3 && e.empty(); ++t) {
@@ -1446,6 +1471,8 @@ int ensure_adjoint(fem_model* m) {
   int rc = ensure_ready(m);
   if (rc) return rc;
   if (m->adj_valid) return FEM_OK;
+  rc = refresh_host(m);
+  if (rc) return rc;
   femdev::AdjointMaps am;
   const size_t N = m->nodes_number;
   for (int t = 0; t < 3; ++t) {
@@ -1569,20 +1596,15 @@ int run_backward(fem_model* m, int mode, const double* g, double* dp_truss, doub
   return e.empty() ? FEM_OK : fail(m, FEM_ERR_DEVICE, e);
 }
 
-// reruns the setup kernels after a parameter or coordinate change; a changed
-// frame zero pattern invalidates the sparsity pattern
-int rerun_setup(fem_model* m, bool all_types, int type) {
-  for (int t = 0; t < 3; ++t) {
-    if (!all_types && t != type) continue;
-    std::vector<uint16_t> rz;
-    auto e = femdev::run_setup(m->dev, t, m->set[t].size(), m->rel_tol, m->abs_tol, rz);
-    if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
-    if (rz != m->rzero[t]) {
-      m->rzero[t] = rz;
+// a frame code that an update changed changes the sparsity pattern
+int apply_report(fem_model* m, const femdev::UpdateReport& r) {
+  for (int t = 0; t < 3; ++t)
+    if (r.changed[t]) {
       m->pattern_valid = false;
       m->adj_valid = false;
+      auto e = femdev::fetch_codes(m->dev, t, m->rzero[t]);
+      if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
     }
-  }
   return FEM_OK;
 }
 
@@ -1969,7 +1991,14 @@ const char* fem_last_error(const fem_model* m) { return m ? m->err.c_str() : "nu
 int fem_add_nodes(fem_model* m, size_t n, const uint32_t* numbers, const double* xyz, size_t* n_ok) {
   if (!m || (n && (!numbers || !xyz))) return FEM_ERR_ARGUMENT;
   size_t i = 0;
-  int rc = FEM_OK;
+  int rc = refresh_host(m);
+  if (rc) n = 0;
+  if (!rc && m->hash_behind) {
+    m->coord_hash.clear();
+    for (size_t k = 0; k < m->node_number.size(); ++k)
+      m->coord_hash[coord_key(m->xyz[3 * k], m->xyz[3 * k + 1], m->xyz[3 * k + 2])].push_back(uint32_t(k));
+    m->hash_behind = false;
+  }
   for (; i < n; ++i) {
     uint32_t number = numbers[i];
     double x = xyz[3 * i], y = xyz[3 * i + 1], z = xyz[3 * i + 2];
@@ -2011,7 +2040,8 @@ int fem_add_trusses(fem_model* m, size_t n, const uint32_t* numbers, const uint3
                     const double* A, const double* A2, size_t* n_ok) {
   if (!m || (n && (!numbers || !conn || !E || !A))) return FEM_ERR_ARGUMENT;
   size_t i = 0;
-  int rc = FEM_OK;
+  int rc = refresh_host(m);
+  if (rc) n = 0;
   auto& S = m->set[TRUSS];
   for (; i < n; ++i) {
     uint32_t number = numbers[i], n1 = conn[2 * i], n2 = conn[2 * i + 1];
@@ -2054,7 +2084,8 @@ int fem_add_beams(fem_model* m, size_t n, const uint32_t* numbers, const uint32_
                   size_t* n_ok) {
   if (!m || (n && (!numbers || !conn || !props))) return FEM_ERR_ARGUMENT;
   size_t i = 0;
-  int rc = FEM_OK;
+  int rc = refresh_host(m);
+  if (rc) n = 0;
   auto& S = m->set[BEAM];
   for (; i < n; ++i) {
     uint32_t number = numbers[i], n1 = conn[2 * i], n2 = conn[2 * i + 1];
@@ -2106,7 +2137,8 @@ int fem_add_plates(fem_model* m, size_t n, const uint32_t* numbers, const uint32
                    size_t* n_ok) {
   if (!m || (n && (!numbers || !conn || !props))) return FEM_ERR_ARGUMENT;
   size_t i = 0;
-  int rc = FEM_OK;
+  int rc = refresh_host(m);
+  if (rc) n = 0;
   auto& S = m->set[PLATE];
   for (; i < n; ++i) {
     uint32_t number = numbers[i];
@@ -2319,28 +2351,28 @@ int fem_update_params(fem_model* m, int type, const double* params_device, void*
   if (!m || type < 0 || type > 2 || (!params_device && m->set[type].size())) return FEM_ERR_ARGUMENT;
   int rc = ensure_ready(m);
   if (rc) return rc;
-  auto e = femdev::replace_params(m->dev, type, params_device, m->set[type].params.data(), stream);
-  if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
+  femdev::UpdateReport rep;
   m->own_vals = false;
+  m->params_behind[type] = m->set[type].size() != 0;
+  auto e = femdev::update_params(m->dev, type, params_device, stream, rep);
+  if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
   if (type == PLATE && m->path == "plate_lanes") {  // the slot layout follows the new parameters
-    double mat[3];
-    e = femdev::set_plate_lane_material(m->dev, plate_material_uniform(m, mat), mat);
+    const double mat[3] = {rep.plate[0], rep.plate[1], rep.plate[3]};
+    e = femdev::set_plate_lane_material(m->dev, !rep.mixed, mat);
     if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
   }
-  return type == BEAM ? rerun_setup(m, false, BEAM) : FEM_OK;
+  return apply_report(m, rep);
 }
 
 int fem_update_nodes(fem_model* m, const double* xyz_device, void* stream) {
   if (!m || (!xyz_device && m->node_number.size())) return FEM_ERR_ARGUMENT;
   int rc = ensure_ready(m);
   if (rc) return rc;
-  auto e = femdev::replace_nodes(m->dev, xyz_device, m->xyz.data(), stream);
-  if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
+  femdev::UpdateReport rep;
   m->own_vals = false;
-  m->coord_hash.clear();
-  for (size_t i = 0; i < m->node_number.size(); ++i)
-    m->coord_hash[coord_key(m->xyz[3 * i], m->xyz[3 * i + 1], m->xyz[3 * i + 2])].push_back(uint32_t(i));
-  return rerun_setup(m, true, 0);
+  m->xyz_behind = m->hash_behind = m->node_number.size() != 0;
+  auto e = femdev::update_nodes(m->dev, xyz_device, stream, rep);
+  return e.empty() ? apply_report(m, rep) : fail(m, FEM_ERR_DEVICE, e);
 }
 
 int fem_add_displacements(fem_model* m, size_t n, const uint32_t* numbers, const int32_t* dofs, const double* values,
@@ -2612,6 +2644,11 @@ int fem_set_option(fem_model* m, const char* key, int64_t value) {
 int fem_batch_create(fem_model* const* models, size_t n, fem_batch** out) {
   if (!out || (!models && n)) return FEM_ERR_ARGUMENT;
   *out = nullptr;
+  for (size_t i = 0; i < n; ++i)
+    if (models[i]) {
+      const int rc = refresh_host(models[i]);
+      if (rc) return rc;
+    }
   for (size_t i = 0; i < n; ++i)
     if (!models[i] || models[i]->rel_tol != models[0]->rel_tol || models[i]->abs_tol != models[0]->abs_tol)
       return FEM_ERR_ARGUMENT;
