@@ -88,9 +88,14 @@ struct Device {
   int32_t* sep_ci = nullptr;
   int64_t* sep_dpos = nullptr;  // diagonal entry of each row (pattern-only)
   uint32_t* sep_pack = nullptr;  // per dof: class << 30 | its index among the a (or b) dofs
+  uint8_t* sep_mark = nullptr;   // rows that hold a column that is not free
+  uint8_t* sep_left = nullptr;   // groups of rows whose entries are not one run of K_aa
+  uint64_t* sep_chunk = nullptr; // per chunk of dofs: a and b dofs (packed), then those before it
+  uint32_t *sep_err = nullptr, *sep_rows2 = nullptr;  // per chunk its first error; per row its a and b entries
+  int64_t* sep_host = nullptr;   // the summary, in pinned host memory
   bool sep_dpos_valid = false;
-  size_t sep_cap[20] = {};
-  int64_t sep_bc_rows = -1;
+  size_t sep_cap[25] = {};
+  int64_t sep_bc_rows = -1, sep_n_cons = 0;  // dofs of the uploaded boundary conditions, and restrained ones among them
   int64_t sep_rows[4] = {0, 0, 0, 0}, sep_nnz[4] = {0, 0, 0, 0}, sep_base[4] = {0, 0, 0, 0};
   bool sep_done = false;
   double sep_ms = 0.0;

@@ -65,6 +65,8 @@ void destroy_device(Device* d) {
   f(d->adj_bmask); f(d->adj_boff); f(d->adj_inc_ptr); f(d->adj_xpos); f(d->adj_xs); f(d->adj_kpack); f(d->adj_eorder);
   f(d->sep_cons); f(d->sep_pack); f(d->sep_cls); f(d->sep_tmp); f(d->sep_disp); f(d->sep_force); f(d->sep_ra); f(d->sep_ub);
   f(d->sep_v); f(d->sep_flag); f(d->sep_pos); f(d->sep_key); f(d->sep_cnt); f(d->sep_off); f(d->sep_aa); f(d->sep_bb);
+  f(d->sep_mark); f(d->sep_left); f(d->sep_chunk); f(d->sep_err); f(d->sep_rows2);
+  if (d->sep_host) { (void)hipHostFree(d->sep_host); d->sep_host = nullptr; }
   f(d->sep_rp); f(d->sep_sum); f(d->sep_ci); f(d->sep_dpos);
   f(d->pb_hdr); f(d->pb_conn); f(d->pb_eid); f(d->pb_blk);
   f(d->pn_eid); f(d->pn_nodes); f(d->pn_wave); f(d->pn_lanes); f(d->pn_geo);
