@@ -643,44 +643,75 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
                    gxl);
 }
 
-// Compliance sensitivities of plates by strain energy: four lanes per element,
-// lane p = integration point p (and node p's drilling term and outputs).  Lane
-// p loads node p's displacements; a quad broadcast gives every lane all four.
-template <bool FLAT>
-__global__ __launch_bounds__(256) void plate_compliance_kernel(AdjArgs A) {
-  const unsigned b = xcd_block(blockIdx.x, gridDim.x);
-  const size_t e0 = size_t(b) * 64 + (threadIdx.x >> 2);
-  const int p = int(threadIdx.x & 3u);
-  const bool live = e0 < A.n;
-  const size_t e = live ? e0 : A.n - 1;  // dead lanes still take part in the lane sums
-  PlateElem el;
-  load_plate_elem<FLAT>(A, e, el);
-  const fem::PlateMat mat = fem::plate_material(el.E, el.nu, el.t, el.k);
-  fem::PlateShear sv;
-  fem::plate_shear_vectors(el.xl, sv);
-  const uint32_t ap = p == 0 ? el.nd[0] : (p == 1 ? el.nd[1] : (p == 2 ? el.nd[2] : el.nd[3]));
-  double up[6];
-  if (FLAT) {
-#pragma unroll
-    for (int i = 0; i < 6; ++i) up[i] = A.g[6 * size_t(ap) + i];
-  } else {
-    local_u(A.g, ap, el.R, up);
-  }
-  double U[4][6];
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    U[0][i] = quad_bcast<0>(up[i]);
-    U[1][i] = quad_bcast<1>(up[i]);
-    U[2][i] = quad_bcast<2>(up[i]);
-    U[3][i] = quad_bcast<3>(up[i]);
-  }
+// Compliance sensitivities of plates by strain energy.  LANES = 1: one lane per
+// element takes the four integration points in turn.  Bound: FP64 arithmetic
+// (about 4 kFLOP per element, 60 loads).  701 x 499 quads: 36 us, where four lanes
+// per element, a point each, took 58: they form the material constants, the frame
+// and the element's finish four times over and sum fifteen values across the
+// lanes.  LANES = 4 does so all the same where there are too few elements to fill
+// the chip, so that the element's chain is short (64 x 64 quads: 9.3 vs 12.1 us).
+constexpr size_t PC_FEW = 32768;  // elements: 16384 take 10.2 (four lanes) vs 12.7 us, 65536 take 19.6 vs 17.5 us
+template <bool FLAT, int LANES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void plate_compliance_kernel(AdjArgs A) {
+  uint32_t e = (xcd_block(blockIdx.x, gridDim.x) * 256u + threadIdx.x) / LANES;
+  const int p = LANES == 4 ? int(threadIdx.x & 3u) : 0;
+  if (e >= A.n) return;  // the lanes of an element together
   double P[7], gxl[6], hx = 0.0, hy = 0.0;
 #pragma unroll
   for (int i = 0; i < 7; ++i) P[i] = 0.0;
 #pragma unroll
   for (int i = 0; i < 6; ++i) gxl[i] = 0.0;
-  fem::plate_compliance_point(el.xl, p, mat, sv, U, P, gxl, hx, hy);
-  plate_write(A, e, p, live, el, P, gxl, hx, hy);
+  {
+    PlateElem el;
+    load_plate_elem<FLAT>(A, e, el);
+    double U[4][6];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      if (FLAT) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) U[a][i] = A.g[6 * size_t(el.nd[a]) + i];
+      } else {
+        local_u(A.g, el.nd[a], el.R, U[a]);
+      }
+    }
+    const fem::PlateMat mat = fem::plate_material(el.E, el.nu, el.t, el.k);
+    const fem::PlateEdges ed = fem::plate_edges(el.xl);
+    if (p == 0) fem::plate_compliance_drilling(U, hx, hy);
+    const double gs = sqrt(double(fem::ONE_THIRD_F32));
+#pragma unroll 1
+    for (int ip = p; ip < p + 4 / LANES; ++ip)
+      fem::plate_compliance_point(el.xl, (ip == 0 || ip == 3) ? gs : -gs, ip < 2 ? gs : -gs, mat, ed, U, P, gxl, hx,
+                                  hy);
+  }
+  if (LANES == 4) {
+#pragma unroll
+    for (int i = 0; i < 7; ++i) P[i] = quad_sum(P[i]);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) gxl[i] = quad_sum(gxl[i]);
+    hx = quad_sum(hx);
+    hy = quad_sum(hy);
+  }
+  // the element's frame, nodes and parameters again: held through the points they
+  // would not fit two waves per SIMD
+  asm volatile("" : "+v"(e));
+  PlateElem el;
+  load_plate_elem<FLAT>(A, e, el);
+  double gp[4], gX[4][3];
+  fem::plate_adjoint_finish(P, gxl, hx, hy, el.loc, el.R, el.E, el.nu, el.t, el.k, gp, gX);
+  if (A.dparam) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (LANES == 1 || i == p) A.dparam[4 * size_t(e) + i] = gp[i];
+  }
+  if (A.xs) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+      if (LANES == 1 || a == p) {
+        double* x = A.xs + 3 * size_t(A.xpos[4 * size_t(e) + a]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) x[i] = gX[a][i];
+      }
+  }
 }
 
 // ---------------------------------------------------------------- trusses
@@ -882,8 +913,12 @@ std::string run_adjoint(Device* d, int mode, const double* g, double* const dpar
       if (mode == MODE_DLDK && d->adj_flat)
         plate_adjoint_flat_kernel<<<unsigned((n + 15) / 16), 64, 0, s>>>(A);
       else if (mode == MODE_DLDK) plate_adjoint_kernel<<<blocks, 256, 0, s>>>(A);
-      else if (d->adj_flat) plate_compliance_kernel<true><<<blocks, 256, 0, s>>>(A);
-      else plate_compliance_kernel<false><<<blocks, 256, 0, s>>>(A);
+      else {
+        const bool few = n < PC_FEW;
+        auto kernel = d->adj_flat ? (few ? plate_compliance_kernel<true, 4> : plate_compliance_kernel<true, 1>)
+                                  : (few ? plate_compliance_kernel<false, 4> : plate_compliance_kernel<false, 1>);
+        kernel<<<few ? blocks : unsigned((n + 255) / 256), 256, 0, s>>>(A);
+      }
     } else {
       const unsigned blocks = unsigned((n + 255) / 256);
       if (t == TRUSS) {

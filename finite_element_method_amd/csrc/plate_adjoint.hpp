@@ -311,27 +311,37 @@ __host__ __device__ inline void plate_block_adjoint(const double acc[24], const 
   for (int k = 0; k < 6; ++k) c[4 * k + q] = cq[k];
 }
 
+// dL/d(E, nu, t, k) from the constitutive partials: cm = E t/(1-nu^2),
+// cb = E t^3/(12 (1-nu^2)), cs = E t k/(2 (1+nu)).  The constants' reciprocals
+// come from two divisions.
+__host__ __device__ inline void plate_adjoint_params(const double P[7], double E, double nu, double t, double k,
+                                                     double grad_param[4]) {
+  const double inv_n = 1.0 / ((1.0 - nu) * (1.0 + nu));  // 1 / (1 - nu^2)
+  const double inv_etk = 1.0 / ((E * t) * k);
+  const double cm = E * t * inv_n;
+  const double cb = E * (t * t * t) * (1.0 / 12.0) * inv_n;
+  const double inv_1pn = (1.0 - nu) * inv_n;  // 1 / (1 + nu)
+  const double cs = E * t * k * 0.5 * inv_1pn;
+  const double h = (1.0 - nu) / 2.0;
+  const double Lm = cm * ((P[0] + nu * P[1]) + h * P[2]);
+  const double Lb = cb * ((P[3] + nu * P[4]) + h * P[5]);
+  const double Ls = cs * P[6];
+  const double dcm = cm * 2.0 * nu * inv_n, dcb = cb * 2.0 * nu * inv_n;
+  grad_param[0] = ((Lm + Lb) + Ls) * (t * k * inv_etk);
+  grad_param[1] = (((P[0] * dcm + P[1] * (cm + nu * dcm)) + P[2] * (h * dcm - 0.5 * cm)) +
+                   ((P[3] * dcb + P[4] * (cb + nu * dcb)) + P[5] * (h * dcb - 0.5 * cb))) -
+                  P[6] * cs * inv_1pn;
+  grad_param[2] = ((Lm + 3.0 * Lb) + Ls) * (E * k * inv_etk);
+  grad_param[3] = Ls * (E * t * inv_etk);
+}
+
 // Element-level finish from the four lanes' sums.
 //   loc[a][k]: local coordinates R (X_a - X_3) of the crate's nodes 1..4 (a = 0..3)
 //   grad_param = dL/d(E, nu, t, k); gX[a][k] = dL/dX_a (world frame)
 __host__ __device__ inline void plate_adjoint_finish(const double P[7], const double gxl_in[6], double hx, double hy,
                                                      const double loc[4][3], const double R[9], double E, double nu,
                                                      double t, double k, double grad_param[4], double gX[4][3]) {
-  // parameters: cm = E t/(1-nu^2), cb = E t^3/(12 (1-nu^2)), cs = E t k/(2 (1+nu))
-  const double cm = E * t / (1.0 - nu * nu);
-  const double cb = E * (t * t * t) / (12.0 * (1.0 - nu * nu));
-  const double cs = E * t * k / (2.0 * (1.0 + nu));
-  const double h = (1.0 - nu) / 2.0;
-  const double Lm = cm * ((P[0] + nu * P[1]) + h * P[2]);
-  const double Lb = cb * ((P[3] + nu * P[4]) + h * P[5]);
-  const double Ls = cs * P[6];
-  const double dcm = cm * 2.0 * nu / (1.0 - nu * nu), dcb = cb * 2.0 * nu / (1.0 - nu * nu);
-  grad_param[0] = ((Lm + Lb) + Ls) / E;
-  grad_param[1] = (((P[0] * dcm + P[1] * (cm + nu * dcm)) + P[2] * (h * dcm - 0.5 * cm)) +
-                   ((P[3] * dcb + P[4] * (cb + nu * dcb)) + P[5] * (h * dcb - 0.5 * cb))) -
-                  P[6] * cs / (1.0 + nu);
-  grad_param[2] = ((Lm + 3.0 * Lb) + Ls) / t;
-  grad_param[3] = Ls / k;
+  plate_adjoint_params(P, E, nu, t, k, grad_param);
   // frame rotation: local z of nodes 1, 2, 4 feed back through dxl = (omega x p)_{x,y}
   double gxl[6];
 #pragma unroll
@@ -349,8 +359,8 @@ __host__ __device__ inline void plate_adjoint_finish(const double P[7], const do
   const double* p2 = loc[1];
   const double* p4 = loc[3];
   const double nx = p4[1] * p2[2] - p4[2] * p2[1], ny = p4[2] * p2[0] - p4[0] * p2[2], nz = p4[0] * p2[1] - p4[1] * p2[0];
-  const double nn = sqrt((nx * nx + ny * ny) + nz * nz);
-  const double gnx = -gwy / nn, gny = gwx / nn;
+  const double rn = rsqrt((nx * nx + ny * ny) + nz * nz);
+  const double gnx = -gwy * rn, gny = gwx * rn;
   double ga[4][3];
   ga[0][0] = gxl[0]; ga[0][1] = gxl[1]; ga[0][2] = 0.0;
   ga[1][0] = gxl[2]; ga[1][1] = gxl[3]; ga[1][2] = 0.0;
@@ -374,27 +384,10 @@ __host__ __device__ inline void plate_adjoint_finish(const double P[7], const do
 
 // plate_adjoint_finish for a plate whose frame is the identity and whose nodes
 // lie in z = 0 with no frame-rotation sums (hx = hy = 0): the rotation term
-// vanishes and the world gradient is the local one.  The constants' reciprocals
-// come from two divisions.
+// vanishes and the world gradient is the local one.
 __host__ __device__ inline void plate_adjoint_finish_flat(const double P[7], const double gxl[6], double E, double nu,
                                                           double t, double k, double grad_param[4], double gX[4][3]) {
-  const double inv_n = 1.0 / ((1.0 - nu) * (1.0 + nu));  // 1 / (1 - nu^2)
-  const double inv_etk = 1.0 / ((E * t) * k);
-  const double cm = E * t * inv_n;
-  const double cb = E * (t * t * t) * (1.0 / 12.0) * inv_n;
-  const double inv_1pn = (1.0 - nu) * inv_n;  // 1 / (1 + nu)
-  const double cs = E * t * k * 0.5 * inv_1pn;
-  const double h = (1.0 - nu) / 2.0;
-  const double Lm = cm * ((P[0] + nu * P[1]) + h * P[2]);
-  const double Lb = cb * ((P[3] + nu * P[4]) + h * P[5]);
-  const double Ls = cs * P[6];
-  const double dcm = cm * 2.0 * nu * inv_n, dcb = cb * 2.0 * nu * inv_n;
-  grad_param[0] = ((Lm + Lb) + Ls) * (t * k * inv_etk);
-  grad_param[1] = (((P[0] * dcm + P[1] * (cm + nu * dcm)) + P[2] * (h * dcm - 0.5 * cm)) +
-                   ((P[3] * dcb + P[4] * (cb + nu * dcb)) + P[5] * (h * dcb - 0.5 * cb))) -
-                  P[6] * cs * inv_1pn;
-  grad_param[2] = ((Lm + 3.0 * Lb) + Ls) * (E * k * inv_etk);
-  grad_param[3] = Ls * (E * t * inv_etk);
+  plate_adjoint_params(P, E, nu, t, k, grad_param);
   const double g3x = -((gxl[0] + gxl[2]) + gxl[4]), g3y = -((gxl[1] + gxl[3]) + gxl[5]);
   gX[0][0] = gxl[0]; gX[0][1] = gxl[1];
   gX[1][0] = gxl[2]; gX[1][1] = gxl[3];
@@ -404,32 +397,45 @@ __host__ __device__ inline void plate_adjoint_finish_flat(const double P[7], con
   for (int a = 0; a < 4; ++a) gX[a][2] = 0.0;
 }
 
-// Compliance by strain energy: the share of integration point ip in
+// Shear edge vectors of an element (plate_shear_vectors): v_a = (+-1/2, e12 or
+// e43), u_a = (+-1/2, e14 or e23).
+struct PlateEdges {
+  double e12[2], e43[2], e14[2], e23[2];
+};
+__host__ __device__ inline PlateEdges plate_edges(const double xl[6]) {
+  const double q = 0.25;
+  PlateEdges o;
+  o.e12[0] = -(xl[1] - xl[3]) * q; o.e12[1] = (xl[0] - xl[2]) * q;
+  o.e43[0] = -xl[5] * q;           o.e43[1] = xl[4] * q;
+  o.e14[0] = -(xl[1] - xl[5]) * q; o.e14[1] = (xl[0] - xl[4]) * q;
+  o.e23[0] = -xl[3] * q;           o.e23[1] = xl[2] * q;
+  return o;
+}
+
+// Compliance by strain energy: the share of the integration point (r, s) in
 // L = -u_l^T k u_l, with U[a] = (u, v, w, theta_x, theta_y, theta_z) the
-// local-frame displacements of node a, plus the drilling term of node ip.
-// Adds to P, gxl, hx, hy what plate_block_adjoint_q adds over the sixteen
-// blocks for G = -u_p u_q^T, without forming a block: each block term is a
-// bilinear form in nodal values, so its contraction with u u^T is the point's
-// quadratic form in the strains
+// local-frame displacements of node a.  Adds to P, gxl, hx, hy what
+// plate_block_adjoint_q adds over the sixteen blocks for G = -u_p u_q^T (but the
+// drilling term: plate_compliance_drilling), without forming a block: each block
+// term is a bilinear form in nodal values, so its contraction with u u^T is the
+// point's quadratic form in the strains
 //   membrane eps = (ux, vy, uy + vx), bending kappa = (ay, -bx, ax - by)
 //   (a = theta_x, b = theta_y), shear gamma_r = mr rho, gamma_s = ms sigma
 // (rho, sigma: the MITC4 tying sums of the shear vectors against U), and
 // every derivative follows from the strains, the stress resultants and the
 // natural-coordinate derivatives of U:
 //   * P from the squared strains;
-//   * the point adjoints of plate_point_reverse: det from the energy density,
-//     the inverse Jacobian from resultant x natural derivative, mr and ms
-//     from the shear strains;
+//   * the point's adjoints: det from the energy density, the inverse Jacobian from
+//     resultant x natural derivative, mr and ms from the shear strains, and from
+//     them the local coordinates (as plate_point_reverse, with the point's own
+//     Jacobian, reciprocals and lengths);
 //   * the shear vectors from the tying sums;
 //   * hx, hy = -2 sum_a (x_a x f_a)_{x,y} over the translation and rotation
 //     triples, f = k u_l the local nodal forces (their point share here).
-__host__ __device__ inline void plate_compliance_point(const double xl[6], int ip, const PlateMat& m,
-                                                       const PlateShear& sv, const double U[4][6], double P[7],
+__host__ __device__ inline void plate_compliance_point(const double xl[6], double r, double s, const PlateMat& m,
+                                                       const PlateEdges& ed, const double U[4][6], double P[7],
                                                        double gxl[6], double& hx, double& hy) {
   const double x1 = xl[0], y1 = xl[1], x2 = xl[2], y2 = xl[3], x4 = xl[4], y4 = xl[5];
-  const double gs = sqrt(double(ONE_THIRD_F32));
-  const double r = (ip == 0 || ip == 3) ? gs : -gs;
-  const double s = (ip < 2) ? gs : -gs;
   const double q4 = 0.25;
   const double pr = 1.0 + r, mr_ = 1.0 - r, ps = 1.0 + s, ms_ = 1.0 - s;
   const double usx = (x1 * ps - x2 * ps) + x4 * ms_, usy = (y1 * ps - y2 * ps) + y4 * ms_;
@@ -438,17 +444,21 @@ __host__ __device__ inline void plate_compliance_point(const double xl[6], int i
   const double det = j00 * j11 - j01 * j10;
   const double rdet = 1.0 / det;
   const double i00 = j11 * rdet, i01 = -j01 * rdet, i10 = -j10 * rdet, i11 = j00 * rdet;
-  const double mr = sqrt(urx * urx + ury * ury) * 0.125 * rdet, ms = sqrt(usx * usx + usy * usy) * 0.125 * rdet;
+  // MITC4 lengths and their reciprocals (0 where the length is 0)
+  const double qr = urx * urx + ury * ury, qs = usx * usx + usy * usy;
+  const double rqr = qr > 0.0 ? rsqrt(qr) : 0.0, rqs = qs > 0.0 ? rsqrt(qs) : 0.0;
+  const double r8 = 0.125 * rdet;
+  const double mr = (qr * rqr) * r8, ms = (qs * rqs) * r8;
   const double dr[4] = {q4 * ps, -q4 * ps, -q4 * ms_, q4 * ms_};
   const double ds[4] = {q4 * pr, q4 * mr_, -q4 * mr_, -q4 * pr};
-  const double fa[4] = {ps, ps, ms_, ms_}, fb[4] = {pr, mr_, mr_, pr};
   // natural derivatives of u, v, theta_x, theta_y
   const int comp[4] = {0, 1, 3, 4};
   double fr[4], fs[4];
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
-    fr[f] = ((dr[0] * U[0][comp[f]] + dr[1] * U[1][comp[f]]) + dr[2] * U[2][comp[f]]) + dr[3] * U[3][comp[f]];
-    fs[f] = ((ds[0] * U[0][comp[f]] + ds[1] * U[1][comp[f]]) + ds[2] * U[2][comp[f]]) + ds[3] * U[3][comp[f]];
+    const int c = comp[f];
+    fr[f] = q4 * (ps * (U[0][c] - U[1][c]) + ms_ * (U[3][c] - U[2][c]));
+    fs[f] = q4 * (pr * (U[0][c] - U[3][c]) + mr_ * (U[1][c] - U[2][c]));
   }
   const double ux = i00 * fr[0] + i01 * fs[0], uy = i10 * fr[0] + i11 * fs[0];
   const double vx = i00 * fr[1] + i01 * fs[1], vy = i10 * fr[1] + i11 * fs[1];
@@ -456,70 +466,97 @@ __host__ __device__ inline void plate_compliance_point(const double xl[6], int i
   const double bx = i00 * fr[3] + i01 * fs[3], by = i10 * fr[3] + i11 * fs[3];
   // stress resultants: derivatives of the energy density phi with respect to
   // ux (Nux), vy (Nvy), uy and vx (Nxy), ay (May), bx (Mbx), ax (Mxy; by: -Mxy)
+  const double exy = uy + vx, kxy = ax - by;
   const double Nux = 2.0 * (m.cm00 * ux + m.cm01 * vy);
   const double Nvy = 2.0 * (m.cm00 * vy + m.cm01 * ux);
-  const double Nxy = 2.0 * m.cm22 * (uy + vx);
+  const double Nxy = 2.0 * m.cm22 * exy;
   const double May = 2.0 * (m.cb00 * ay - m.cb01 * bx);
   const double Mbx = 2.0 * (m.cb00 * bx - m.cb01 * ay);
-  const double Mxy = 2.0 * m.cb22 * (ax - by);
-  const double phi = 0.5 * (((Nux * ux + Nvy * vy) + Nxy * (uy + vx)) + ((May * ay + Mbx * bx) + Mxy * (ax - by)));
+  const double Mxy = 2.0 * m.cb22 * kxy;
+  const double phi = 0.5 * (((Nux * ux + Nvy * vy) + Nxy * exy) + ((May * ay + Mbx * bx) + Mxy * kxy));
   // transverse shear: tying sums of the shear vectors against (w, theta_x, theta_y)
-  double sp[4], tp[4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    sp[a] = (sv.v[a][0] * U[a][2] + sv.v[a][1] * U[a][3]) + sv.v[a][2] * U[a][4];
-    tp[a] = (sv.u[a][0] * U[a][2] + sv.u[a][1] * U[a][3]) + sv.u[a][2] * U[a][4];
-  }
-  const double rho = ps * (sp[0] + sp[1]) + ms_ * (sp[2] + sp[3]);
-  const double sig = pr * (tp[0] + tp[3]) + mr_ * (tp[1] + tp[2]);
+  const double t12 = 0.5 * (U[0][2] - U[1][2]) + (ed.e12[0] * (U[0][3] + U[1][3]) + ed.e12[1] * (U[0][4] + U[1][4]));
+  const double t43 = 0.5 * (U[3][2] - U[2][2]) + (ed.e43[0] * (U[2][3] + U[3][3]) + ed.e43[1] * (U[2][4] + U[3][4]));
+  const double t14 = 0.5 * (U[0][2] - U[3][2]) + (ed.e14[0] * (U[0][3] + U[3][3]) + ed.e14[1] * (U[0][4] + U[3][4]));
+  const double t23 = 0.5 * (U[1][2] - U[2][2]) + (ed.e23[0] * (U[1][3] + U[2][3]) + ed.e23[1] * (U[1][4] + U[2][4]));
+  const double rho = ps * t12 + ms_ * t43, sig = pr * t14 + mr_ * t23;
   const double gr = mr * rho, gz = ms * sig;
   const double w = det;
   // constitutive partials
+  const double g2 = gr * gr + gz * gz;
   P[0] -= w * (ux * ux + vy * vy);
   P[1] -= w * (2.0 * ux * vy);
-  P[2] -= w * ((uy + vx) * (uy + vx));
+  P[2] -= w * (exy * exy);
   P[3] -= w * (ay * ay + bx * bx);
   P[4] += w * (2.0 * ay * bx);
-  P[5] -= w * ((ax - by) * (ax - by));
-  P[6] -= w * (gr * gr + gz * gz);
-  // point adjoints -> local coordinates
+  P[5] -= w * (kxy * kxy);
+  P[6] -= w * g2;
+  // the point's adjoints: det, inverse Jacobian, mr and ms
   const double cs2 = 2.0 * m.cs;
-  double s7[7];
-  s7[0] = -(phi + m.cs * (gr * gr + gz * gz));
-  s7[1] = -w * (((Nux * fr[0] + Nxy * fr[1]) + Mxy * fr[2]) + Mbx * fr[3]);
-  s7[2] = -w * (((Nux * fs[0] + Nxy * fs[1]) + Mxy * fs[2]) + Mbx * fs[3]);
-  s7[3] = -w * (((Nxy * fr[0] + Nvy * fr[1]) + May * fr[2]) - Mxy * fr[3]);
-  s7[4] = -w * (((Nxy * fs[0] + Nvy * fs[1]) + May * fs[2]) - Mxy * fs[3]);
-  s7[5] = -w * cs2 * gr * rho;
-  s7[6] = -w * cs2 * gz * sig;
-  plate_point_reverse(xl, ip, s7, gxl);
-  // shear vectors, and this point's share of the nodal forces f = k u_l
-  const double cr = -w * cs2 * gr * mr, cz = -w * cs2 * gz * ms;  // dL/d(tying sums) per unit multiplier
+  const double g_i00 = -w * (((Nux * fr[0] + Nxy * fr[1]) + Mxy * fr[2]) + Mbx * fr[3]);
+  const double g_i01 = -w * (((Nux * fs[0] + Nxy * fs[1]) + Mxy * fs[2]) + Mbx * fs[3]);
+  const double g_i10 = -w * (((Nxy * fr[0] + Nvy * fr[1]) + May * fr[2]) - Mxy * fr[3]);
+  const double g_i11 = -w * (((Nxy * fs[0] + Nvy * fs[1]) + May * fs[2]) - Mxy * fs[3]);
+  const double wr = -w * cs2 * gr, wz = -w * cs2 * gz;
+  const double g_mr = wr * rho, g_ms = wz * sig;
+  double g_det = -(phi + m.cs * g2);
+  g_det -= (g_mr * mr + g_ms * ms) * rdet;
+  g_det -= (((g_i00 * i00 + g_i01 * i01) + g_i10 * i10) + g_i11 * i11) * rdet;
+  const double g_sqr = g_mr * r8 * rqr, g_sqs = g_ms * r8 * rqs;
+  const double kux = (g_i11 * rdet + g_det * j11) * q4 + g_sqs * usx;
+  const double kuy = (-g_i01 * rdet - g_det * j10) * q4 + g_sqs * usy;
+  const double krx = (-g_i10 * rdet - g_det * j01) * q4 + g_sqr * urx;
+  const double kry = (g_i00 * rdet + g_det * j00) * q4 + g_sqr * ury;
+  gxl[0] += kux * ps + krx * pr;
+  gxl[1] += kuy * ps + kry * pr;
+  gxl[2] += -kux * ps + krx * mr_;
+  gxl[3] += -kuy * ps + kry * mr_;
+  gxl[4] += kux * ms_ - krx * pr;
+  gxl[5] += kuy * ms_ - kry * pr;
+  // shear edge vectors: dL/d(tying sums) against the edges' rotation sums, a
+  // quarter of the edge
+  const double c12 = (wr * mr) * ps * q4, c43 = (wr * mr) * ms_ * q4, c14 = (wz * ms) * pr * q4, c23 = (wz * ms) * mr_ * q4;
+  const double a12 = c12 * (U[0][3] + U[1][3]), b12 = c12 * (U[0][4] + U[1][4]);
+  const double a43 = c43 * (U[2][3] + U[3][3]), b43 = c43 * (U[2][4] + U[3][4]);
+  const double a14 = c14 * (U[0][3] + U[3][3]), b14 = c14 * (U[0][4] + U[3][4]);
+  const double a23 = c23 * (U[1][3] + U[2][3]), b23 = c23 * (U[1][4] + U[2][4]);
+  gxl[0] += b12 + b14;
+  gxl[1] -= a12 + a14;
+  gxl[2] += b23 - b12;
+  gxl[3] += a12 - a23;
+  gxl[4] += b43 - b14;
+  gxl[5] += a14 - a43;
+  // this point's share of the nodal forces f = k u_l
   const double hw = 0.5 * w;
+  const double sr = (w * m.cs) * gr * mr, sz = (w * m.cs) * gz * ms;  // per unit tying sum
+  const double fa[4] = {ps, ps, ms_, ms_}, fb[4] = {pr, mr_, mr_, pr};
   double ex = 0.0, ey = 0.0;
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
-    const double dsp = cr * fa[a], dtp = cz * fb[a];
-    plate_shear_vector_adjoint(a, dsp * U[a][3], dsp * U[a][4], dtp * U[a][3], dtp * U[a][4], gxl);
-    const double dxa = i00 * dr[a] + i01 * ds[a], dya = i10 * dr[a] + i11 * ds[a];
-    const double cv = (w * m.cs) * gr * (fa[a] * mr), cu = (w * m.cs) * gz * (fb[a] * ms);
-    const double fu = hw * (Nux * dxa + Nxy * dya);
-    const double fv = hw * (Nxy * dxa + Nvy * dya);
-    const double fw = cv * sv.v[a][0] + cu * sv.u[a][0];
-    const double fta = hw * (Mxy * dxa + May * dya) + (cv * sv.v[a][1] + cu * sv.u[a][1]);
-    const double ftb = hw * (Mbx * dxa - Mxy * dya) + (cv * sv.v[a][2] + cu * sv.u[a][2]);
+    const double dxa = hw * (i00 * dr[a] + i01 * ds[a]), dya = hw * (i10 * dr[a] + i11 * ds[a]);
+    const double cv = sr * fa[a], cu = sz * fb[a];
+    const double* ev = a < 2 ? ed.e12 : ed.e43;
+    const double* eu = (a == 0 || a == 3) ? ed.e14 : ed.e23;
+    const double fu = Nux * dxa + Nxy * dya;
+    const double fv = Nxy * dxa + Nvy * dya;
+    const double fw = ((a == 0 || a == 3) ? 0.5 : -0.5) * cv + (a < 2 ? 0.5 : -0.5) * cu;
+    const double fta = (Mxy * dxa + May * dya) + (cv * ev[0] + cu * eu[0]);
+    const double ftb = (Mbx * dxa - Mxy * dya) + (cv * ev[1] + cu * eu[1]);
     ex += (U[a][1] * fw - U[a][2] * fv) - U[a][5] * ftb;
     ey += (U[a][2] * fu - U[a][0] * fw) + U[a][5] * fta;
   }
-  // drilling force of node ip (KROT6 on its theta_z)
-  const double tzx = ip == 0 ? U[0][3] : (ip == 1 ? U[1][3] : (ip == 2 ? U[2][3] : U[3][3]));
-  const double tzy = ip == 0 ? U[0][4] : (ip == 1 ? U[1][4] : (ip == 2 ? U[2][4] : U[3][4]));
-  const double tzz = ip == 0 ? U[0][5] : (ip == 1 ? U[1][5] : (ip == 2 ? U[2][5] : U[3][5]));
-  const double fz = KROT6 * tzz;
-  ex += tzy * fz;
-  ey -= tzx * fz;
   hx -= 2.0 * ex;
   hy -= 2.0 * ey;
+}
+
+// the drilling forces' share (KROT6 on each node's theta_z)
+__host__ __device__ inline void plate_compliance_drilling(const double U[4][6], double& hx, double& hy) {
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const double fz = KROT6 * U[a][5];
+    hx -= 2.0 * (U[a][4] * fz);
+    hy += 2.0 * (U[a][3] * fz);
+  }
 }
 
 }  // namespace fem
