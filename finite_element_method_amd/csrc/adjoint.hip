@@ -48,6 +48,7 @@ struct AdjArgs {
   const uint2* kpack;
   const uint32_t* eorder;  // flat plates: the elements in workgroup order
   const int64_t* row_ptr;
+  const uint4* rec;  // BlockPos records, or null
   double* dparam;  // n x params_per, may be null
   double* xs;      // coordinate-gradient rows in node-major slots (3 doubles each), may be null
   const uint32_t* xpos;  // per (element, node) of this type: its slot in xs
@@ -63,28 +64,79 @@ __device__ inline unsigned xcd_block(unsigned b, unsigned nb) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + j;
 }
 
-// global-frame 6x6 gradient block of node pair block k, rows of node a.  The
-// block's entries of row i are contiguous in the CSR row: load the run, then
-// place it by the row mask.
-// With g_bytes set the run is read in 16-byte pairs (and one 8-byte tail) by
-// buffer loads, range-checked against g: half the memory requests of one load
-// per value, and the requests, not the bytes, bound this gather.
-__device__ inline void gather_block(const AdjArgs& A, uint32_t k, uint32_t a, double G[36]) {
-  const uint64_t um = A.bmask[k];
-  const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(A.g), 0, int(A.g_bytes), 0x00020000);
-  uint32_t bo[3];  // the block's six row offsets, two per word (boff rows start 4-byte aligned)
+// Where the block of an element's node pair sits: CSR positions of its six rows'
+// runs and its union mask, in one 32-byte record per (element, pair).  Looked up
+// through the pattern (pair -> block -> mask and row offsets -> row pointers)
+// the same costs four loads that wait for each other and 72 gathered bytes.
+// Frame of 33 x 33 x 33 nodes: 38.6 -> 34.1 us.
+struct BlockPos {
+  uint32_t pos[6];
+  uint64_t mask;
+};
+__device__ inline BlockPos block_pos(const AdjArgs& A, size_t pair) {
+  const uint4 a = A.rec[2 * pair], b = A.rec[2 * pair + 1];
+  return {{a.x, a.y, a.z, a.w, b.x, b.y}, uint64_t(b.z) | uint64_t(b.w) << 32};
+}
+
+__global__ __launch_bounds__(256) void adjoint_records_kernel(const uint32_t* __restrict__ conn,
+                                                              const uint32_t* __restrict__ bid,
+                                                              const uint64_t* __restrict__ bmask,
+                                                              const uint16_t* __restrict__ boff,
+                                                              const int64_t* __restrict__ row_ptr, size_t n_pairs,
+                                                              int nodes, uint4* __restrict__ rec) {
+  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n_pairs) return;
+  const size_t e = i / (nodes * nodes);
+  const uint32_t k = bid[i], a = conn[e * nodes + (i % (nodes * nodes)) / nodes];
+  uint32_t pos[6];
 #pragma unroll
-  for (int m = 0; m < 3; ++m) bo[m] = reinterpret_cast<const uint32_t*>(A.boff + 6 * size_t(k))[m];
+  for (int r = 0; r < 6; ++r) pos[r] = uint32_t(row_ptr[6 * size_t(a) + r] + boff[6 * size_t(k) + r]);
+  const uint64_t m = bmask[k];
+  rec[2 * i] = make_uint4(pos[0], pos[1], pos[2], pos[3]);
+  rec[2 * i + 1] = make_uint4(pos[4], pos[5], uint32_t(m), uint32_t(m >> 32));
+}
+
+// the same from the pattern's arrays (values past 32-bit positions have no records)
+__device__ inline void gather_block_far(const AdjArgs& A, uint32_t k, uint32_t a, double G[36]) {
+  const uint64_t um = A.bmask[k];
 #pragma unroll
   for (int i = 0; i < 6; ++i) {
     const uint32_t mi = uint32_t(um >> (6 * i)) & 63u;
+    const double* src = A.g + A.row_ptr[6 * size_t(a) + i] + A.boff[6 * size_t(k) + i];
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      G[i * 6 + j] = ((mi >> j) & 1u) ? src[__builtin_popcount(mi & ((1u << j) - 1u))] : 0.0;
+  }
+}
+
+// global-frame 6x6 gradient block at b: the block's entries of row i are
+// contiguous in the CSR row; load the run, then place it by the row mask.
+// With g_bytes set the run is read in 16-byte pairs (and one 8-byte tail) by
+// buffer loads, range-checked against g: half the memory requests of one load
+// per value, and the requests, not the bytes, bound this gather.
+__device__ inline void gather_block(const AdjArgs& A, const BlockPos& b, double G[36]) {
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(A.g), 0, int(A.g_bytes), 0x00020000);
+  constexpr uint64_t FULL = (1ull << 36) - 1ull;
+  if (A.g_bytes && __all(b.mask == FULL)) {  // shells: every run is the row itself
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+      for (int c = 0; c < 6; c += 2) {
+        const double2 w = __builtin_bit_cast(
+            double2, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 8u * (b.pos[i] + uint32_t(c)), 0, 0));
+        G[6 * i + c] = w.x;
+        G[6 * i + c + 1] = w.y;
+      }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    const uint32_t mi = uint32_t(b.mask >> (6 * i)) & 63u;
     const int n = __builtin_popcount(mi);
-    const uint32_t off_i = (bo[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
-    const int64_t pos = A.row_ptr[6 * size_t(a) + i] + off_i;
     double v[6];
     if (A.g_bytes) {
-      const uint32_t byte = uint32_t(pos) * 8u;
+      const uint32_t byte = b.pos[i] * 8u;
 #pragma unroll
       for (int c = 0; c < 6; c += 2) {
         v[c] = 0.0;
@@ -98,21 +150,20 @@ __device__ inline void gather_block(const AdjArgs& A, uint32_t k, uint32_t a, do
         }
       }
     } else {
-      const double* src = A.g + pos;
+      const double* src = A.g + b.pos[i];
 #pragma unroll
       for (int c = 0; c < 6; ++c) v[c] = c < n ? src[c] : 0.0;
     }
+    // open the gaps of the mask from the left
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
-      const int c = __builtin_popcount(mi & ((1u << j) - 1u));
-      double x = v[0];
+      const bool on = (mi >> j) & 1u;
 #pragma unroll
-      for (int cc = 1; cc <= j; ++cc) x = c == cc ? v[cc] : x;
-      G[i * 6 + j] = ((mi >> j) & 1u) ? x : 0.0;
+      for (int c = 5; c > j; --c) v[c] = on ? v[c] : v[c - 1];
+      G[i * 6 + j] = on ? v[j] : 0.0;
     }
   }
 }
-
 __device__ inline bool is_identity(const double R[9]) {
   return R[0] == 1.0 && R[4] == 1.0 && R[8] == 1.0 && R[1] == 0.0 && R[2] == 0.0 && R[3] == 0.0 && R[5] == 0.0 &&
          R[6] == 0.0 && R[7] == 0.0;
@@ -167,34 +218,6 @@ __device__ inline double quad_sum(double v) {
 }
 
 // ---------------------------------------------------------------- plates
-// point data of the block's 64 elements: lane p of an element computes point p
-constexpr int PA_POINT = 9;  // double2 per (element, point): plate_point's 17 values and a pad
-__device__ inline void store_point(double2* dst, const fem::PlatePoint& g) {
-  const double v[18] = {g.w, g.dx[0], g.dx[1], g.dx[2], g.dx[3], g.dy[0], g.dy[1], g.dy[2], g.dy[3],
-                        g.al[0], g.al[1], g.al[2], g.al[3], g.be[0], g.be[1], g.be[2], g.be[3], 0.0};
-#pragma unroll
-  for (int k = 0; k < PA_POINT; ++k) dst[k] = make_double2(v[2 * k], v[2 * k + 1]);
-}
-__device__ inline fem::PlatePoint load_point(const double2* src) {
-  double v[18];
-#pragma unroll
-  for (int k = 0; k < PA_POINT; ++k) {
-    const double2 x = src[k];
-    v[2 * k] = x.x;
-    v[2 * k + 1] = x.y;
-  }
-  fem::PlatePoint g;
-  g.w = v[0];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    g.dx[a] = v[1 + a];
-    g.dy[a] = v[5 + a];
-    g.al[a] = v[9 + a];
-    g.be[a] = v[13 + a];
-  }
-  return g;
-}
-
 // element data of plate e: nodes, frame, local coordinates relative to node 3
 // (xl = x, y of nodes 1, 2, 4), parameters
 struct PlateElem {
@@ -258,99 +281,6 @@ __device__ inline void plate_write(const AdjArgs& A, size_t e, int p, bool live,
   }
 }
 
-// Plates in any frame: four lanes per element (lane p = row block of node p),
-// 64 elements per block; gradient blocks gathered through the block maps.
-__global__ __launch_bounds__(256) void plate_adjoint_kernel(AdjArgs A) {
-  __shared__ double2 pts[64 * 4 * PA_POINT];
-  const unsigned b = xcd_block(blockIdx.x, gridDim.x);
-  const size_t e0 = size_t(b) * 64 + (threadIdx.x >> 2);
-  const int p = int(threadIdx.x & 3u);
-  const bool live = e0 < A.n;
-  const size_t e = live ? e0 : A.n - 1;  // dead lanes still take part in the lane sums
-  PlateElem el;
-  load_plate_elem<false>(A, e, el);
-  const uint32_t* nd = el.nd;
-  const double* R = el.R;
-  const bool ident = is_identity(R);
-  const double* xl = el.xl;
-  const fem::PlateMat mat = fem::plate_material(el.E, el.nu, el.t, el.k);
-  fem::PlateShear sv;
-  fem::plate_shear_vectors(xl, sv);
-  const uint32_t ap = p == 0 ? nd[0] : (p == 1 ? nd[1] : (p == 2 ? nd[2] : nd[3]));
-  // pass 1: integrals of row p; the point data of point p come from lane p
-  double2* my_pts = pts + (threadIdx.x >> 2) * 4 * PA_POINT;
-  {
-    fem::PlatePoint g;
-    fem::plate_point(xl, p, g);
-    store_point(my_pts + p * PA_POINT, g);
-  }
-  __syncthreads();
-  double acc[24];
-#pragma unroll
-  for (int i = 0; i < 24; ++i) acc[i] = 0.0;
-#pragma unroll 1
-  for (int ip = 0; ip < 4; ++ip) {
-    const fem::PlatePoint g = load_point(my_pts + ip * PA_POINT);
-    const double wdx = g.w * fem::sel4(g.dx[0], g.dx[1], g.dx[2], g.dx[3], p);
-    const double wdy = g.w * fem::sel4(g.dy[0], g.dy[1], g.dy[2], g.dy[3], p);
-    const double wal = g.w * fem::sel4(g.al[0], g.al[1], g.al[2], g.al[3], p);
-    const double wbe = g.w * fem::sel4(g.be[0], g.be[1], g.be[2], g.be[3], p);
-    fem::plate_row_accumulate(g, wdx, wdy, wal, wbe, acc);
-  }
-  // pass 2: gradient blocks of row p.  acc[] doubles as c[]: column q's
-  // integral coefficients replace its integrals once they are consumed.
-  double* c = acc;
-  double P[7], gxl[6], hx = 0.0, hy = 0.0;
-#pragma unroll
-  for (int i = 0; i < 7; ++i) P[i] = 0.0;
-#pragma unroll
-  for (int i = 0; i < 6; ++i) gxl[i] = 0.0;
-  double vp_[3], up_[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    vp_[i] = fem::sel4(sv.v[0][i], sv.v[1][i], sv.v[2][i], sv.v[3][i], p);
-    up_[i] = fem::sel4(sv.u[0][i], sv.u[1][i], sv.u[2][i], sv.u[3][i], p);
-  }
-  // one block per iteration (q is wave-uniform): only one block's temporaries live
-#pragma unroll 1
-  for (int q = 0; q < 4; ++q) {
-    double gl[36];
-    gather_block(A, A.bid[16 * e + 4 * p + q], ap, gl);
-    if (!ident) to_local(gl, R);
-    double Mq[6], vq[3], uq_[3], cq[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) Mq[k] = fem::sel4(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3], q);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      vq[i] = fem::sel4(sv.v[0][i], sv.v[1][i], sv.v[2][i], sv.v[3][i], q);
-      uq_[i] = fem::sel4(sv.u[0][i], sv.u[1][i], sv.u[2][i], sv.u[3][i], q);
-    }
-    fem::plate_block_adjoint_q(Mq, mat, vp_, up_, vq, uq_, p, q, gl, P, cq, gxl, hx, hy, true);
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) c[4 * k + j] = j == q ? cq[k] : c[4 * k + j];
-  }
-  // pass 3: reverse sweep over the integration points.  The sweep is linear in
-  // the seven adjoints of a point's forward quantities: the four rows' values
-  // are added first, and lane p sweeps point p.
-  {
-    double mine[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll 1
-    for (int ip = 0; ip < 4; ++ip) {
-      double s7[7];
-      fem::plate_point_scalars(load_point(my_pts + ip * PA_POINT), ip, p, c, s7);
-#pragma unroll
-      for (int k = 0; k < 7; ++k) {
-        const double tot = quad_sum(s7[k]);
-        mine[k] = ip == p ? tot : mine[k];
-      }
-    }
-    fem::plate_point_reverse(xl, p, mine, gxl);
-  }
-  plate_write(A, e, p, live, el, P, gxl, hx, hy);
-}
-
 // plate_write for a flat plate (identity frame, nodes in z = 0, no frame term)
 __device__ inline void plate_write_flat(const AdjArgs& A, size_t e, int p, bool live, double E, double nu, double t,
                                         double k, double P[7], double gxl[6]) {
@@ -369,7 +299,7 @@ __device__ inline void plate_write_flat(const AdjArgs& A, size_t e, int p, bool 
   }
 }
 
-// ------------------------------------------------ flat plates, dL/dK
+// ------------------------------------------------ plates, dL/dK
 // One wave per block, 16 elements, four lanes per element.  Lane p is row
 // block p while the gradient blocks are read and integration point p while
 // the integrals are swept back; the element's data meet in LDS:
@@ -423,7 +353,17 @@ __device__ inline void shear_vector_adjoint_lane(int a, double gv1, double gv2, 
   gxl[5] += gu1 * u14 - gv1 * v43;
 }
 
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void plate_adjoint_flat_kernel(AdjArgs A) {
+//
+// FLAT: every frame is the identity and the pattern has no coupling of membrane
+// and bending, 13 values per block.  Otherwise the block is read whole through
+// its record, turned to the element's frame, and the frame's own rotation
+// (hx, hy) is collected.  Bound: the lines of K's gradient between L2 and L1 (a
+// lane's row run of 48 bytes brings in 128 or 256) and FP64 arithmetic.  Shells
+// of 256 x 256: 140 -> 99 us, 128 x 128: 37 -> 31 us, up to 64 x 64: 25 -> 15 us
+// (before: 256-lane blocks whose point data, integrals and shear vectors sat in
+// 342 registers, one wave per SIMD; here they meet in LDS and two waves fit).
+template <bool FLAT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void plate_adjoint_kernel(AdjArgs A) {
   __shared__ double2 pts[16 * PF_PTS / 2];
   __shared__ double2 rows[16 * PF_ROWS / 2];
   const unsigned b = xcd_block(blockIdx.x, gridDim.x);
@@ -431,21 +371,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
   const int p = int(threadIdx.x & 3u);
   const size_t i0 = size_t(b) * 16 + le;
   const bool live = i0 < A.n;
-  const size_t e = A.eorder[live ? i0 : A.n - 1];  // dead lanes still take part in the lane sums
+  const size_t i = live ? i0 : A.n - 1;  // dead lanes still take part in the lane sums
+  size_t e = FLAT ? A.eorder[i] : i;
   // gradient-block positions first: the value loads wait on this one load only
-  const uint2 kr = A.kpack[4 * e + p];
+  const uint2 kr = FLAT ? A.kpack[4 * e + p] : make_uint2(0, 0);
   const uint32_t g0 = kr.x, kp = kr.y;
   const int nb = int(kp >> 24);
   double nxt[13], nxt2[13];
-  load_flat_k13(A.g + g0, nb, int(kp & 63u), nxt);
-  load_flat_k13(A.g + g0, nb, int((kp >> 6) & 63u), nxt2);
+  BlockPos pos{};
+  double R[9];
+  uint32_t ap = 0;
+  if (FLAT) {
+    load_flat_k13(A.g + g0, nb, int(kp & 63u), nxt);
+    load_flat_k13(A.g + g0, nb, int((kp >> 6) & 63u), nxt2);
+  } else {
+    if (A.rec) pos = block_pos(A, 16 * e + 4 * p);
+    ap = A.conn[4 * e + p];
+  }
   double xl[6];
   fem::PlateMat mat;
   {
     PlateElem el;
-    load_plate_elem<true>(A, e, el);
+    load_plate_elem<FLAT>(A, e, el);
 #pragma unroll
     for (int i = 0; i < 6; ++i) xl[i] = el.xl[i];
+    if (!FLAT) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) R[i] = el.R[i];
+    }
     mat = fem::plate_material(el.E, el.nu, el.t, el.k);
   }
   double* const ep = reinterpret_cast<double*>(pts) + le * PF_PTS;
@@ -511,16 +464,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
 #pragma unroll
   for (int i = 0; i < 6; ++i) gxl[i] = 0.0;
   double gv1 = 0.0, gv2 = 0.0, gu1 = 0.0, gu2 = 0.0;  // dL/d(v_p), dL/d(u_p), components 1 and 2
+  double hx = 0.0, hy = 0.0;                          // dL/d(rotation of the frame)
   // blocks (p, q): q is wave-uniform; block q + 1's values load during block q
 #pragma unroll 1
   for (int q = 0; q < 4; ++q) {
-    double G[13];
+    double G[13], gl[36];
+    if (FLAT) {
 #pragma unroll
-    for (int i = 0; i < 13; ++i) {
-      G[i] = nxt[i];
-      nxt[i] = nxt2[i];
+      for (int i = 0; i < 13; ++i) {
+        G[i] = nxt[i];
+        nxt[i] = nxt2[i];
+      }
+      if (q < 2) load_flat_k13(A.g + g0, nb, int((kp >> (6 * (q + 2))) & 63u), nxt2);
+    } else {
+      if (A.rec) {
+        gather_block(A, pos, gl);
+        if (q < 3) pos = block_pos(A, 16 * e + 4 * p + q + 1);
+      } else {
+        gather_block_far(A, A.bid[16 * e + 4 * p + q], ap, gl);
+      }
+      if (!is_identity(R)) to_local(gl, R);
+      G[0] = gl[0];
+      G[1] = gl[1];
+      G[2] = gl[6];
+      G[3] = gl[7];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) G[4 + 3 * i + j] = gl[(2 + i) * 6 + 2 + j];
     }
-    if (q < 2) load_flat_k13(A.g + g0, nb, int((kp >> (6 * (q + 2))) & 63u), nxt2);
     double2* r = reinterpret_cast<double2*>(er + p * 24 + 6 * q);
     const double2 m0 = r[0], m1 = r[1], m2 = r[2];
     const double Mxx = m0.x, Mxy = m0.y, Myx = m1.x, Myy = m1.y, Aq = m2.x, Bq = m2.y;
@@ -562,6 +534,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
     gu1 += sb * Gu[1];
     gu2 += sb * Gu[2];
     shear_vector_adjoint_lane(q, sa * vG[1], sa * vG[2], sb * uG[1], sb * uG[2], gxl);
+    if (!FLAT) {
+      double o[13], vps[3], ups[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        vps[i] = mat.cs * vp[i];
+        ups[i] = mat.cs * up[i];
+      }
+      fem::plate_block_entries(Mxx, Mxy, Myx, Myy, Aq, Bq, mat, vps, ups, vq, uq, o);
+      fem::plate_frame_adjoint(o, p == q ? fem::KROT6 : 0.0, gl, hx, hy);
+    }
   }
   shear_vector_adjoint_lane(p, gv1, gv2, gu1, gu2, gxl);
   __syncthreads();
@@ -638,7 +620,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
     for (int k = 1; k < 7; ++k) s7[k] *= w;
     fem::plate_point_reverse_r(xl, p, s7, rdet, rqr, rqs, gxl);
   }
-  // the parameters again (not held through the sweeps)
+  // the element's data again (not held through the sweeps)
+  if (!FLAT) {
+    asm volatile("" : "+v"(e));
+    PlateElem el;
+    load_plate_elem<false>(A, e, el);
+    plate_write(A, e, p, live, el, P, gxl, hx, hy);
+    return;
+  }
   plate_write_flat(A, e, p, live, A.params[4 * e], A.params[4 * e + 1], A.params[4 * e + 2], A.params[4 * e + 3], P,
                    gxl);
 }
@@ -801,7 +790,10 @@ __global__ __launch_bounds__(256) void beam_adjoint_kernel(AdjArgs A) {
     const int p = pq >> 1, q = pq & 1;
     double gl[36];
     if (MODE == MODE_DLDK) {
-      gather_block(A, A.bid[4 * e + pq], nd[p], gl);
+      if (A.rec)
+        gather_block(A, block_pos(A, 4 * e + pq), gl);
+      else
+        gather_block_far(A, A.bid[4 * e + pq], nd[p], gl);
       to_local(gl, R);
     } else {
       double up[6], uq[6];
@@ -876,6 +868,21 @@ std::string upload_adjoint_maps(Device* d, const AdjointMaps& am) {
     e = dupload(d->adj_eorder, am.eorder.data(), am.eorder.size());
     if (!e.empty()) return e;
   }
+  // block records of beams, and of plates where the flat kernel does not serve
+  for (int t = 0; t < 3; ++t) {
+    const size_t pairs = am.bid[t].size();
+    const bool want = pairs && t != TRUSS && !(t == PLATE && am.flat) && uint64_t(d->nnz) < (uint64_t(1) << 32);
+    // without room for the records the kernels look blocks up in the pattern
+    if (!dalloc(d->adj_rec[t], want ? 2 * pairs : 0).empty()) {
+      (void)hipGetLastError();
+      d->adj_rec[t] = nullptr;
+    }
+    if (!d->adj_rec[t]) continue;
+    adjoint_records_kernel<<<unsigned((pairs + 255) / 256), 256>>>(d->conn[t], d->adj_bid[t], d->adj_bmask, d->adj_boff,
+                                                                   d->row_ptr, pairs, NODES_PER[t], d->adj_rec[t]);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipDeviceSynchronize());
+  }
   d->adj_nxs = am.n_xs_rows;
   return dalloc(d->adj_xs, size_t(3 * am.n_xs_rows));
 }
@@ -901,6 +908,7 @@ std::string run_adjoint(Device* d, int mode, const double* g, double* const dpar
     A.kpack = reinterpret_cast<const uint2*>(d->adj_kpack);
     A.eorder = d->adj_eorder;
     A.row_ptr = d->row_ptr;
+    A.rec = d->adj_rec[t];
     A.dparam = dparam[t];
     A.xs = (dxyz && t != BEAM) ? d->adj_xs : nullptr;
     A.xpos = d->adj_xpos + d->adj_xoff[t];
@@ -910,10 +918,10 @@ std::string run_adjoint(Device* d, int mode, const double* g, double* const dpar
                     : 0u;
     if (t == PLATE) {
       const unsigned blocks = unsigned((n + 63) / 64);
-      if (mode == MODE_DLDK && d->adj_flat)
-        plate_adjoint_flat_kernel<<<unsigned((n + 15) / 16), 64, 0, s>>>(A);
-      else if (mode == MODE_DLDK) plate_adjoint_kernel<<<blocks, 256, 0, s>>>(A);
-      else {
+      if (mode == MODE_DLDK) {
+        auto kernel = d->adj_flat ? plate_adjoint_kernel<true> : plate_adjoint_kernel<false>;
+        kernel<<<unsigned((n + 15) / 16), 64, 0, s>>>(A);
+      } else {
         const bool few = n < PC_FEW;
         auto kernel = d->adj_flat ? (few ? plate_compliance_kernel<true, 4> : plate_compliance_kernel<true, 1>)
                                   : (few ? plate_compliance_kernel<false, 4> : plate_compliance_kernel<false, 1>);

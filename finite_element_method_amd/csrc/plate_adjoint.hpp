@@ -19,95 +19,6 @@
 
 namespace fem {
 
-// Reverse sweep of one integration point: the derivative with respect to xl of
-//   l = sum_q w [dx_p (cxx_q dx_q + cxy_q dy_q) + dy_p (cyx_q dx_q + cyy_q dy_q)
-//               + al_p cA_q al_q + be_p cB_q be_q]
-// with c = {cxx[4], cxy[4], cyx[4], cyy[4], cA[4], cB[4]} held fixed, where
-// w, dx, dy, al, be are the per-point data of plate_point (w = det J).  It
-// runs in two parts.  The second is linear in the seven adjoints of the
-// point's forward quantities (det, the inverse Jacobian, the two MITC4
-// multipliers), so the four row lanes of an element add their seven values
-// first and run the second part once per point.
-// Part 1: the seven adjoints s7 = (g_det, g_i00, g_i01, g_i10, g_i11, g_mr,
-// g_ms) of row p at point ip, from that point's data g (plate_point).
-__host__ __device__ inline void plate_point_scalars(const PlatePoint& g, int ip, int p, const double c[24],
-                                                    double s7[7]) {
-  const double gs = sqrt(double(ONE_THIRD_F32));
-  const double r = (ip == 0 || ip == 3) ? gs : -gs;
-  const double s = (ip < 2) ? gs : -gs;
-  const double q4 = 0.25;
-  const double pr = 1.0 + r, mr_ = 1.0 - r, ps = 1.0 + s, ms_ = 1.0 - s;
-  const double dr[4] = {q4 + q4 * s, -(q4 + q4 * s), -(q4 - q4 * s), q4 - q4 * s};
-  const double ds[4] = {q4 + q4 * r, q4 - q4 * r, -(q4 - q4 * r), -(q4 + q4 * r)};
-  const double fa[4] = {ps, ps, ms_, ms_}, fb[4] = {pr, mr_, mr_, pr};
-  const double det = g.w;
-  const double dxp = sel4(g.dx[0], g.dx[1], g.dx[2], g.dx[3], p), dyp = sel4(g.dy[0], g.dy[1], g.dy[2], g.dy[3], p);
-  const double alp = sel4(g.al[0], g.al[1], g.al[2], g.al[3], p), bep = sel4(g.be[0], g.be[1], g.be[2], g.be[3], p);
-  double SX = 0.0, SY = 0.0, SA = 0.0, SB = 0.0;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    SX += c[q] * g.dx[q] + c[4 + q] * g.dy[q];
-    SY += c[8 + q] * g.dx[q] + c[12 + q] * g.dy[q];
-    SA += c[16 + q] * g.al[q];
-    SB += c[20 + q] * g.be[q];
-  }
-  double g_det = ((dxp * SX + dyp * SY) + alp * SA) + bep * SB;
-  double g_i00 = 0.0, g_i01 = 0.0, g_i10 = 0.0, g_i11 = 0.0, g_mr = 0.0, g_ms = 0.0;
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const bool self = a == p;
-    const double gdx = det * ((dxp * c[a] + dyp * c[8 + a]) + (self ? SX : 0.0));
-    const double gdy = det * ((dxp * c[4 + a] + dyp * c[12 + a]) + (self ? SY : 0.0));
-    const double gal = det * (alp * c[16 + a] + (self ? SA : 0.0));
-    const double gbe = det * (bep * c[20 + a] + (self ? SB : 0.0));
-    g_i00 += gdx * dr[a];
-    g_i01 += gdx * ds[a];
-    g_i10 += gdy * dr[a];
-    g_i11 += gdy * ds[a];
-    g_mr += gal * fa[a];
-    g_ms += gbe * fb[a];
-  }
-  s7[0] = g_det; s7[1] = g_i00; s7[2] = g_i01; s7[3] = g_i10; s7[4] = g_i11; s7[5] = g_mr; s7[6] = g_ms;
-}
-
-// Part 2: from the seven adjoints of point ip (summed over rows) to xl.
-__host__ __device__ inline void plate_point_reverse(const double xl[6], int ip, const double s7[7], double gxl[6]) {
-  const double x1 = xl[0], y1 = xl[1], x2 = xl[2], y2 = xl[3], x4 = xl[4], y4 = xl[5];
-  const double gs = sqrt(double(ONE_THIRD_F32));
-  const double r = (ip == 0 || ip == 3) ? gs : -gs;
-  const double s = (ip < 2) ? gs : -gs;
-  const double q4 = 0.25;
-  const double pr = 1.0 + r, mr_ = 1.0 - r, ps = 1.0 + s, ms_ = 1.0 - s;
-  const double usx = (x1 * ps - x2 * ps) + x4 * ms_, usy = (y1 * ps - y2 * ps) + y4 * ms_;
-  const double urx = (x1 * pr + x2 * mr_) - x4 * pr, ury = (y1 * pr + y2 * mr_) - y4 * pr;
-  const double j00 = usx * q4, j01 = usy * q4, j10 = urx * q4, j11 = ury * q4;
-  const double det = j00 * j11 - j01 * j10;
-  const double rdet = 1.0 / det;
-  const double i00 = j11 * rdet, i01 = -j01 * rdet, i10 = -j10 * rdet, i11 = j00 * rdet;
-  const double sqr = sqrt(urx * urx + ury * ury), sqs = sqrt(usx * usx + usy * usy);
-  const double m_r = sqr * 0.125 * rdet, m_s = sqs * 0.125 * rdet;
-  double g_det = s7[0];
-  const double g_i00 = s7[1], g_i01 = s7[2], g_i10 = s7[3], g_i11 = s7[4], g_mr = s7[5], g_ms = s7[6];
-  g_det -= (g_mr * m_r + g_ms * m_s) * rdet;
-  const double g_sqr = g_mr * 0.125 * rdet, g_sqs = g_ms * 0.125 * rdet;
-  double g_j11 = g_i00 * rdet, g_j01 = -g_i01 * rdet, g_j10 = -g_i10 * rdet, g_j00 = g_i11 * rdet;
-  g_det -= (((g_i00 * i00 + g_i01 * i01) + g_i10 * i10) + g_i11 * i11) * rdet;
-  g_j00 += g_det * j11;
-  g_j11 += g_det * j00;
-  g_j01 -= g_det * j10;
-  g_j10 -= g_det * j01;
-  const double kux = g_j00 * q4 + (sqs > 0.0 ? g_sqs * usx / sqs : 0.0);
-  const double kuy = g_j01 * q4 + (sqs > 0.0 ? g_sqs * usy / sqs : 0.0);
-  const double krx = g_j10 * q4 + (sqr > 0.0 ? g_sqr * urx / sqr : 0.0);
-  const double kry = g_j11 * q4 + (sqr > 0.0 ? g_sqr * ury / sqr : 0.0);
-  gxl[0] += kux * ps + krx * pr;
-  gxl[1] += kuy * ps + kry * pr;
-  gxl[2] += -kux * ps + krx * mr_;
-  gxl[3] += -kuy * ps + kry * mr_;
-  gxl[4] += kux * ms_ - krx * pr;
-  gxl[5] += kuy * ms_ - kry * pr;
-}
-
 // plate_point (element_math.hpp) that also returns the reciprocals the
 // reverse sweep of the point needs (plate_point_reverse_r)
 __host__ __device__ inline void plate_point_x(const double xl[6], int ip, PlatePoint& o, double& rdet_o,
@@ -141,7 +52,10 @@ __host__ __device__ inline void plate_point_x(const double xl[6], int ip, PlateP
   rqs = sqs > 0.0 ? 1.0 / sqs : 0.0;
 }
 
-// plate_point_reverse with the point's reciprocals given: rdet = 1 / det J and
+// Reverse sweep of integration point ip: from the adjoints s7 = (g_det, g_i00,
+// g_i01, g_i10, g_i11, g_mr, g_ms) of its forward quantities (det, the inverse
+// Jacobian, the two MITC4 multipliers), summed over the element's rows, to
+// gxl.  The point's reciprocals are given: rdet = 1 / det J and
 // rqr, rqs = 1 / |(cx + r bx, cy + r by)|, 1 / |(ax + s bx, ay + s by)| (the
 // MITC4 lengths; 0 where the length is 0), as the forward point formed them
 __host__ __device__ inline void plate_point_reverse_r(const double xl[6], int ip, const double s7[7], double rdet,
@@ -180,135 +94,29 @@ __host__ __device__ inline void plate_point_reverse_r(const double xl[6], int ip
   gxl[5] += kuy * ms_ - kry * pr;
 }
 
-// adjoint of the shear vectors of node a (components 1 and 2; component 0 is
-// the constant +-1/2): gv = dL/dv_a, gu = dL/du_a, mapped onto xl through
-//   e12 = (-(y1-y2), x1-x2)/4, e43 = (-y4, x4)/4, e14 = (-(y1-y4), x1-x4)/4, e23 = (-y2, x2)/4
-__host__ __device__ inline void plate_shear_vector_adjoint(int a, double gv1, double gv2, double gu1, double gu2,
-                                                           double gxl[6]) {
-  const double q = 0.25;
-  if (a <= 1) {  // v_a carries e12
-    gxl[1] -= gv1 * q; gxl[3] += gv1 * q;
-    gxl[0] += gv2 * q; gxl[2] -= gv2 * q;
-  } else {       // e43
-    gxl[5] -= gv1 * q;
-    gxl[4] += gv2 * q;
+// h += antisymmetric parts (omega_x, omega_y) of K G^T + K^T G for a block's four
+// pairs of 3x3 sub-blocks K, G (gl: 6x6 row-major, local frame).  K is given by
+// its entries o (plate_block_entries: (u, v) x (u, v) and (w, theta_x, theta_y) x
+// the same) and its drilling entry; the products with its zeros are left out.
+__host__ __device__ inline void plate_frame_adjoint(const double o[13], double drilling, const double gl[36],
+                                                    double& hx, double& hy) {
+  // translations, then rotations: [[a, b], [c, d]] and the entry f of the axis
+  const double sub[2][5] = {{o[0], o[1], o[2], o[3], o[4]}, {o[8], o[9], o[11], o[12], drilling}};
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const double* k = sub[h];
+    const double* g = gl + 21 * h;
+    const double g12 = g[8] + g[13], g02 = g[2] + g[12];
+    hx += ((k[4] - k[3]) * g12 - k[2] * g[12]) - k[1] * g[2];
+    hy += ((k[0] - k[4]) * g02 + k[1] * g[13]) + k[2] * g[8];
   }
-  if (a == 0 || a == 3) {  // u_a carries e14
-    gxl[1] -= gu1 * q; gxl[5] += gu1 * q;
-    gxl[0] += gu2 * q; gxl[4] -= gu2 * q;
-  } else {                 // e23
-    gxl[3] -= gu1 * q;
-    gxl[2] += gu2 * q;
-  }
-}
-
-// h += antisymmetric parts (omega_x, omega_y) of K G^T + K^T G for one pair of
-// 3x3 sub-blocks K = k[r0.., c0..], G = gl[r0.., c0..] of 6x6 row-major blocks
-__host__ __device__ inline void plate_frame_adjoint_sub(const double* k, const double* gl, int r0, int c0, double& hx,
-                                                        double& hy) {
-#pragma unroll
-  for (int cc = 0; cc < 3; ++cc) {
-    const double k0c = k[(r0 + 0) * 6 + c0 + cc], k1c = k[(r0 + 1) * 6 + c0 + cc], k2c = k[(r0 + 2) * 6 + c0 + cc];
-    const double g0c = gl[(r0 + 0) * 6 + c0 + cc], g1c = gl[(r0 + 1) * 6 + c0 + cc], g2c = gl[(r0 + 2) * 6 + c0 + cc];
-    const double kc0 = k[(r0 + cc) * 6 + c0 + 0], kc1 = k[(r0 + cc) * 6 + c0 + 1], kc2 = k[(r0 + cc) * 6 + c0 + 2];
-    const double gc0 = gl[(r0 + cc) * 6 + c0 + 0], gc1 = gl[(r0 + cc) * 6 + c0 + 1], gc2 = gl[(r0 + cc) * 6 + c0 + 2];
-    hx += (k2c * g1c - k1c * g2c) + (kc2 * gc1 - kc1 * gc2);
-    hy += (k0c * g2c - k2c * g0c) + (kc0 * gc2 - kc2 * gc0);
-  }
-}
-
-// Per-lane share of the adjoint sums for block q of row p.  Mq: the six
-// integrals of column q (Mxx, Mxy, Myx, Myy, A, B; plate_row_accumulate),
-// vp/up and vq/uq: the unscaled shear vectors of nodes p and q, gl: the
-// local-frame gradient block (p, q), 6x6 row-major.  cq receives the integral
-// coefficients of column q (layout of plate_point_scalars: cxx, cxy, cyx, cyy,
-// cA, cB).
-__host__ __device__ inline void plate_block_adjoint_q(const double Mq[6], const PlateMat& m, const double vp[3],
-                                                      const double up[3], const double vq[3], const double uq[3],
-                                                      int p, int q, const double gl[36], double P[7], double cq[6],
-                                                      double gxl[6], double& hx, double& hy, bool frame = true) {
-  const double Mxx = Mq[0], Mxy = Mq[1], Myx = Mq[2], Myy = Mq[3], A = Mq[4], B = Mq[5];
-  const double Guu = gl[0], Guv = gl[1], Gvu = gl[6], Gvv = gl[7];
-  const double Gxx = gl[21], Gxy = gl[22], Gyx = gl[27], Gyy = gl[28];
-  // constitutive partials
-  P[0] += Guu * Mxx + Gvv * Myy;
-  P[1] += Guv * Mxy + Gvu * Myx;
-  P[2] += ((Guu * Myy + Guv * Myx) + Gvu * Mxy) + Gvv * Mxx;
-  P[3] += Gxx * Myy + Gyy * Mxx;
-  P[4] -= Gxy * Myx + Gyx * Mxy;
-  P[5] += ((Gxx * Mxx - Gxy * Mxy) - Gyx * Myx) + Gyy * Myy;
-  // shear: Gs = gl[2..4][2..4]; v_p^T Gs v_q, u_p^T Gs u_q and the one-sided products
-  double Gv_q[3], Gu_q[3], vG[3], uG[3];  // Gs v_q, Gs u_q, v_p^T Gs, u_p^T Gs
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    Gv_q[i] = 0.0; Gu_q[i] = 0.0; vG[i] = 0.0; uG[i] = 0.0;
-  }
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const double gs = gl[(2 + i) * 6 + 2 + j];
-      Gv_q[i] += gs * vq[j];
-      Gu_q[i] += gs * uq[j];
-      vG[j] += vp[i] * gs;
-      uG[j] += up[i] * gs;
-    }
-  const double sv_ = (vp[0] * Gv_q[0] + vp[1] * Gv_q[1]) + vp[2] * Gv_q[2];
-  const double su_ = (up[0] * Gu_q[0] + up[1] * Gu_q[1]) + up[2] * Gu_q[2];
-  P[6] += A * sv_ + B * su_;
-  // integral coefficients of column q
-  cq[0] = ((m.cm00 * Guu + m.cm22 * Gvv) + m.cb22 * Gxx) + m.cb00 * Gyy;
-  cq[1] = ((m.cm01 * Guv + m.cm22 * Gvu) - m.cb22 * Gxy) - m.cb01 * Gyx;
-  cq[2] = ((m.cm22 * Guv + m.cm01 * Gvu) - m.cb01 * Gxy) - m.cb22 * Gyx;
-  cq[3] = ((m.cm22 * Guu + m.cm00 * Gvv) + m.cb00 * Gxx) + m.cb22 * Gyy;
-  cq[4] = m.cs * sv_;
-  cq[5] = m.cs * su_;
-  // shear vectors: d/dv_p = cs A Gs v_q, d/dv_q = cs A v_p^T Gs (same with u, B)
-  const double sa = m.cs * A, sb = m.cs * B;
-  plate_shear_vector_adjoint(p, sa * Gv_q[1], sa * Gv_q[2], sb * Gu_q[1], sb * Gu_q[2], gxl);
-  plate_shear_vector_adjoint(q, sa * vG[1], sa * vG[2], sb * uG[1], sb * uG[2], gxl);
-  // frame rotation: needs the local block values (skipped by callers whose
-  // gradient blocks carry no in-plane / out-of-plane coupling: then it is 0)
-  if (!frame) return;
-  double kb[36];
-#pragma unroll
-  for (int i = 0; i < 36; ++i) kb[i] = 0.0;
-  double o[13];
-  double vps[3], ups[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    vps[i] = m.cs * vp[i];
-    ups[i] = m.cs * up[i];
-  }
-  plate_block_entries(Mxx, Mxy, Myx, Myy, A, B, m, vps, ups, vq, uq, o);
-  kb[0] = o[0]; kb[1] = o[1]; kb[6] = o[2]; kb[7] = o[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) kb[(2 + i) * 6 + 2 + j] = o[4 + 3 * i + j];
-  if (p == q) kb[35] = KROT6;
-  plate_frame_adjoint_sub(kb, gl, 0, 0, hx, hy);
-  plate_frame_adjoint_sub(kb, gl, 0, 3, hx, hy);
-  plate_frame_adjoint_sub(kb, gl, 3, 0, hx, hy);
-  plate_frame_adjoint_sub(kb, gl, 3, 3, hx, hy);
-}
-
-// Same for block q of row p given the whole row's integrals acc[24] and the
-// element's shear vectors; writes column q of c[24].
-__host__ __device__ inline void plate_block_adjoint(const double acc[24], const PlateMat& m, const PlateShear& sv,
-                                                    int p, int q, const double gl[36], double P[7], double c[24],
-                                                    double gxl[6], double& hx, double& hy, bool frame = true) {
-  const double Mq[6] = {acc[q], acc[4 + q], acc[8 + q], acc[12 + q], acc[16 + q], acc[20 + q]};
-  double vp[3], up[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    vp[i] = sel4(sv.v[0][i], sv.v[1][i], sv.v[2][i], sv.v[3][i], p);
-    up[i] = sel4(sv.u[0][i], sv.u[1][i], sv.u[2][i], sv.u[3][i], p);
-  }
-  double cq[6];
-  plate_block_adjoint_q(Mq, m, vp, up, sv.v[q], sv.u[q], p, q, gl, P, cq, gxl, hx, hy, frame);
-#pragma unroll
-  for (int k = 0; k < 6; ++k) c[4 * k + q] = cq[k];
+  // (w, theta) and (theta, w)
+  const double* g = gl + 3;
+  hx += (o[5] * g[6] + o[6] * g[7]) - o[6] * g[14];
+  hy += (o[5] * g[14] - o[5] * g[0]) - o[6] * g[1];
+  g = gl + 18;
+  hx += (o[7] * g[1] + o[10] * g[7]) - o[10] * g[14];
+  hy += (o[7] * g[14] - o[7] * g[0]) - o[10] * g[6];
 }
 
 // dL/d(E, nu, t, k) from the constitutive partials: cm = E t/(1-nu^2),
@@ -415,7 +223,7 @@ __host__ __device__ inline PlateEdges plate_edges(const double xl[6]) {
 // Compliance by strain energy: the share of the integration point (r, s) in
 // L = -u_l^T k u_l, with U[a] = (u, v, w, theta_x, theta_y, theta_z) the
 // local-frame displacements of node a.  Adds to P, gxl, hx, hy what
-// plate_block_adjoint_q adds over the sixteen blocks for G = -u_p u_q^T (but the
+// the sixteen blocks of plate_adjoint_kernel add for G = -u_p u_q^T (but the
 // drilling term: plate_compliance_drilling), without forming a block: each block
 // term is a bilinear form in nodal values, so its contraction with u u^T is the
 // point's quadratic form in the strains
@@ -427,7 +235,7 @@ __host__ __device__ inline PlateEdges plate_edges(const double xl[6]) {
 //   * P from the squared strains;
 //   * the point's adjoints: det from the energy density, the inverse Jacobian from
 //     resultant x natural derivative, mr and ms from the shear strains, and from
-//     them the local coordinates (as plate_point_reverse, with the point's own
+//     them the local coordinates (as plate_point_reverse_r, with the point's own
 //     Jacobian, reciprocals and lengths);
 //   * the shear vectors from the tying sums;
 //   * hx, hy = -2 sum_a (x_a x f_a)_{x,y} over the translation and rotation
