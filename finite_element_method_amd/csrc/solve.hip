@@ -15,6 +15,8 @@
 // direction.  The last two begin by summing the partial sums of the one before
 // in every workgroup (the same tree, so every workgroup has the same bits),
 // which takes the place of two one-workgroup launches per update.
+//
+// Small systems (SM_N rows, SM_NNZ entries) are solved by one workgroup, sv_small.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -26,6 +28,7 @@
 
 #include "device_state.hpp"
 #include "fem_device.hpp"
+#include "lane_ops.hpp"
 
 namespace femdev {
 
@@ -393,11 +396,8 @@ struct Sum2 {
 };
 __device__ inline Sum2 block_sum2(double a, double b) {
   __shared__ Sum2 w[SV_B / 64];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    a += __shfl_xor(a, o);
-    b += __shfl_xor(b, o);
-  }
+  a = wave_sum(a);
+  b = wave_sum(b);
   if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = {a, b};
   __syncthreads();
   Sum2 t = w[0];
@@ -480,10 +480,12 @@ __global__ void sv_block_starts(const uint32_t* __restrict__ flag, const uint32_
   else if (flag[i]) starts[id[i]] = int32_t(i);
 }
 
-// inverse of each node block (Gauss-Jordan, partial pivoting); status bit 1 on a singular block
+// inverse of each node block (Gauss-Jordan, partial pivoting); status bit 1 on a
+// singular block.  `count`, where given, holds the number of blocks (nblk is then its bound).
 __global__ __launch_bounds__(256) void sv_block_inverse(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
                                                         const double* __restrict__ v,
                                                         const int32_t* __restrict__ starts, int64_t nblk,
+                                                        const uint32_t* __restrict__ count,
                                                         double* __restrict__ inv, double* s) {
   // The augmented block [A | I] lives in registers: every loop below runs over
   // compile-time indices, so row swaps and column placement are selects (a
@@ -492,7 +494,7 @@ __global__ __launch_bounds__(256) void sv_block_inverse(const int64_t* __restric
   // pivots or elimination targets of the first m columns, so the m x m inverse
   // is the one the unpadded elimination gives.
   const int64_t b = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (b >= nblk) return;
+  if (b >= (count ? int64_t(*count) : nblk)) return;
   const int s0 = starts[b], m = starts[b + 1] - s0;
   double* o = inv + 36 * b;
   if (m > BJ_MAX) {  // a node has at most six dofs; guard the fixed-size arrays anyway
@@ -624,7 +626,7 @@ __device__ inline BjLane bj_lane(const int32_t* __restrict__ starts, int64_t nbl
   o.act = o.row < o.m;
   return o;
 }
-__device__ inline double bj_row_apply(const double* __restrict__ inv, const BjLane& L, int lane, double ri) {
+__device__ inline void bj_row(const double* __restrict__ inv, const BjLane& L, double w[6]) {
   double2 w0 = make_double2(0.0, 0.0), w1 = w0, w2 = w0;
   if (L.act) {
     const double2* row = reinterpret_cast<const double2*>(inv + 36 * L.k + 6 * L.row);
@@ -632,7 +634,9 @@ __device__ inline double bj_row_apply(const double* __restrict__ inv, const BjLa
     w1 = row[1];
     w2 = row[2];
   }
-  const double w[6] = {w0.x, w0.y, w1.x, w1.y, w2.x, w2.y};
+  w[0] = w0.x; w[1] = w0.y; w[2] = w1.x; w[3] = w1.y; w[4] = w2.x; w[5] = w2.y;
+}
+__device__ inline double bj_apply(const double w[6], const BjLane& L, int lane, double ri) {
   double zi = 0.0;
   const int first = lane - L.row;
 #pragma unroll
@@ -641,6 +645,11 @@ __device__ inline double bj_row_apply(const double* __restrict__ inv, const BjLa
     if (j < L.m) zi = __builtin_fma(w[j], rj, zi);
   }
   return zi;
+}
+__device__ inline double bj_row_apply(const double* __restrict__ inv, const BjLane& L, int lane, double ri) {
+  double w[6];
+  bj_row(inv, L, w);
+  return bj_apply(w, L, lane, ri);
 }
 __global__ void sv_start_block(const double* __restrict__ b, const double* __restrict__ inv,
                                const int32_t* __restrict__ starts, int64_t nblk, double* __restrict__ x,
@@ -724,6 +733,300 @@ __global__ __launch_bounds__(SV_B) void sv_direction(const double* __restrict__ 
     p[i] = __builtin_fma(beta, p[i], z[i]);
 }
 
+// ---- small systems: the whole solve in one workgroup
+//
+// Up to SM_N rows the update loop above is launches and the gaps between them
+// (four per update, a host wait per batch), its work a few hundred KiB.  Here
+// one workgroup keeps the vectors in LDS and runs the updates behind barriers.
+// Bound: K_aa read from L2 by one CU (64 B per clock) and the chain of its
+// product, two sums and the preconditioner.  Sums follow the grid kernels' trees
+// (a "virtual wave" here is a wave of theirs), so both ways have the same bits.
+// 50 block-Jacobi updates with their set-up, grid kernels and here:
+//   rows 24 (24 updates) 657 -> 99 us; 192: 895 -> 226; 1008 (18 k entries):
+//   900 -> 383; 1649 (30 k): 961 -> 547; 1275 (62 k): 979 -> 731; 1649 (82 k):
+//   973 -> 845.
+// SM_NNZ is where that ends: one CU's reading of 100 k entries costs an update
+// of the grid kernels.  SM_N is the size of the vectors in LDS (91 KB).
+constexpr int SM_T = 1024;
+constexpr int64_t SM_N = 2048;
+constexpr int64_t SM_NNZ = 80 * 1024;
+constexpr int SM_CHUNK = 4096;               // updates per launch, so that no launch runs on unboundedly
+constexpr int SM_VW = int(SM_N) / 64;        // virtual waves
+
+// zeroes the scalars; for node blocks their starts and number (one workgroup)
+__global__ __launch_bounds__(SM_T) void sv_small_setup(const int64_t* __restrict__ aa, int n, bool blocks,
+                                                       int32_t* __restrict__ starts, uint32_t* __restrict__ count,
+                                                       double* __restrict__ s) {
+  __shared__ uint32_t waves[SM_T / 64];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  if (t < S_COUNT) s[t] = 0.0;
+  if (!blocks) return;
+  uint32_t before = 0;
+  for (int base = 0; base < n; base += SM_T) {
+    const int i = base + t;
+    const bool flag = i < n && (i == 0 || aa[i] / 6 != aa[i - 1] / 6);
+    const uint64_t m = __ballot(flag);
+    if (lane == 0) waves[wave] = uint32_t(__popcll(m));
+    __syncthreads();
+    uint32_t at = before + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+    for (int w = 0; w < SM_T / 64; ++w) {
+      if (w < wave) at += waves[w];
+      before += waves[w];
+    }
+    if (flag) starts[at] = i;
+    __syncthreads();
+  }
+  if (t == 0) {
+    starts[before] = n;
+    *count = before;
+  }
+}
+
+// sums of a virtual wave's two values into slot vw
+__device__ inline void small_wave_sum(double a, double b, int vw, Sum2* slots) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if ((threadIdx.x & 63) == 0) slots[vw] = {a, b};
+}
+// total_partials of `parts` blocks (at most eight) of four virtual waves, in
+// every thread: the steps of the butterfly that would add zeros are left out
+__device__ inline Sum2 small_total(const Sum2* slots, int parts) {
+  const int lane = threadIdx.x & 7;
+  Sum2 t{0.0, 0.0};
+  if (lane < parts) {
+    t = slots[4 * lane];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+      t.a += slots[4 * lane + k].a;
+      t.b += slots[4 * lane + k].b;
+    }
+  }
+  t.a += lane_xor<4>(t.a);
+  t.b += lane_xor<4>(t.b);
+  t.a += lane_xor<2>(t.a);
+  t.b += lane_xor<2>(t.b);
+  t.a += lane_xor<1>(t.a);
+  t.b += lane_xor<1>(t.b);
+  return t;
+}
+
+// four neighbouring entries of K_aa (zeros past the end of the array)
+struct SmQuad {
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  double2 w0, w1;
+  u32x4 c;
+};
+__device__ inline SmQuad small_quad(__amdgpu_buffer_rsrc_t rv, __amdgpu_buffer_rsrc_t rc, uint32_t e) {
+  SmQuad q;
+  q.w0 = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rv, 8u * e, 0, 0));
+  q.w1 = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rv, 8u * e + 16u, 0, 0));
+  q.c = __builtin_amdgcn_raw_buffer_load_b128(rc, 4u * e, 0, 0);
+  return q;
+}
+
+template <bool BLOCK>
+__global__ __launch_bounds__(SM_T) void sv_small(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
+                                                 const double* __restrict__ v, uint32_t v_bytes,
+                                                 const double* __restrict__ b, const double* __restrict__ diag,
+                                                 const double* __restrict__ inv, const int32_t* __restrict__ starts,
+                                                 const uint32_t* __restrict__ count, int n, int parts, double rel_tol,
+                                                 double abs_tol, int max_iter, bool resume, double* __restrict__ x,
+                                                 double* __restrict__ r, double* __restrict__ p, double* s) {
+  __shared__ double lx[SM_N], lr[SM_N], lz[SM_N], lp[SM_N], lap[SM_N];
+  __shared__ uint32_t lrp[SM_N + 1];
+  __shared__ Sum2 dots[SM_VW], sums[SM_VW];
+  if (BLOCK && s[S_STATUS] != 0.0) return;  // a singular block: the host reports it
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nvw = 4 * parts;
+  const int64_t nblk = BLOCK ? int64_t(*count) : 0;
+  // the preconditioner of the wave's first two turns, kept: rows of the block
+  // inverses (turns w = wave and w1), or diagonal entries (virtual waves wave, wave + 16)
+  const int w1 = wave + (nvw <= SM_T / 64 ? nvw : SM_T / 64);
+  BjLane k0{}, k1{};
+  double inv0[6], inv1[6], d0 = 1.0, d1 = 1.0;
+  if (BLOCK) {
+    k0 = bj_lane(starts, nblk, wave, lane);
+    k1 = bj_lane(starts, nblk, w1, lane);
+    bj_row(inv, k0, inv0);
+    bj_row(inv, k1, inv1);
+  } else {
+    if (t < n) d0 = diag[t];
+    if (t + SM_T < n) d1 = diag[t + SM_T];
+  }
+  for (int i = t; i <= n; i += SM_T) lrp[i] = uint32_t(rp[i]);
+  double rz, rr, bb;
+  int it = 0;
+  if (resume) {
+    for (int i = t; i < n; i += SM_T) {
+      lx[i] = x[i];
+      lr[i] = r[i];
+      lp[i] = p[i];
+    }
+    rz = s[S_RZ];
+    rr = s[S_RR];
+    bb = s[S_BB];
+    it = int(s[S_ITER]);
+    __syncthreads();  // thread 0 writes the scalars at the end
+  } else {
+    for (int vw = wave; vw < nvw; vw += SM_T / 64) {
+      double ra = 0.0, rb = 0.0;
+      if (BLOCK) {
+        for (int64_t w = vw; w * BJ_PER_WAVE < nblk; w += nvw) {
+          const BjLane L = bj_lane(starts, nblk, w, lane);
+          const int i = L.s0 + L.row;
+          const double ri = L.act ? b[i] : 0.0;
+          const double zi = bj_row_apply(inv, L, lane, ri);
+          if (L.act) {
+            lx[i] = 0.0;
+            lr[i] = ri;
+            lp[i] = zi;
+            ra = __builtin_fma(ri, zi, ra);
+            rb = __builtin_fma(ri, ri, rb);
+          }
+        }
+      } else if (64 * vw + lane < n) {
+        const int i = 64 * vw + lane;
+        const double bi = b[i], zi = bi / (vw == wave ? d0 : d1);
+        lx[i] = 0.0;
+        lr[i] = bi;
+        lp[i] = zi;
+        ra = __builtin_fma(bi, zi, 0.0);
+        rb = __builtin_fma(bi, bi, 0.0);
+      }
+      small_wave_sum(ra, rb, vw, sums);
+    }
+    __syncthreads();
+    const Sum2 t2 = small_total(sums, parts);
+    rz = t2.a;
+    rr = t2.b;
+    bb = t2.b;
+  }
+  const double rel = rel_tol * sqrt(bb);
+  const double stop = rel < abs_tol ? abs_tol : rel;
+  bool conv = sqrt(rr) <= stop;
+  bool done = conv || it >= max_iter;
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(v), 0, int(v_bytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(ci), 0, int(v_bytes / 2u), 0x00020000);
+  // every thread has the same scalars, so all leave the loop together
+#pragma unroll 1
+  for (int k = 0; k < SM_CHUNK && !done; ++k) {
+    __syncthreads();
+    // Ap = K p: sv_spmv_it_quad's four lanes per row, two rows per lane, each
+    // row's next entries loaded while the last ones are summed
+    const int lig = t & 3;
+    for (int r0 = t >> 2; r0 < n; r0 += 2 * (SM_T / 4)) {
+      const int r1 = r0 + SM_T / 4;
+      uint32_t e[2] = {lrp[r0] + 4u * lig, 0u}, end[2] = {lrp[r0 + 1], 0u};
+      if (r1 < n) {
+        e[1] = lrp[r1] + 4u * lig;
+        end[1] = lrp[r1 + 1];
+      }
+      double acc[2] = {0.0, 0.0};
+      SmQuad cur[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) cur[h] = small_quad(rv, rc, e[h]);
+      while (e[0] < end[0] || e[1] < end[1]) {
+        SmQuad next[2];
+        const bool more = e[0] + 16u < end[0] || e[1] + 16u < end[1];
+        if (more) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) next[h] = small_quad(rv, rc, e[h] + 16u);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {  // past a row's end: loaded, not summed
+          const double p0 = lp[cur[h].c.x], p1 = lp[cur[h].c.y], p2 = lp[cur[h].c.z], p3 = lp[cur[h].c.w];
+          if (e[h] < end[h]) acc[h] = __builtin_fma(cur[h].w0.x, p0, acc[h]);
+          if (e[h] + 1 < end[h]) acc[h] = __builtin_fma(cur[h].w0.y, p1, acc[h]);
+          if (e[h] + 2 < end[h]) acc[h] = __builtin_fma(cur[h].w1.x, p2, acc[h]);
+          if (e[h] + 3 < end[h]) acc[h] = __builtin_fma(cur[h].w1.y, p3, acc[h]);
+          e[h] += 16u;
+        }
+        if (!more) break;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) cur[h] = next[h];
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        acc[h] += lane_xor<2>(acc[h]);
+        acc[h] += lane_xor<1>(acc[h]);
+      }
+      if (lig == 0) {
+        lap[r0] = acc[0];
+        if (r1 < n) lap[r1] = acc[1];
+      }
+    }
+    __syncthreads();
+    for (int vw = wave; vw < nvw; vw += SM_T / 64) {
+      const int i = 64 * vw + lane;
+      small_wave_sum(i < n ? __builtin_fma(lp[i], lap[i], 0.0) : 0.0, 0.0, vw, dots);
+    }
+    __syncthreads();
+    const double alpha = rz / small_total(dots, parts).a;
+    for (int vw = wave; vw < nvw; vw += SM_T / 64) {
+      double ra = 0.0, rb = 0.0;
+      if (BLOCK) {
+        for (int w = vw; w * BJ_PER_WAVE < nblk; w += nvw) {
+          BjLane L = w == wave ? k0 : k1;
+          double row[6];
+#pragma unroll
+          for (int j = 0; j < 6; ++j) row[j] = w == wave ? inv0[j] : inv1[j];
+          if (w != wave && w != w1) {
+            L = bj_lane(starts, nblk, w, lane);
+            bj_row(inv, L, row);
+          }
+          const int i = L.s0 + L.row;
+          double ri = 0.0;
+          if (L.act) {
+            lx[i] = __builtin_fma(alpha, lp[i], lx[i]);
+            ri = __builtin_fma(-alpha, lap[i], lr[i]);
+            lr[i] = ri;
+          }
+          const double zi = bj_apply(row, L, lane, ri);
+          if (L.act) {
+            lz[i] = zi;
+            ra = __builtin_fma(ri, zi, ra);
+            rb = __builtin_fma(ri, ri, rb);
+          }
+        }
+      } else if (64 * vw + lane < n) {
+        const int i = 64 * vw + lane;
+        lx[i] = __builtin_fma(alpha, lp[i], lx[i]);
+        const double ri = __builtin_fma(-alpha, lap[i], lr[i]);
+        lr[i] = ri;
+        const double zi = ri / (vw == wave ? d0 : d1);
+        lz[i] = zi;
+        ra = __builtin_fma(ri, zi, 0.0);
+        rb = __builtin_fma(ri, ri, 0.0);
+      }
+      small_wave_sum(ra, rb, vw, sums);
+    }
+    __syncthreads();
+    const Sum2 t2 = small_total(sums, parts);
+    const double beta = t2.a / rz;
+    rz = t2.a;
+    rr = t2.b;
+    ++it;
+    conv = sqrt(rr) <= stop;
+    done = conv || it >= max_iter;
+    for (int i = t; i < n; i += SM_T) lp[i] = __builtin_fma(beta, lp[i], lz[i]);
+  }
+  __syncthreads();
+  for (int i = t; i < n; i += SM_T) {
+    x[i] = lx[i];
+    r[i] = lr[i];
+    p[i] = lp[i];
+  }
+  if (t == 0) {
+    s[S_RZ] = rz;
+    s[S_RR] = rr;
+    s[S_BB] = bb;
+    s[S_ITER] = double(it);
+    s[S_CONV] = conv ? 1.0 : 0.0;
+    s[S_DONE] = done ? 1.0 : 0.0;
+  }
+}
+
 // r_b: forces at the k_bb indexes
 __global__ void sv_gather(const double* __restrict__ src, const int64_t* __restrict__ idx, int64_t n,
                           double* __restrict__ dst) {
@@ -744,6 +1047,7 @@ unsigned grid_for(int64_t items, int per_block) { return unsigned(std::max<int64
 struct SolveBuffers {
   virtual std::string get(int slot, size_t bytes, void** out) = 0;
   virtual bool grows() const { return false; }
+  virtual size_t room() const { return size_t(1) << 62; }  // bytes that get() can still hand out
   double* host = nullptr;  // S_COUNT + 1 doubles of host memory for the scalar reads
 };
 
@@ -842,102 +1146,138 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
   double* diag = nullptr;
   double* inv = nullptr;
   int32_t* starts = nullptr;
-  sv_zero<<<1, 64, 0, s>>>(sc, S_COUNT);
-  HIP_TRY(hipGetLastError());
-  if (precond == 0) {
-    if (!(e = take(bufs, 10, una, diag)).empty()) return e;
-    if (na) {
-      sv_diag<<<grid_for(na, B), B, 0, s>>>(rp[0], ci[0], v[0], na, diag);
-      HIP_TRY(hipGetLastError());
-    }
-  } else {
-    uint32_t *flag = nullptr, *bid = nullptr;
-    if (!(e = take(bufs, 11, una + 1, flag)).empty()) return e;
-    if (!(e = take(bufs, 12, una + 1, bid)).empty()) return e;
-    if (!(e = take(bufs, 13, una + 1, starts)).empty()) return e;
-    sv_block_flags<<<grid_for(na + 1, B), B, 0, s>>>(aa_idx, na, flag);
-    HIP_TRY(hipGetLastError());
-    size_t bytes = 0;
-    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, flag, bid, int(na + 1), s));
-    void* tmp = nullptr;
-    if (!(e = bufs.get(14, std::max<size_t>(bytes, 1), &tmp)).empty()) return e;
-    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, flag, bid, int(na + 1), s));
-    sv_block_starts<<<grid_for(na + 1, B), B, 0, s>>>(flag, bid, na, starts);
-    HIP_TRY(hipGetLastError());
-    uint32_t nb32 = 0;
-    HIP_TRY(hipMemcpyAsync(host, bid + na, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    std::memcpy(&nb32, host, sizeof(uint32_t));
-    nblk = int64_t(nb32);
-    if (!(e = take(bufs, 15, size_t(36 * std::max<int64_t>(nblk, 1)), inv)).empty()) return e;
-    if (nblk) {
-      sv_block_inverse<<<grid_for(nblk, B), B, 0, s>>>(rp[0], ci[0], v[0], starts, nblk, inv, sc);
-      HIP_TRY(hipGetLastError());
-    }
-  }
-  // start.  The reductions' grid: one block per SV_B dofs, at most SV_PARTS (a
-  // function of n, and the same for every launch of the solve)
+  // the reductions' grid: one block per SV_B dofs, at most SV_PARTS (a function
+  // of n, and the same for every launch of the solve)
   const unsigned parts = unsigned(std::min<int64_t>(SV_PARTS, grid_for(na, SV_B)));
-  if (precond == 0)
-    sv_start_jacobi<<<parts, B, 0, s>>>(b, diag, na, x, r, z, p, pa, pb);
-  else
-    sv_start_block<<<parts, B, 0, s>>>(b, inv, starts, nblk, x, r, z, p, pa, pb);
-  HIP_TRY(hipGetLastError());
-  sv_start_scalars<<<1, B, 0, s>>>(pa, pb, int(parts), sc);
-  HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(host, sc, sizeof(double) * S_COUNT, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  if (host[S_STATUS] != 0.0) return "PCG(BlockJacobi): singular node block";
-  const double stop = std::max(rel_tol * std::sqrt(host[S_BB]), abs_tol);
+  const bool quad = wide && size_t(d->sep_nnz[0]) * 8 < (size_t(1) << 32);
+  const uint32_t v_bytes = quad ? uint32_t(size_t(d->sep_nnz[0]) * 8) : 0u;
+  double stop = 0.0;
   int it = 0;
-  bool conv = std::sqrt(host[S_RR]) <= stop;
-  if (!conv && max_iter > 0) {
-    // Updates are queued in growing batches; the last scalar kernel of an
-    // update raises the stop flag on convergence or at max_iter, and every
-    // kernel queued after that returns at once.  The count stays exact and the
-    // host waits once per batch, not once per update.
-    const bool quad = wide && size_t(d->sep_nnz[0]) * 8 < (size_t(1) << 32);
-    const uint32_t v_bytes = quad ? uint32_t(size_t(d->sep_nnz[0]) * 8) : 0u;
-    const unsigned spmv_blocks = grid_for(na * (quad ? SPMV_QUAD_LANES : SPMV_LANES), B);
-    Slices sl;
-    bool slice = quad && bufs.grows() && d->sep_nnz[0] >= SL_MIN_NNZ && max_iter >= SL_MIN_UPDATES;
-    uint32_t slice_total = 0;
-    int queued = 0, batch = 1;
-    for (;;) {
-      const int nq = std::min(batch, max_iter - queued);
-      for (int q = 0; q < nq; ++q) {
-        const int turn = (queued + q) & 1;
-        if (sl.data)
-          sv_spmv_slices<<<grid_for(sl.n, 4), 256, 0, s>>>(sl.data, rp[0], sl.rows, sl.pairs, sl.cbase, sl.offset,
-                                                           sl.n, p, ap, sc, turn);
-        else if (quad) sv_spmv_it_quad<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, turn, v_bytes);
-        else sv_spmv_it<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, turn);
-        sv_dot_it<<<parts, B, 0, s>>>(p, ap, na, sc, turn, pc);
-        if (precond == 0)
-          sv_update_jacobi<<<parts, B, 0, s>>>(diag, p, ap, sc, turn, pc, na, x, r, z, pa, pb);
-        else
-          sv_update_block<<<parts, B, 0, s>>>(inv, starts, nblk, p, ap, sc, turn, pc, x, r, z, pa, pb);
-        sv_direction<<<parts, B, 0, s>>>(z, sc, turn, pa, pb, stop, double(max_iter), na, p);
-      }
+  bool conv = false;
+  // a small system: one block inverse per dof is room enough, so the number of
+  // node blocks stays on the device, and so do the tolerance and the updates
+  if (quad && na > 0 && na <= SM_N && d->sep_nnz[0] <= SM_NNZ &&
+      bufs.room() >= una * (36 * sizeof(double) + sizeof(int32_t)) + 4096) {
+    uint32_t* count = nullptr;
+    if (precond == 0) {
+      if (!(e = take(bufs, 10, una, diag)).empty()) return e;
+      sv_diag<<<grid_for(na, B), B, 0, s>>>(rp[0], ci[0], v[0], na, diag);
+    } else {
+      if (!(e = take(bufs, 15, 36 * una, inv)).empty()) return e;
+      if (!(e = take(bufs, 13, una + 1, starts)).empty()) return e;
+      if (!(e = take(bufs, 12, 1, count)).empty()) return e;
+    }
+    sv_small_setup<<<1, SM_T, 0, s>>>(aa_idx, int(na), precond != 0, starts, count, sc);
+    if (precond != 0)
+      sv_block_inverse<<<grid_for(na, B), B, 0, s>>>(rp[0], ci[0], v[0], starts, na, count, inv, sc);
+    auto kernel = precond == 0 ? sv_small<false> : sv_small<true>;
+    bool resume = false;
+    do {
+      kernel<<<1, SM_T, 0, s>>>(rp[0], ci[0], v[0], v_bytes, b, diag, inv, starts, count, int(na), int(parts), rel_tol,
+                                abs_tol, max_iter, resume, x, r, p, sc);
       HIP_TRY(hipGetLastError());
-      const bool first = queued == 0;
-      queued += nq;
-      if (slice && first) {
-        slice = slices_size(bufs, rp[0], ci[0], na, s, sl).empty();  // no memory: the solve goes on without
-        if (slice) HIP_TRY(hipMemcpyAsync(host + S_COUNT, sl.offset + sl.n, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        else (void)hipGetLastError();
-      }
       HIP_TRY(hipMemcpyAsync(host, sc, sizeof(double) * S_COUNT, hipMemcpyDeviceToHost, s));
       HIP_TRY(hipStreamSynchronize(s));
-      if (host[S_DONE] != 0.0 || host[S_DONE + 1] != 0.0 || queued >= max_iter) break;
-      if (slice && first) {
-        std::memcpy(&slice_total, host + S_COUNT, sizeof(uint32_t));
-        if (!slices_fill(bufs, rp[0], ci[0], v[0], v_bytes, slice_total, s, sl)) sl.data = nullptr;
-      }
-      batch = std::min(batch * 2, 64);
-    }
+      if (host[S_STATUS] != 0.0) return "PCG(BlockJacobi): singular node block";
+      resume = true;
+    } while (host[S_DONE] == 0.0);
+    stop = std::max(rel_tol * std::sqrt(host[S_BB]), abs_tol);
     it = int(host[S_ITER]);
     conv = host[S_CONV] != 0.0;
+  } else {
+    sv_zero<<<1, 64, 0, s>>>(sc, S_COUNT);
+    HIP_TRY(hipGetLastError());
+    if (precond == 0) {
+      if (!(e = take(bufs, 10, una, diag)).empty()) return e;
+      if (na) {
+        sv_diag<<<grid_for(na, B), B, 0, s>>>(rp[0], ci[0], v[0], na, diag);
+        HIP_TRY(hipGetLastError());
+      }
+    } else {
+      uint32_t *flag = nullptr, *bid = nullptr;
+      if (!(e = take(bufs, 11, una + 1, flag)).empty()) return e;
+      if (!(e = take(bufs, 12, una + 1, bid)).empty()) return e;
+      if (!(e = take(bufs, 13, una + 1, starts)).empty()) return e;
+      sv_block_flags<<<grid_for(na + 1, B), B, 0, s>>>(aa_idx, na, flag);
+      HIP_TRY(hipGetLastError());
+      size_t bytes = 0;
+      HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, flag, bid, int(na + 1), s));
+      void* tmp = nullptr;
+      if (!(e = bufs.get(14, std::max<size_t>(bytes, 1), &tmp)).empty()) return e;
+      HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, flag, bid, int(na + 1), s));
+      sv_block_starts<<<grid_for(na + 1, B), B, 0, s>>>(flag, bid, na, starts);
+      HIP_TRY(hipGetLastError());
+      uint32_t nb32 = 0;
+      HIP_TRY(hipMemcpyAsync(host, bid + na, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+      HIP_TRY(hipStreamSynchronize(s));
+      std::memcpy(&nb32, host, sizeof(uint32_t));
+      nblk = int64_t(nb32);
+      if (!(e = take(bufs, 15, size_t(36 * std::max<int64_t>(nblk, 1)), inv)).empty()) return e;
+      if (nblk) {
+        sv_block_inverse<<<grid_for(nblk, B), B, 0, s>>>(rp[0], ci[0], v[0], starts, nblk, nullptr, inv, sc);
+        HIP_TRY(hipGetLastError());
+      }
+    }
+    // start
+    if (precond == 0)
+      sv_start_jacobi<<<parts, B, 0, s>>>(b, diag, na, x, r, z, p, pa, pb);
+    else
+      sv_start_block<<<parts, B, 0, s>>>(b, inv, starts, nblk, x, r, z, p, pa, pb);
+    HIP_TRY(hipGetLastError());
+    sv_start_scalars<<<1, B, 0, s>>>(pa, pb, int(parts), sc);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(host, sc, sizeof(double) * S_COUNT, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    if (host[S_STATUS] != 0.0) return "PCG(BlockJacobi): singular node block";
+    stop = std::max(rel_tol * std::sqrt(host[S_BB]), abs_tol);
+    it = 0;
+    conv = std::sqrt(host[S_RR]) <= stop;
+    if (!conv && max_iter > 0) {
+      // Updates are queued in growing batches; the last scalar kernel of an
+      // update raises the stop flag on convergence or at max_iter, and every
+      // kernel queued after that returns at once.  The count stays exact and the
+      // host waits once per batch, not once per update.
+      const unsigned spmv_blocks = grid_for(na * (quad ? SPMV_QUAD_LANES : SPMV_LANES), B);
+      Slices sl;
+      bool slice = quad && bufs.grows() && d->sep_nnz[0] >= SL_MIN_NNZ && max_iter >= SL_MIN_UPDATES;
+      uint32_t slice_total = 0;
+      int queued = 0, batch = 1;
+      for (;;) {
+        const int nq = std::min(batch, max_iter - queued);
+        for (int q = 0; q < nq; ++q) {
+          const int turn = (queued + q) & 1;
+          if (sl.data)
+            sv_spmv_slices<<<grid_for(sl.n, 4), 256, 0, s>>>(sl.data, rp[0], sl.rows, sl.pairs, sl.cbase, sl.offset,
+                                                             sl.n, p, ap, sc, turn);
+          else if (quad) sv_spmv_it_quad<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, turn, v_bytes);
+          else sv_spmv_it<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, turn);
+          sv_dot_it<<<parts, B, 0, s>>>(p, ap, na, sc, turn, pc);
+          if (precond == 0)
+            sv_update_jacobi<<<parts, B, 0, s>>>(diag, p, ap, sc, turn, pc, na, x, r, z, pa, pb);
+          else
+            sv_update_block<<<parts, B, 0, s>>>(inv, starts, nblk, p, ap, sc, turn, pc, x, r, z, pa, pb);
+          sv_direction<<<parts, B, 0, s>>>(z, sc, turn, pa, pb, stop, double(max_iter), na, p);
+        }
+        HIP_TRY(hipGetLastError());
+        const bool first = queued == 0;
+        queued += nq;
+        if (slice && first) {
+          slice = slices_size(bufs, rp[0], ci[0], na, s, sl).empty();  // no memory: the solve goes on without
+          if (slice) HIP_TRY(hipMemcpyAsync(host + S_COUNT, sl.offset + sl.n, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+          else (void)hipGetLastError();
+        }
+        HIP_TRY(hipMemcpyAsync(host, sc, sizeof(double) * S_COUNT, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        if (host[S_DONE] != 0.0 || host[S_DONE + 1] != 0.0 || queued >= max_iter) break;
+        if (slice && first) {
+          std::memcpy(&slice_total, host + S_COUNT, sizeof(uint32_t));
+          if (!slices_fill(bufs, rp[0], ci[0], v[0], v_bytes, slice_total, s, sl)) sl.data = nullptr;
+        }
+        batch = std::min(batch * 2, 64);
+      }
+      it = int(host[S_ITER]);
+      conv = host[S_CONV] != 0.0;
+    }
   }
   // r_r = (K_ba u_a + K_bb u_b) - r_b
   if (nb) {
@@ -1031,6 +1371,7 @@ struct StaticBuffers : SolveBuffers {
   unsigned char* base = nullptr;
   size_t used = 0;
   double *u_a = nullptr, *r_r = nullptr;
+  size_t room() const override { return STATIC_SCRATCH_BYTES - std::min(STATIC_SCRATCH_BYTES, (used + 255) & ~size_t(255)); }
   std::string get(int slot, size_t bytes, void** out) override {
     if (slot == 1) { *out = u_a; return ""; }
     if (slot == 6) { *out = r_r; return ""; }
