@@ -5,14 +5,15 @@
 // record, rows 0..2 only); the others to bar_owner_kernel:
 //
 // One workgroup per range of owned nodes (<= 40 nodes, <= 256 incident
-// (node, element) entries, <= 5120 CSR values).  Each entry's constants (the
-// element frame and term scales, its blocks' masks and row offsets) sit in a
-// 160-byte slot formed once per model change (bar_slot_kernel), in the order
-// the workgroup reads them.  One lane per (owned node a, CSR row i) walks a's
-// entries in element-insertion order and computes row i of each entry's global
-// blocks (p, p) and (p, 1 - p) (p = a's position in the element).  The six
-// lanes of a node sit in one wave and load each slot together (two 16-byte
-// loads per lane), one entry ahead of the arithmetic, into the node's LDS slot,
+// (node, element) entries, <= 5120 CSR values).  Each element's constants (frame
+// and term scales) sit in one 128-byte record, formed once per model change
+// (bar_record_kernel) in the order in which the ranges meet the elements; an
+// entry's block mask and row offsets are part of the pattern.  One lane per
+// (owned node a, CSR row i) walks a's entries in element-insertion order and
+// computes row i of each entry's global blocks (p, p) and (p, 1 - p) (p = a's
+// position in the element).  The six lanes of a node sit in one wave and load
+// each record together (16-byte loads), two entries ahead of the arithmetic,
+// into the node's LDS slot,
 // from which every lane reads it.  The diagonal block (a, a) is summed in
 // registers over all incident elements (insertion order, starting from the
 // first contribution); an off-diagonal block (a, b) has exactly one
@@ -41,8 +42,7 @@ typedef double bo_d2 __attribute__((ext_vector_type(2)));
 constexpr int BO_THREADS = 256;
 constexpr int BO_NODES = 40;     // owned nodes per workgroup (10 per wave, 6 row lanes each)
 constexpr int BO_ENTRIES = 256;  // (owned node, incident element) entries per workgroup
-constexpr int BO_DATA = 16;      // element constants per entry slot
-constexpr int BO_SLOT = 20;      // doubles per entry slot
+constexpr int BO_REC = 16;       // doubles per element record
 constexpr int BO_VALUES = 5120;  // CSR values of the owned rows per workgroup
 constexpr int TO_NODES = 85;     // truss kernel: owned nodes per workgroup (3 row lanes each)
 constexpr int TO_ENTRIES = 512;  // truss kernel: entries per workgroup
@@ -60,15 +60,20 @@ struct BarArgs {
   const uint32_t* __restrict__ inc_ptr;
   const uint32_t* __restrict__ inc;
   const uint2* __restrict__ ranges;  // per workgroup: first node, node count
-  const double* __restrict__ slot;   // bar kernel: staged entries (BO_SLOT doubles each), range r from slot_ptr[r]
-  const uint32_t* __restrict__ slot_ptr;
+  const double* __restrict__ rec;    // bar kernel: element records, BO_REC doubles each
+  const uint32_t* __restrict__ entry_rec;  // entries, range r from entry_ptr[r]: type << 31 | record << 1 | p
+  const uint32_t* __restrict__ entry_ptr;
+  const uint4* __restrict__ entry;   // per entry: block (p, 1 - p); per node: its diagonal block (block_word)
+  const uint4* __restrict__ self;
   const int64_t* __restrict__ row_ptr;
   double* __restrict__ val;
 };
 
 struct BarLds {
   uint32_t first[BO_NODES + 1];         // entry range of each owned node
-  double2 slot[BO_NODES][BO_SLOT / 2];  // each owned node's current entry slot
+  double2 slot[BO_NODES][BO_REC / 2 + 1];  // each owned node's current element record (padded: banks)
+  uint4 block[BO_ENTRIES];              // the entries' off-diagonal blocks
+  uint32_t rec[BO_ENTRIES];             // and their elements
   double out[BO_VALUES];                // the owned rows
 };
 static_assert(3 * sizeof(BarLds) <= 160 * 1024, "three workgroups per CU");
@@ -88,21 +93,6 @@ struct TrussLds {
 };
 static_assert(4 * sizeof(TrussLds) <= 160 * 1024, "four workgroups per CU");
 static_assert(TO_NODES == TRUSS_WG_NODES && TO_ENTRIES == TRUSS_WG_ENTRIES && 3 * TO_NODES <= BO_THREADS, "range cut");
-
-// T^T v_t for the beam's rank-one term t with nodal shape value b
-// (v: u = b e0; v = b e1 - e5/2; w = b e2 - e4/2; tu = b e3; tv = b e4; tw = b e5)
-__device__ inline void beam_term_vec(int t, double b, const double R[9], double o[6]) {
-#pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    double tr = 0.0, rr = 0.0;
-    if (t == 0) tr = b * R[0 * 3 + m];
-    else if (t == 1) { tr = b * R[1 * 3 + m]; rr = -0.5 * R[2 * 3 + m]; }
-    else if (t == 2) { tr = b * R[2 * 3 + m]; rr = -0.5 * R[1 * 3 + m]; }
-    else rr = b * R[(t - 3) * 3 + m];
-    o[m] = tr;
-    o[3 + m] = rr;
-  }
-}
 
 // Jacobian of element e of `type` and the nodal shape derivatives b_p, b_q
 // of its end p and the other end
@@ -134,28 +124,22 @@ __device__ inline void truss_constants(const BarArgs& A, size_t e, int p, double
   o[4] = (bp * bq) * scale;
 }
 
-// One (owned node, incident element) entry's constants, as a slot of BO_SLOT
-// doubles: the element constants (BO_DATA doubles; beam: R (9), the six term
-// scales, b_p = -b_q; truss: r (3), k_pp, k_pq; truss.rs:132-189,
-// beam.rs:495-605), then the masks of its blocks (p, p) and (p, 1 - p) (36
-// bits each) with the offsets of rows 0 and 1 in the bits above them (12 bits
-// each: a row holds at most 6 x 257 values) and the element type in bit 63,
-// then the offsets of rows 2..5 of both blocks (16 bits each).  The slots are
-// formed once per model change by bar_slot_kernel, so that the assembly reads
-// each entry with ten 16-byte loads instead of a chain of dependent ones.
-static_assert(BO_DATA + 4 == BO_SLOT && BO_SLOT == 20, "slot layout: ten 16-byte chunks");
-
-__device__ inline void form_slot(const BarArgs& A, uint32_t u, double* __restrict__ slot) {
-  const int type = int(u >> 31), p = int(u & 1u);
+// An element's constants (beam: R (9), the scales of the rank-one terms u, v and
+// w, tu, tv, tw, and |b_p|; truss: r (3), k_pp, k_pq; truss.rs:132-189,
+// beam.rs:495-605).  One record serves both ends: with a copy per end (and the
+// pattern's words in it, 160 bytes) the 64 x 64 x 64 frame read 248 MB of
+// constants, here 99 MB and 31 MB of entries.
+__device__ inline void form_record(const BarArgs& A, uint32_t u, double* __restrict__ rec) {
+  const int type = int(u >> 31);
   const size_t e = (u >> 1) & 0x3FFFFFFFu;
-  double o[BO_DATA + 1];
+  double o[BO_REC];
 #pragma unroll
-  for (int k = 0; k <= BO_DATA; ++k) o[k] = 0.0;
+  for (int k = 0; k < BO_REC; ++k) o[k] = 0.0;
   if (type == 0) {
-    truss_constants(A, e, p, o);
+    truss_constants(A, e, 0, o);  // k_pp and k_pq are the same from either end
   } else {
     double bp, bq;
-    const double J = bar_shape(A, 1, e, p, bp, bq);
+    const double J = bar_shape(A, 1, e, 1, bp, bq);
     const double* Rp = A.R[1] + 9 * e;
     const double* prm = A.params[1] + 11 * e;
     const double E = prm[0], nu = prm[1], Ar = prm[2], it = prm[6], k = prm[7];
@@ -166,89 +150,92 @@ __device__ inline void form_slot(const BarArgs& A, uint32_t u, double* __restric
     for (int m = 0; m < 9; ++m) o[m] = Rp[m];
     o[9] = Ar * E * det_j * alpha;
     o[10] = G * Ar * k * det_j * alpha;
-    o[11] = G * Ar * k * det_j * alpha;
-    o[12] = G * it * det_j * alpha;
-    o[13] = E * i22p * det_j * alpha;
-    o[14] = E * i11p * det_j * alpha;
-    o[15] = bp;
-    (void)bq;  // -bp exactly
+    o[11] = G * it * det_j * alpha;
+    o[12] = E * i22p * det_j * alpha;
+    o[13] = E * i11p * det_j * alpha;
+    o[14] = bp;  // of end 1; -bp exactly at end 0
+    (void)bq;
   }
-  const uint32_t ks = A.bid[type][4 * e + 3 * p], kn = A.bid[type][4 * e + 2 * p + (1 - p)];
-  uint16_t off[12];
+  double2* dst = reinterpret_cast<double2*>(rec);
 #pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    off[i] = A.boff[6 * size_t(ks) + i];
-    off[6 + i] = A.boff[6 * size_t(kn) + i];
-  }
-  double w[BO_SLOT];
-#pragma unroll
-  for (int k = 0; k < BO_DATA; ++k) w[k] = o[k];
-  // masks (36 bits) with the offsets of rows 0, 1 (12 bits each) above them and
-  // the type in bit 63; the offsets of rows 2..5 as 16-bit fields
-  const uint64_t m0 = A.bmask[ks], m1 = A.bmask[kn];
-  w[BO_DATA] = __builtin_bit_cast(double, m0 | uint64_t(off[0]) << 36 | uint64_t(off[1]) << 48 | uint64_t(type) << 63);
-  w[BO_DATA + 1] = __builtin_bit_cast(double, m1 | uint64_t(off[6]) << 36 | uint64_t(off[7]) << 48);
-#pragma unroll
-  for (int b = 0; b < 2; ++b)
-    w[BO_DATA + 2 + b] = __builtin_bit_cast(double, uint64_t(off[6 * b + 2]) | uint64_t(off[6 * b + 3]) << 16 |
-                                                        uint64_t(off[6 * b + 4]) << 32 | uint64_t(off[6 * b + 5]) << 48);
-  double2* dst = reinterpret_cast<double2*>(slot);
-#pragma unroll
-  for (int k = 0; k < BO_SLOT / 2; ++k) dst[k] = make_double2(w[2 * k], w[2 * k + 1]);
+  for (int k = 0; k < BO_REC / 2; ++k) dst[k] = make_double2(o[2 * k], o[2 * k + 1]);
 }
 
-// slot s <- entry slot_inc[s]
-__global__ __launch_bounds__(256) void bar_slot_kernel(BarArgs A, const uint32_t* __restrict__ slot_inc, size_t n,
-                                                       double* __restrict__ slot) {
+__global__ __launch_bounds__(256) void bar_record_kernel(BarArgs A, const uint32_t* __restrict__ elem, size_t n,
+                                                         double* __restrict__ rec) {
   const size_t s = blockIdx.x * size_t(blockDim.x) + threadIdx.x;
-  if (s >= n) return;
-  form_slot(A, A.inc[slot_inc[s]], slot + BO_SLOT * s);
+  if (s < n) form_record(A, elem[s], rec + BO_REC * s);
 }
 
-// slot fields: element type, mask of block b (0: (p, p), 1: (p, 1 - p)) and
-// the offset of its row i within the owned node's row
-__device__ inline uint32_t slot_type(const double* o) {
-  return uint32_t(__builtin_bit_cast(uint64_t, o[BO_DATA]) >> 63);
+// a block's mask (36 bits) and the offsets of its rows within the owned node's
+// rows (12 bits each: a row holds at most 6 x 257 values)
+__device__ inline uint4 block_word(const BarArgs& A, uint32_t k) {
+  const uint64_t m = A.bmask[k];
+  const uint16_t* o = A.boff + 6 * size_t(k);
+  return make_uint4(uint32_t(m), uint32_t(m >> 32) | uint32_t(o[0]) << 4 | uint32_t(o[1]) << 16,
+                    uint32_t(o[2]) | uint32_t(o[3]) << 12, uint32_t(o[4]) | uint32_t(o[5]) << 12);
 }
-__device__ inline uint64_t slot_mask(const double* o, int b) {
-  return __builtin_bit_cast(uint64_t, b ? o[BO_DATA + 1] : o[BO_DATA]) & ((uint64_t(1) << 36) - 1);
+__device__ inline uint32_t word_mask(const uint4& w, int i) {  // of row i
+  return uint32_t((uint64_t(w.x) | uint64_t(w.y & 0xFu) << 32) >> (6 * i)) & 63u;
 }
-__device__ inline int slot_off(const double* o, int b, int i) {
-  const uint64_t lo = __builtin_bit_cast(uint64_t, b ? o[BO_DATA + 1] : o[BO_DATA]);
-  const uint64_t hi = __builtin_bit_cast(uint64_t, b ? o[BO_DATA + 3] : o[BO_DATA + 2]);
-  return i < 2 ? int((lo >> (36 + 12 * i)) & 0xFFFu) : int((hi >> (16 * (i - 2))) & 0xFFFFu);
+__device__ inline int word_off(const uint4& w, int i) {
+  const uint32_t h = i < 2 ? w.y >> 4 : (i < 4 ? w.z : w.w);
+  return int((i & 1 ? h >> 12 : h) & 0xFFFu);
 }
 
-// row i of an entry's blocks (p, p) -> self and (p, 1 - p) -> nb
-__device__ inline void entry_rows(const double* __restrict__ o, uint32_t type, int i, double self[6], double nb[6]) {
+// the entries' off-diagonal blocks, then the nodes' diagonal blocks (once per pattern)
+__global__ __launch_bounds__(256) void bar_block_kernel(BarArgs A, const uint32_t* __restrict__ elem, size_t n_entries,
+                                                        size_t n_nodes, uint4* __restrict__ entry,
+                                                        uint4* __restrict__ self) {
+  size_t s = blockIdx.x * size_t(blockDim.x) + threadIdx.x;
+  if (s < n_entries) {
+    const uint32_t u = A.entry_rec[s], type = u >> 31, p = u & 1u;
+    const size_t e = (elem[(u >> 1) & 0x3FFFFFFFu] >> 1) & 0x3FFFFFFFu;
+    entry[s] = block_word(A, A.bid[type][4 * e + 2 * p + (1 - p)]);
+    return;
+  }
+  s -= n_entries;
+  if (s >= n_nodes || A.inc_ptr[s] == A.inc_ptr[s + 1]) return;
+  const uint32_t u = A.inc[A.inc_ptr[s]], p = u & 1u;
+  self[s] = block_word(A, A.bid[u >> 31][4 * size_t((u >> 1) & 0x3FFFFFFFu) + 3 * p]);
+}
+
+// Row i = 3 h + m of an entry's blocks (p, p) -> self and (p, 1 - p) -> nb; o is
+// the element's record, rec the same in LDS, from which a lane takes column m of
+// R.  With v_t = T^T v_t,p the row is sum_t s_t v_t,i v_t in the order of t, where
+//   u: (b r0, 0)  v: (b r1, -r2/2)  w: (b r2, -r1/2)  tu, tv, tw: (0, b r0..r2);
+// products with those zeros are left out, and the other end's vectors (b turns
+// its sign) share their products: 60 FP64 operations where the general sum over
+// six-vectors took 110 and selected each v_t,i from six values.  This arithmetic
+// bounded the kernel (64 x 64 x 64 frame: 125 -> 86 us; without the arithmetic 75).
+__device__ inline void entry_rows(const double* __restrict__ o, const double* __restrict__ rec, uint32_t u, int h, int m,
+                                  double self[6], double nb[6]) {
+  const double x0 = rec[m];
+  if (u >> 31 == 0) {  // truss: rows and columns 0..2
 #pragma unroll
-  for (int j = 0; j < 6; ++j) { self[j] = 0.0; nb[j] = 0.0; }
-  if (type == 0) {
-    if (i >= 3) return;
-    const double ri = i == 0 ? o[0] : (i == 1 ? o[1] : o[2]);
+    for (int j = 0; j < 6; ++j) { self[j] = 0.0; nb[j] = 0.0; }
+    if (h) return;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      self[j] = (ri * o[3]) * o[j];
-      nb[j] = (ri * o[4]) * o[j];
+      self[j] = (x0 * o[3]) * o[j];
+      nb[j] = (x0 * o[4]) * o[j];
     }
     return;
   }
-  double R[9];
+  const double xv = rec[3 + 3 * h + m], xw = rec[6 - 3 * h + m];  // r1, r2 in a translation row; r2, r1 in a rotation row
+  const double b = u & 1u ? o[14] : -o[14];
+  const double bt = h ? 0.0 : b, br = h ? b : 0.0, bs = h ? -0.5 : b;
+  const double su = o[9] * (bt * x0), sv = o[10] * (bs * xv), sw = o[10] * (bs * xw);
+  const double s3 = o[11] * (br * x0), s4 = o[12] * (br * xw), s5 = o[13] * (br * xv);
 #pragma unroll
-  for (int m = 0; m < 9; ++m) R[m] = o[m];
-  const double bp = o[15], bq = -bp;
-#pragma unroll
-  for (int t = 0; t < 6; ++t) {
-    double vp[6], vq[6];
-    beam_term_vec(t, bp, R, vp);
-    beam_term_vec(t, bq, R, vq);
-    const double ai = i == 0 ? vp[0] : (i == 1 ? vp[1] : (i == 2 ? vp[2] : (i == 3 ? vp[3] : (i == 4 ? vp[4] : vp[5]))));
-    const double sa = o[9 + t] * ai;
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-      self[j] += sa * vp[j];
-      nb[j] += sa * vq[j];
-    }
+  for (int j = 0; j < 3; ++j) {
+    const double b0 = b * o[j], b1 = b * o[3 + j], b2 = b * o[6 + j];
+    const double t = __builtin_fma(sw, b2, __builtin_fma(sv, b1, su * b0));
+    self[j] = t;
+    nb[j] = -t;
+    const double r = __builtin_fma(sw, -0.5 * o[3 + j], sv * (-0.5 * o[6 + j]));
+    self[3 + j] = __builtin_fma(s5, b2, __builtin_fma(s4, b1, __builtin_fma(s3, b0, r)));
+    nb[3 + j] = __builtin_fma(-s5, b2, __builtin_fma(-s4, b1, __builtin_fma(-s3, b0, r)));
   }
 }
 
@@ -259,87 +246,92 @@ __device__ inline void wave_lds_sync() {
 }
 
 // row i of one block into the staged rows (r0: the row's start within them)
-__device__ inline void write_row(BarLds& L, uint64_t mask, int off_i, int i, int r0, const double v[6]) {
-  const uint32_t mi = uint32_t(mask >> (6 * i)) & 63u;
-  const int d0 = r0 + off_i;
+__device__ inline void write_row(BarLds& L, const uint4& w, int i, int r0, const double v[6]) {
+  const uint32_t mi = word_mask(w, i);
+  const int d0 = r0 + word_off(w, i);
 #pragma unroll
   for (int j = 0; j < 6; ++j)
     if ((mi >> j) & 1u) L.out[d0 + __builtin_popcount(mi & ((1u << j) - 1u))] = v[j];
 }
 
 // One workgroup per range of owned nodes: one lane per (owned node, row) forms
-// the rows in LDS, each entry's slot loaded during the previous entry's
-// arithmetic; then consecutive lanes write the range out.
+// the rows in LDS, element records loaded two entries ahead; then consecutive
+// lanes write the range out.  Bound: latency and LDS traffic at the three
+// workgroups per CU that the staged rows leave room for, close to the bytes
+// (64 x 64 x 64 frame: 86 us; 261 MB out and 130 MB in take 66 us at fill and
+// read rate).
 __global__ __launch_bounds__(BO_THREADS) void bar_owner_kernel(BarArgs A) {
   __shared__ BarLds L;
   const int t = threadIdx.x;
   const uint2 rg = A.ranges[blockIdx.x];
   const uint32_t a0 = rg.x, na = rg.y;
+  const uint32_t k0 = A.entry_ptr[blockIdx.x];
+  const int ne = int(A.entry_ptr[blockIdx.x + 1] - k0);  // <= BO_ENTRIES (cut on the host)
   const uint32_t e0 = A.inc_ptr[a0];
   const int64_t base = A.row_ptr[6 * size_t(a0)];
   const int nv = int(A.row_ptr[6 * size_t(a0 + na)] - base);  // <= BO_VALUES (cut on the host)
+  if (t < ne) {
+    L.block[t] = A.entry[k0 + t];
+    L.rec[t] = A.entry_rec[k0 + t];
+  }
   if (t <= int(na)) L.first[t] = A.inc_ptr[a0 + t] - e0;
   __syncthreads();
-  const double2* __restrict__ slots =
-      reinterpret_cast<const double2*>(A.slot + BO_SLOT * size_t(A.slot_ptr[blockIdx.x]));
   // lane (owned node j, row i), ten nodes per wave (lanes 60..63 idle here).
-  // The six lanes of a node load one entry slot together (lane i: 16-byte
-  // chunks i and i + 6) into the node's LDS slot, one entry ahead of the
-  // arithmetic, and each reads the whole slot from there.
+  // The six lanes of a node load one record together (lane i: 16-byte chunk i,
+  // lanes 0 and 1 also chunks 6 and 7) into the node's LDS slot, and each reads
+  // the whole record from there.
   const int jl = (t & 63) / 6, i = (t & 63) - 6 * jl;
-  const int j = 10 * (t >> 6) + jl;
+  const int j = 10 * (t >> 6) + jl, h = i >= 3;
   if (jl < 10 && j < int(na)) {
     const size_t a = size_t(a0) + j;
     const int r0 = int(A.row_ptr[6 * a + i] - base);
     const bool row = A.row_ptr[6 * a + i + 1] - base > r0;
     const int s0 = int(L.first[j]), s1 = int(L.first[j + 1]);
+    const uint4 diag = A.self[a];
     double2* __restrict__ buf = L.slot[j];
-    double2 c0 = make_double2(0.0, 0.0), c1 = c0;
+    const double2* __restrict__ recs = reinterpret_cast<const double2*>(A.rec);
+    // chunks of the records one and two entries ahead
+    double2 c0 = make_double2(0.0, 0.0), c1 = c0, f0 = c0, f1 = c0;
+    auto load = [&](int sl, double2& x0, double2& x1) {
+      if (sl >= s1) return;
+      const double2* r = recs + (BO_REC / 2) * size_t((L.rec[sl] >> 1) & 0x3FFFFFFFu) + i;
+      x0 = r[0];
+      if (i < 2) x1 = r[6];
+    };
+    load(s0, c0, c1);
+    load(s0 + 1, f0, f1);
     if (s1 > s0) {
-      c0 = slots[(BO_SLOT / 2) * s0 + i];
-      if (i < 4) c1 = slots[(BO_SLOT / 2) * s0 + 6 + i];
       buf[i] = c0;
-      if (i < 4) buf[6 + i] = c1;
-      if (s0 + 1 < s1) {
-        c0 = slots[(BO_SLOT / 2) * (s0 + 1) + i];
-        if (i < 4) c1 = slots[(BO_SLOT / 2) * (s0 + 1) + 6 + i];
-      }
+      if (i < 2) buf[6 + i] = c1;
     }
     wave_lds_sync();
     double acc[6];
-    uint64_t m0 = 0;  // block (a, a): mask and row offset, from the first entry
-    int o0 = 0;
     for (int sl = s0; sl < s1; ++sl) {
-      double o[BO_SLOT];
+      c0 = f0;
+      c1 = f1;
+      load(sl + 2, f0, f1);
+      double o[BO_REC];
 #pragma unroll
-      for (int m = 0; m < BO_SLOT / 2; ++m) {
+      for (int m = 0; m < BO_REC / 2; ++m) {
         const double2 v = buf[m];
         o[2 * m] = v.x;
         o[2 * m + 1] = v.y;
       }
       if (row) {
         double self[6], nb[6];
-        entry_rows(o, slot_type(o), i, self, nb);
+        entry_rows(o, reinterpret_cast<const double*>(buf), L.rec[sl], h, i - 3 * h, self, nb);
 #pragma unroll
         for (int q = 0; q < 6; ++q) acc[q] = sl == s0 ? self[q] : acc[q] + self[q];
-        if (sl == s0) {
-          m0 = slot_mask(o, 0);
-          o0 = slot_off(o, 0, i);
-        }
-        write_row(L, slot_mask(o, 1), slot_off(o, 1, i), i, r0, nb);
+        write_row(L, L.block[sl], i, r0, nb);
       }
       if (sl + 1 < s1) {
         wave_lds_sync();  // every lane of the node has read the slot
         buf[i] = c0;
-        if (i < 4) buf[6 + i] = c1;
+        if (i < 2) buf[6 + i] = c1;
         wave_lds_sync();
-        if (sl + 2 < s1) {
-          c0 = slots[(BO_SLOT / 2) * (sl + 2) + i];
-          if (i < 4) c1 = slots[(BO_SLOT / 2) * (sl + 2) + 6 + i];
-        }
       }
     }
-    if (row && s1 > s0) write_row(L, m0, o0, i, r0, acc);
+    if (row && s1 > s0) write_row(L, diag, i, r0, acc);
   }
   __syncthreads();
   double* __restrict__ dst = A.val + base;
@@ -471,23 +463,25 @@ BarArgs bar_args(Device* d, double* val) {
   A.inc_ptr = d->bo_inc_ptr;
   A.inc = d->bo_inc;
   A.ranges = reinterpret_cast<const uint2*>(d->bo_ranges);
-  A.slot = d->bo_slot;
-  A.slot_ptr = d->bo_slot_ptr;
+  A.rec = d->bo_rec;
+  A.entry_rec = d->bo_entry_rec;
+  A.entry_ptr = d->bo_entry_ptr;
+  A.entry = d->bo_entry;
+  A.self = d->bo_self;
   A.row_ptr = d->row_ptr;
   A.val = val;
   return A;
 }
 
-// (re)forms the bar kernel's entry slots from the current coordinates,
+// (re)forms the bar kernel's element records from the current coordinates,
 // frames and parameters
-std::string fill_bar_slots(Device* d, hipStream_t s) {
-  if (d->bo_n_slots) {
+std::string fill_bar_records(Device* d, hipStream_t s) {
+  if (d->bo_n_recs) {
     BarArgs A = bar_args(d, nullptr);
-    bar_slot_kernel<<<unsigned((d->bo_n_slots + 255) / 256), 256, 0, s>>>(A, d->bo_slot_inc, d->bo_n_slots,
-                                                                          d->bo_slot);
+    bar_record_kernel<<<unsigned((d->bo_n_recs + 255) / 256), 256, 0, s>>>(A, d->bo_rec_elem, d->bo_n_recs, d->bo_rec);
     HIP_TRY(hipGetLastError());
   }
-  d->bo_slot_dirty = false;
+  d->bo_rec_dirty = false;
   return "";
 }
 
@@ -504,11 +498,20 @@ std::string upload_bar_maps(Device* d, const BarMaps& bm) {
   d->bo_n_ranges = bm.n_bar_ranges;
   d->bo_n_truss_ranges = bm.ranges.size() / 2 - bm.n_bar_ranges;
   if (!(e = dupload(d->bo_inc, bm.inc.data(), bm.inc.size())).empty()) return e;
-  if (!(e = dupload(d->bo_slot_inc, bm.slot_inc.data(), bm.slot_inc.size())).empty()) return e;
-  if (!(e = dupload(d->bo_slot_ptr, bm.slot_ptr.data(), bm.slot_ptr.size())).empty()) return e;
-  d->bo_n_slots = bm.slot_inc.size();
-  if (!(e = dalloc(d->bo_slot, size_t(BO_SLOT) * d->bo_n_slots)).empty()) return e;
-  e = fill_bar_slots(d, nullptr);
+  if (!(e = dupload(d->bo_rec_elem, bm.rec_elem.data(), bm.rec_elem.size())).empty()) return e;
+  if (!(e = dupload(d->bo_entry_rec, bm.entry_rec.data(), bm.entry_rec.size())).empty()) return e;
+  if (!(e = dupload(d->bo_entry_ptr, bm.entry_ptr.data(), bm.entry_ptr.size())).empty()) return e;
+  d->bo_n_recs = bm.rec_elem.size();
+  const size_t ne = bm.entry_rec.size(), nn = ne ? bm.inc_ptr.size() - 1 : 0;
+  if (!(e = dalloc(d->bo_rec, size_t(BO_REC) * d->bo_n_recs)).empty()) return e;
+  if (!(e = dalloc(d->bo_entry, ne)).empty()) return e;
+  if (!(e = dalloc(d->bo_self, nn)).empty()) return e;
+  if (ne) {
+    BarArgs A = bar_args(d, nullptr);
+    bar_block_kernel<<<unsigned((ne + nn + 255) / 256), 256>>>(A, d->bo_rec_elem, ne, nn, d->bo_entry, d->bo_self);
+    HIP_TRY(hipGetLastError());
+  }
+  e = fill_bar_records(d, nullptr);
   if (!e.empty()) return e;
   HIP_TRY(hipDeviceSynchronize());
   return "";
@@ -516,8 +519,8 @@ std::string upload_bar_maps(Device* d, const BarMaps& bm) {
 
 std::string assemble_bar_owner(Device* d, double* val, void* stream, bool timed) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (d->bo_slot_dirty) {  // coordinates or parameters changed since the slots were formed
-    auto e = fill_bar_slots(d, s);
+  if (d->bo_rec_dirty) {  // coordinates or parameters changed since the records were formed
+    auto e = fill_bar_records(d, s);
     if (!e.empty()) return e;
   }
   if (timed) HIP_TRY(hipEventRecord(d->ev0, s));

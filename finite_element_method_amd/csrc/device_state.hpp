@@ -64,10 +64,11 @@ struct Device {
   uint16_t* bo_boff = nullptr;
   uint32_t *bo_inc_ptr = nullptr, *bo_inc = nullptr, *bo_ranges = nullptr;
   size_t bo_n_ranges = 0, bo_n_truss_ranges = 0;  // bar-kernel ranges, then truss-kernel ranges
-  uint32_t *bo_slot_inc = nullptr, *bo_slot_ptr = nullptr;
-  double* bo_slot = nullptr;   // staged entry constants of the bar-kernel ranges
-  size_t bo_n_slots = 0;
-  bool bo_slot_dirty = false;  // coordinates or bar parameters changed since bo_slot was filled
+  uint32_t *bo_rec_elem = nullptr, *bo_entry_rec = nullptr, *bo_entry_ptr = nullptr;
+  double* bo_rec = nullptr;    // element constants of the bar-kernel ranges
+  uint4 *bo_entry = nullptr, *bo_self = nullptr;  // masks and row offsets: off-diagonal per entry, diagonal per node
+  size_t bo_n_recs = 0;
+  bool bo_rec_dirty = false;   // coordinates or bar parameters changed since bo_rec was filled
   // adjoint maps
   uint32_t* adj_bid[3] = {nullptr, nullptr, nullptr};
   uint64_t* adj_bmask = nullptr;

@@ -61,7 +61,7 @@ void destroy_device(Device* d) {
   for (int t = 0; t < 3; ++t) { f(d->adj_bid[t]); f(d->adj_rec[t]); }
   for (int t = 0; t < 2; ++t) f(d->bo_bid[t]);
   f(d->bo_bmask); f(d->bo_boff); f(d->bo_inc_ptr); f(d->bo_inc); f(d->bo_ranges);
-  f(d->bo_slot_inc); f(d->bo_slot_ptr); f(d->bo_slot);
+  f(d->bo_rec_elem); f(d->bo_entry_rec); f(d->bo_entry_ptr); f(d->bo_rec); f(d->bo_entry); f(d->bo_self);
   f(d->adj_bmask); f(d->adj_boff); f(d->adj_inc_ptr); f(d->adj_xpos); f(d->adj_xs); f(d->adj_kpack); f(d->adj_eorder);
   f(d->sep_cons); f(d->sep_pack); f(d->sep_cls); f(d->sep_tmp); f(d->sep_disp); f(d->sep_force); f(d->sep_ra); f(d->sep_ub);
   f(d->sep_v); f(d->sep_flag); f(d->sep_pos); f(d->sep_key); f(d->sep_cnt); f(d->sep_off); f(d->sep_aa); f(d->sep_bb);
@@ -281,7 +281,7 @@ std::string update_params(Device* d, int type, const double* src, void* stream, 
     d->pl_geo_dirty = d->pn_geo_dirty = true;
     copy_plate_params_kernel<<<blocks_of(count), 256, 0, s>>>(src, n, d->params[PLATE], d->upd_words, d->upd_number);
   } else {
-    d->bo_slot_dirty = true;
+    d->bo_rec_dirty = true;
     copy_kernel<<<blocks_of(count), 256, 0, s>>>(src, count, d->params[type]);
   }
   HIP_TRY(hipGetLastError());
@@ -297,7 +297,7 @@ std::string update_nodes(Device* d, const double* src, void* stream, UpdateRepor
   auto e = begin_update(d);
   if (!e.empty()) return e;
   d->pl_geo_dirty = d->pn_geo_dirty = true;
-  d->bo_slot_dirty = true;
+  d->bo_rec_dirty = true;
   copy_kernel<<<blocks_of(n), 256, 0, s>>>(src, n, d->xyz);
   HIP_TRY(hipGetLastError());
   for (int t = 0; t < 3; ++t)

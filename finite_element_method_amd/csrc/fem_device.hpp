@@ -193,9 +193,10 @@ struct BarMaps {
   // nodes touch trusses only, to the truss kernel (<= 85 nodes, <= 512 entries)
   std::vector<uint32_t> ranges;
   size_t n_bar_ranges = 0;
-  // bar-kernel entries in range order: slot s holds the staged constants of
-  // entry slot_inc[s] (an index into inc); range r owns slots slot_ptr[r] ..
-  std::vector<uint32_t> slot_inc, slot_ptr;
+  // bar kernel: element records, in the order in which the ranges first meet
+  // their elements (type << 31 | element << 1), and the entries in range order
+  // (type << 31 | record << 1 | p); range r owns entries entry_ptr[r] ..
+  std::vector<uint32_t> rec_elem, entry_rec, entry_ptr;
 };
 constexpr int BAR_WG_NODES = 40, BAR_WG_ENTRIES = 256, BAR_WG_VALUES = 5120;
 constexpr int TRUSS_WG_NODES = 85, TRUSS_WG_ENTRIES = 512;

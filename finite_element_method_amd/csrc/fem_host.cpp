@@ -1367,11 +1367,22 @@ std::string build_pattern(fem_model* m) {
         a0 += na;
       }
       bm.n_bar_ranges = bm.ranges.size() / 2;
-      bm.slot_ptr.assign(1, 0);
+      bm.entry_ptr.assign(1, 0);
+      std::vector<uint32_t> record_of[2];
+      if (bm.n_bar_ranges)
+        for (int t = 0; t < 2; ++t) record_of[t].assign(m->set[t].size(), 0xFFFFFFFFu);
       for (size_t r = 0; r < bm.n_bar_ranges; ++r) {
         const uint32_t r0 = bm.ranges[2 * r], rn = bm.ranges[2 * r + 1];
-        for (uint32_t k = bm.inc_ptr[r0]; k < bm.inc_ptr[r0 + rn]; ++k) bm.slot_inc.push_back(k);
-        bm.slot_ptr.push_back(uint32_t(bm.slot_inc.size()));
+        for (uint32_t k = bm.inc_ptr[r0]; k < bm.inc_ptr[r0 + rn]; ++k) {
+          const uint32_t u = bm.inc[k];
+          uint32_t& at = record_of[u >> 31][(u >> 1) & 0x3FFFFFFFu];
+          if (at == 0xFFFFFFFFu) {
+            at = uint32_t(bm.rec_elem.size());
+            bm.rec_elem.push_back(u & ~1u);
+          }
+          bm.entry_rec.push_back((u & 0x80000001u) | at << 1);
+        }
+        bm.entry_ptr.push_back(uint32_t(bm.entry_rec.size()));
       }
       bm.ranges.insert(bm.ranges.end(), truss_ranges.begin(), truss_ranges.end());
     }

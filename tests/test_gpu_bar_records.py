@@ -1,0 +1,77 @@
+"""Frames and frames with trusses (bar_owner_kernel, element records shared by
+both ends) against the oracle and against the path that sums element
+contributions: node counts about the 40 nodes of a range, either end order,
+full masks (beams in any direction) and partial ones (along the axes), trusses
+beside beams on the same nodes, and updates of coordinates and parameters."""
+
+import numpy as np
+import pytest
+
+from finite_element_method_amd import BEAM, FEM, meshgen
+from oracle.oracle import OracleModel
+from tests.parity import compare, entry_bound, oracle_reference
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def _chain(n, seed, along_axes, trusses):
+    """A chain of n nodes (ends swapped at random), every other node braced to
+    the node three ahead by a beam or, with `trusses`, a truss."""
+    rng = np.random.default_rng(seed)
+    step = np.eye(3)[rng.integers(0, 3, n - 1)] if along_axes else rng.normal(size=(n - 1, 3)) + 1.5
+    xyz = np.vstack([np.zeros((1, 3)), np.cumsum(step, 0)])
+    conn = np.stack([np.arange(n - 1), np.arange(1, n)], 1)
+    braces = np.stack([np.arange(0, n - 3, 2), np.arange(3, n, 2)], 1)
+    conn = conn if trusses else np.vstack([conn, braces])
+    flip = rng.random(len(conn)) < 0.5
+    conn[flip] = conn[flip][:, ::-1]
+    axis = xyz[conn[:, 1]] - xyz[conn[:, 0]]
+    axis /= np.linalg.norm(axis, axis=1, keepdims=True)
+    v1 = rng.normal(size=axis.shape)
+    if along_axes:  # local axes along the axes too, where the beam lies along one
+        v1 = np.roll(axis, 1, axis=1) * [1.0, 2.0, 3.0]
+    v1 -= (v1 * axis).sum(1, keepdims=True) * axis
+    v1 /= np.linalg.norm(v1, axis=1, keepdims=True)
+    ne = len(conn)
+    props = np.stack([np.full(ne, 2.1e11), np.full(ne, 0.3), rng.uniform(1e-4, 1e-2, ne), rng.uniform(1e-8, 1e-6, ne),
+                      rng.uniform(1e-8, 1e-6, ne), np.zeros(ne), rng.uniform(1e-8, 1e-6, ne), np.full(ne, 5.0 / 6.0),
+                      v1[:, 0], v1[:, 1], v1[:, 2]], 1)
+    return xyz, conn.astype(np.uint32) + 1, props, (braces.astype(np.uint32) + 1 if trusses else None)
+
+
+def _load(model, xyz, conn, props, braces):
+    n, ne = len(xyz), len(conn)
+    model.add_nodes(np.arange(1, n + 1, dtype=np.uint32), xyz)
+    if braces is not None:
+        k = len(braces)
+        area = np.linspace(1e-4, 3e-4, k)
+        model.add_trusses(np.arange(ne + 1, ne + k + 1, dtype=np.uint32), braces, np.full(k, 2.1e11), area, np.full(k, np.nan))
+    model.add_beams(np.arange(1, ne + 1, dtype=np.uint32), conn, props)
+    return model
+
+
+@pytest.mark.parametrize("n,along_axes,trusses", [(4, False, False), (39, True, False), (40, False, True), (41, True, True),
+                                                  (41, False, False), (81, False, True), (123, True, False)])
+def test_chains_match_oracle_and_general_path(gpu, n, along_axes, trusses):
+    print("case", n, along_axes, trusses, flush=True)
+    data = _chain(n, n, along_axes, trusses)
+    ref = oracle_reference(_load(OracleModel(1e-4, 1e-12, n), *data))
+    m = _load(FEM.create(1e-4, 1e-12, n), *data)
+    got = m.stiffness_csr()
+    assert m.assembly_path() == "bar_owner"
+    r = compare(got, ref)
+    assert r["pattern_equal"] and r["max_ratio"] <= 1.0, r
+    m.set_option("force_generic", 1)
+    general = m.stiffness_csr()
+    assert np.array_equal(got[0], general[0]) and np.array_equal(got[1], general[1])
+    assert np.all(np.abs(got[2] - general[2]) <= entry_bound(ref[2], ref[3]))
+    m.set_option("force_generic", 0)
+    xyz, conn, props, braces = data
+    props = props.copy()
+    props[:, 2] *= 1.5
+    m.update_params(BEAM, torch.tensor(props, device="cuda"))
+    m.update_nodes(torch.tensor(1.25 * xyz, device="cuda"))
+    fresh = _load(FEM.create(1e-4, 1e-12, n), 1.25 * xyz, conn, props, braces)
+    assert all(np.array_equal(a, b) for a, b in zip(m.stiffness_csr(), fresh.stiffness_csr()))
