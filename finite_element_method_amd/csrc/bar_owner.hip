@@ -414,7 +414,7 @@ __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
   if (ne > 0) {
     TrussEntry E0, E1;
     truss_entry(A, A.inc[e0 + min(t, ne - 1)], E0);
-    truss_entry(A, A.inc[e0 + min(t + BO_THREADS, ne - 1)], E1);
+    if (ne > BO_THREADS) truss_entry(A, A.inc[e0 + min(t + BO_THREADS, ne - 1)], E1);
     if (t < ne) put_entry(L, t, E0);
     if (t + BO_THREADS < ne) put_entry(L, t + BO_THREADS, E1);
   }

@@ -41,6 +41,19 @@ def _chain(n, seed, along_axes, trusses):
     return xyz, conn.astype(np.uint32) + 1, props, (braces.astype(np.uint32) + 1 if trusses else None)
 
 
+@pytest.mark.parametrize("kind,size", [("truss", (2,)), ("truss", (3,)), ("truss", (12,)), ("truss", (13,)),
+                                       ("beam", (3, 3, 1)), ("beam", (10, 10, 10)), ("beam", (11, 10, 10))])
+def test_small_lattices_match_oracle(gpu, kind, size):
+    """Ranges of a small mesh: the least nodes per range and one more range, and
+    the sizes about which a range grows by a node."""
+    mesh = (meshgen.truss_lattice if kind == "truss" else meshgen.beam_frame)(*size, seed=size[0])
+    print("case", kind, mesh.n_nodes, flush=True)
+    ref = oracle_reference(meshgen.load_oracle(mesh, OracleModel))
+    m = FEM.from_mesh(mesh)
+    r = compare(m.stiffness_csr(), ref)
+    assert m.assembly_path() == "bar_owner" and r["pattern_equal"] and r["max_ratio"] <= 1.0, r
+
+
 def _load(model, xyz, conn, props, braces):
     n, ne = len(xyz), len(conn)
     model.add_nodes(np.arange(1, n + 1, dtype=np.uint32), xyz)
