@@ -46,7 +46,7 @@ struct AdjArgs {
   // flat plates, per (element, p): CSR position of row 6 a of corner p's node a,
   // and the block index k of each q (6 bits each) | nb << 24
   const uint2* kpack;
-  const uint32_t* eorder;  // flat plates: the elements in workgroup order
+  const uint32_t* eorder;  // dL/dK of beams and flat plates: the elements in workgroup order
   const int64_t* row_ptr;
   const uint4* rec;  // BlockPos records, or null
   double* dparam;  // n x params_per, may be null
@@ -82,12 +82,14 @@ __global__ __launch_bounds__(256) void adjoint_records_kernel(const uint32_t* __
                                                               const uint32_t* __restrict__ bid,
                                                               const uint64_t* __restrict__ bmask,
                                                               const uint16_t* __restrict__ boff,
-                                                              const int64_t* __restrict__ row_ptr, size_t n_pairs,
+                                                              const int64_t* __restrict__ row_ptr,
+                                                              const uint32_t* __restrict__ eorder, size_t n_pairs,
                                                               int nodes, uint4* __restrict__ rec) {
   const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n_pairs) return;
-  const size_t e = i / (nodes * nodes);
-  const uint32_t k = bid[i], a = conn[e * nodes + (i % (nodes * nodes)) / nodes];
+  const int pairs = nodes * nodes, pq = int(i % pairs);
+  const size_t e = eorder ? eorder[i / pairs] : i / pairs;
+  const uint32_t k = bid[e * pairs + pq], a = conn[e * nodes + pq / nodes];
   uint32_t pos[6];
 #pragma unroll
   for (int r = 0; r < 6; ++r) pos[r] = uint32_t(row_ptr[6 * size_t(a) + r] + boff[6 * size_t(k) + r]);
@@ -385,7 +387,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
     load_flat_k13(A.g + g0, nb, int(kp & 63u), nxt);
     load_flat_k13(A.g + g0, nb, int((kp >> 6) & 63u), nxt2);
   } else {
-    if (A.rec) pos = block_pos(A, 16 * e + 4 * p);
+    if (A.rec) pos = block_pos(A, 16 * i + 4 * p);
     ap = A.conn[4 * e + p];
   }
   double xl[6];
@@ -479,7 +481,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
     } else {
       if (A.rec) {
         gather_block(A, pos, gl);
-        if (q < 3) pos = block_pos(A, 16 * e + 4 * p + q + 1);
+        if (q < 3) pos = block_pos(A, 16 * i + 4 * p + q + 1);
       } else {
         gather_block_far(A, A.bid[16 * e + 4 * p + q], ap, gl);
       }
@@ -770,9 +772,10 @@ constexpr int beam_lanes() { return MODE == MODE_DLDK ? 4 : 1; }
 template <int MODE>
 __global__ __launch_bounds__(256) void beam_adjoint_kernel(AdjArgs A) {
   constexpr int LANES = beam_lanes<MODE>();
-  const size_t e = (size_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x) / LANES;
+  const size_t at = (size_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x) / LANES;
   const int pq0 = LANES == 4 ? int(threadIdx.x & 3u) : 0;
-  if (e >= A.n) return;  // whole quads: the four lanes share e
+  if (at >= A.n) return;  // whole quads: the four lanes share an element
+  const size_t e = MODE == MODE_DLDK ? A.eorder[at] : at;
   const uint32_t nd[2] = {A.conn[2 * e], A.conn[2 * e + 1]};
   double d[3];
 #pragma unroll
@@ -791,7 +794,7 @@ __global__ __launch_bounds__(256) void beam_adjoint_kernel(AdjArgs A) {
     double gl[36];
     if (MODE == MODE_DLDK) {
       if (A.rec)
-        gather_block(A, block_pos(A, 4 * e + pq), gl);
+        gather_block(A, block_pos(A, 4 * at + pq), gl);
       else
         gather_block_far(A, A.bid[4 * e + pq], nd[p], gl);
       to_local(gl, R);
@@ -865,7 +868,9 @@ std::string upload_adjoint_maps(Device* d, const AdjointMaps& am) {
   if (am.flat) {
     e = dupload(d->adj_kpack, am.kpack.data(), am.kpack.size());
     if (!e.empty()) return e;
-    e = dupload(d->adj_eorder, am.eorder.data(), am.eorder.size());
+  }
+  for (int t = 0; t < 3; ++t) {
+    e = dupload(d->adj_eorder[t], am.eorder[t].data(), am.eorder[t].size());
     if (!e.empty()) return e;
   }
   // block records of beams, and of plates where the flat kernel does not serve
@@ -879,7 +884,8 @@ std::string upload_adjoint_maps(Device* d, const AdjointMaps& am) {
     }
     if (!d->adj_rec[t]) continue;
     adjoint_records_kernel<<<unsigned((pairs + 255) / 256), 256>>>(d->conn[t], d->adj_bid[t], d->adj_bmask, d->adj_boff,
-                                                                   d->row_ptr, pairs, NODES_PER[t], d->adj_rec[t]);
+                                                                   d->row_ptr, d->adj_eorder[t], pairs, NODES_PER[t],
+                                                                   d->adj_rec[t]);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipDeviceSynchronize());
   }
@@ -906,7 +912,7 @@ std::string run_adjoint(Device* d, int mode, const double* g, double* const dpar
     A.bmask = d->adj_bmask;
     A.boff = d->adj_boff;
     A.kpack = reinterpret_cast<const uint2*>(d->adj_kpack);
-    A.eorder = d->adj_eorder;
+    A.eorder = d->adj_eorder[t];
     A.row_ptr = d->row_ptr;
     A.rec = d->adj_rec[t];
     A.dparam = dparam[t];

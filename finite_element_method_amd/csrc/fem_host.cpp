@@ -1538,29 +1538,55 @@ int ensure_adjoint(fem_model* m) {
           am.kpack[8 * e + 2 * p] = uint32_t(m->row_ptr_host[6 * size_t(a)]);
           am.kpack[8 * e + 2 * p + 1] = w;
         }
-      double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-      for (size_t a = 0; a < N; ++a)
-        for (int k = 0; k < 3; ++k) {
-          lo[k] = std::min(lo[k], m->xyz[3 * a + k]);
-          hi[k] = std::max(hi[k], m->xyz[3 * a + k]);
-        }
-      // Morton order of the element centroids on a 2^21 grid over the bounding
-      // box (a regular 2^k x 2^k mesh then falls into aligned 4 x 4 patches)
-      std::vector<std::pair<uint64_t, uint32_t>> ord(S.size());
-      for (size_t e = 0; e < S.size(); ++e) {
-        uint64_t code = 0;
-        for (int k = 0; k < 3; ++k) {
-          double c = 0.0;
-          for (int p = 0; p < 4; ++p) c += m->xyz[3 * size_t(S.conn[4 * e + p]) + k];
-          const double span = hi[k] - lo[k];
-          const double qd = span > 0 ? (0.25 * c - lo[k]) / span * 2097152.0 : 0.0;
-          code |= spread3(uint64_t(std::min(std::max(qd, 0.0), 2097151.0))) << k;
-        }
-        ord[e] = {code, uint32_t(e)};
+    }
+  }
+  // Flat plates and beams are taken in Morton order of their centroids: elements
+  // at one node read its rows while a cache holds them, in whatever order they
+  // were added (for shells it gave nothing).
+  if (am.flat || m->set[BEAM].size()) {
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    for (size_t a = 0; a < N; ++a)
+      for (int k = 0; k < 3; ++k) {
+        lo[k] = std::min(lo[k], m->xyz[3 * a + k]);
+        hi[k] = std::max(hi[k], m->xyz[3 * a + k]);
       }
+    auto code = [&](int t, size_t e, double cells) {
+      const int nn = femdev::NODES_PER[t];
+      uint64_t w = 0;
+      for (int k = 0; k < 3; ++k) {
+        double c = 0.0;
+        for (int p = 0; p < nn; ++p) c += m->xyz[3 * size_t(m->set[t].conn[nn * e + p]) + k];
+        const double span = hi[k] - lo[k];
+        const double qd = span > 0 ? (c / nn - lo[k]) / span * cells : 0.0;
+        w |= spread3(qd > 0.0 ? uint64_t(std::min(qd, cells - 1.0)) : 0) << k;
+      }
+      return w;
+    };
+    if (am.flat) {
+      // on a 2^21 grid over the bounding box: a regular 2^k x 2^k mesh falls
+      // into aligned 4 x 4 patches
+      const size_t n = m->set[PLATE].size();
+      std::vector<std::pair<uint64_t, uint32_t>> ord(n);
+      for (size_t e = 0; e < n; ++e) ord[e] = {code(PLATE, e, 2097152.0), uint32_t(e)};
       std::sort(ord.begin(), ord.end());
-      am.eorder.resize(S.size());
-      for (size_t i = 0; i < S.size(); ++i) am.eorder[i] = ord[i].second;
+      am.eorder[PLATE].resize(n);
+      for (size_t i = 0; i < n; ++i) am.eorder[PLATE][i] = ord[i].second;
+    }
+    if (const size_t n = m->set[BEAM].size()) {
+      // on a 2^10 grid, by three counting passes over ten bits each
+      std::vector<uint32_t> key(n), to(n), next(n);
+      for (size_t e = 0; e < n; ++e) {
+        key[e] = uint32_t(code(BEAM, e, 1024.0));
+        to[e] = uint32_t(e);
+      }
+      for (int shift = 0; shift < 30; shift += 10) {
+        std::vector<uint32_t> at(1025, 0);
+        for (size_t e = 0; e < n; ++e) at[((key[e] >> shift) & 1023u) + 1]++;
+        for (int k = 0; k < 1024; ++k) at[k + 1] += at[k];
+        for (size_t i = 0; i < n; ++i) next[at[(key[to[i]] >> shift) & 1023u]++] = to[i];
+        to.swap(next);
+      }
+      am.eorder[BEAM] = std::move(to);
     }
   }
   am.bmask = m->pat_bmask;
