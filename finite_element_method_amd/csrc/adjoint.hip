@@ -763,30 +763,35 @@ __global__ __launch_bounds__(256) void truss_adjoint_kernel(AdjArgs A) {
 // ---------------------------------------------------------------- beams
 
 // dL/dK: four lanes per beam, lane pq = block (p, q), so the four blocks'
-// scattered gathers run in parallel; lane 0 adds the term sums in block order
-// (pq = 0, 1, 2, 3) and writes the gradients.  Compliance: one lane per beam
-// (its two nodal displacements serve all four blocks).
+// scattered gathers run in parallel; the term sums are added in block order
+// (pq = 0, 1, 2, 3).  The parameter derivatives (angle, sines, divisions: about
+// half of the instructions) are then taken by the block's first wave, a lane per
+// beam, where every wave had one lane in four at it (frame of 26 k nodes: 28.4 ->
+// 24.8 us).  Compliance: one lane per beam (its two nodal displacements serve all
+// four blocks).
 template <int MODE>
 constexpr int beam_lanes() { return MODE == MODE_DLDK ? 4 : 1; }
 
 template <int MODE>
 __global__ __launch_bounds__(256) void beam_adjoint_kernel(AdjArgs A) {
   constexpr int LANES = beam_lanes<MODE>();
-  const size_t at = (size_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x) / LANES;
+  __shared__ double sums[LANES == 4 ? 64 * 7 : 1];
+  const size_t first = size_t(xcd_block(blockIdx.x, gridDim.x)) * (256 / LANES);
+  const size_t own = first + threadIdx.x / LANES;
   const int pq0 = LANES == 4 ? int(threadIdx.x & 3u) : 0;
-  if (at >= A.n) return;  // whole quads: the four lanes share an element
-  const size_t e = MODE == MODE_DLDK ? A.eorder[at] : at;
+  if (LANES == 1 && own >= A.n) return;
+  const size_t at = own < A.n ? own : A.n - 1;  // spare quads repeat the last beam
+  size_t e = MODE == MODE_DLDK ? A.eorder[at] : at;
   const uint32_t nd[2] = {A.conn[2 * e], A.conn[2 * e + 1]};
   double d[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) d[i] = A.xyz[3 * size_t(nd[1]) + i] - A.xyz[3 * size_t(nd[0]) + i];
   const double L = fem::norm3(d[0], d[1], d[2]);
-  const double J = fem::bar_jacobian(L);
+  double J = fem::bar_jacobian(L);
   const double inv_j = 1.0 / J;
   double R[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) R[k] = A.R[9 * e + k];
-  const double* prm = A.params + 11 * e;
   double S[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll 1
   for (int pq = pq0; pq < pq0 + 4 / LANES; ++pq) {
@@ -815,8 +820,20 @@ __global__ __launch_bounds__(256) void beam_adjoint_kernel(AdjArgs A) {
       const double s1 = quad_bcast<1>(S[k]), s2 = quad_bcast<2>(S[k]), s3 = quad_bcast<3>(S[k]);
       S[k] = ((S[k] + s1) + s2) + s3;
     }
-    if (pq0 != 0) return;
+    double* const mine = sums + 7 * (threadIdx.x >> 2);
+    if (pq0 == 0) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) mine[k] = S[k];
+      mine[6] = J;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64 || first + threadIdx.x >= A.n) return;
+    e = A.eorder[first + threadIdx.x];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) S[k] = sums[7 * threadIdx.x + k];
+    J = sums[7 * threadIdx.x + 6];
   }
+  const double* prm = A.params + 11 * e;
   double i11p, i22p, angle;
   fem::beam_principal(prm[3], prm[4], prm[5], A.rel_tol, i11p, i22p, angle);
   double gp[11];
