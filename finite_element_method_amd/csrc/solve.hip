@@ -14,7 +14,8 @@
 // An update is four launches: product, p.Ap, the vector update and the
 // direction.  The last two begin by summing the partial sums of the one before
 // in every workgroup (the same tree, so every workgroup has the same bits),
-// which takes the place of two one-workgroup launches per update.
+// which takes the place of two one-workgroup launches per update.  Up to FU_N
+// rows it is two (sv_direction_product).
 //
 // Small systems (SM_N rows, SM_NNZ entries) are solved by one workgroup, sv_small.
 #include <hip/hip_runtime.h>
@@ -1027,6 +1028,122 @@ __global__ __launch_bounds__(SM_T) void sv_small(const int64_t* __restrict__ rp,
   }
 }
 
+// ---- two launches per update
+//
+// For systems of up to FU_N rows an update of four launches is mostly launches.
+// Here the direction, K p and p.Ap are one: a workgroup owns 256 rows, forms the
+// entries of p that its columns name from the last z and p (the same fused
+// multiply-add that sv_direction does, so the same bits in every workgroup),
+// writes its own to `p_new` and its partial of p.Ap.  The other launch is the
+// vector update.  Sums follow the trees of sv_dot_it and sv_direction: the same
+// bits.  50 block-Jacobi updates with set-up, four launches and two:
+//   plates of 2541 rows 1001 -> 770 us, 14161: 969 -> 805, 55969: 1021 -> 866;
+//   frame of 45600: 1020 -> 850; trusses of 50700: 1053 -> 910.
+// FU_N is a workgroup per CU: with 76049 rows 1131 -> 1101, 136051: 1501 -> 1517
+// (a second round of workgroups, and the second gather).
+// turn: the update's; its predecessor left r.z and the stop flag in turn ^ 1.
+// with_direction: false for the first update after the scalars were read, whose
+// p is already the direction (and stays where it is).
+constexpr int64_t FU_N = 256 * SV_B;
+constexpr int FU_T = 1024;
+static_assert(3 * ((FU_N + SV_B - 1) / SV_B) <= 2 * SV_PARTS, "three sets of partials in the array of two");
+__global__ __launch_bounds__(FU_T) void sv_direction_product(const int64_t* __restrict__ rp,
+                                                             const int32_t* __restrict__ ci,
+                                                             const double* __restrict__ v, uint32_t v_bytes,
+                                                             const double* __restrict__ z, const double* __restrict__ p,
+                                                             double* __restrict__ p_new, double* __restrict__ ap,
+                                                             int64_t n, double* s, int turn, bool with_direction,
+                                                             const double* __restrict__ part_a,
+                                                             const double* __restrict__ part_b, double stop,
+                                                             double* __restrict__ part_pap) {
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  __shared__ double own_p[SV_B], own_ap[SV_B];
+  __shared__ Sum2 w[SV_B / 64];
+  const int t = threadIdx.x;
+  const bool first = blockIdx.x == 0 && t == 0;
+  double beta = 0.0;
+  if (!with_direction) {
+    if (s[S_DONE + turn] != 0.0) return;
+  } else {
+    if (s[S_DONE + (turn ^ 1)] != 0.0) {
+      if (first) s[S_DONE + turn] = 1.0;
+      return;
+    }
+    const double rz = s[S_RZ + (turn ^ 1)];
+    if (t < SV_B) {  // total_partials
+      double a = 0.0, b = 0.0;
+      for (unsigned i = t; i < gridDim.x; i += SV_B) {
+        a += part_a[i];
+        b += part_b[i];
+      }
+      a = wave_sum(a);
+      b = wave_sum(b);
+      if ((t & 63) == 0) w[t >> 6] = {a, b};
+    }
+    __syncthreads();
+    Sum2 sum = w[0];
+#pragma unroll
+    for (int k = 1; k < SV_B / 64; ++k) {
+      sum.a += w[k].a;
+      sum.b += w[k].b;
+    }
+    __syncthreads();  // w is written again below
+    beta = sum.a / rz;
+    // the host queues no update past the last one, so only convergence stops here
+    const bool conv = sqrt(sum.b) <= stop;
+    if (first) {
+      s[S_RZ + turn] = sum.a;
+      s[S_RR] = sum.b;
+      s[S_ITER] += 1.0;
+      s[S_CONV] = conv ? 1.0 : 0.0;
+      s[S_DONE + turn] = conv ? 1.0 : 0.0;
+    }
+    if (conv) return;
+  }
+  auto direction = [&](int32_t c) { return with_direction ? __builtin_fma(beta, p[c], z[c]) : p[c]; };
+  // Ap = K p: sv_spmv_it_quad
+  const int64_t r = int64_t(blockIdx.x) * SV_B + (t >> 2);
+  const int lig = t & 3;
+  if (r < n) {
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(v), 0, int(v_bytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(ci), 0, int(v_bytes / 2u), 0x00020000);
+    const int64_t end = rp[r + 1];
+    double acc = 0.0;
+    for (int64_t e = rp[r] + 4 * lig; e < end; e += 4 * SPMV_QUAD_LANES) {
+      const uint32_t ev = uint32_t(e);
+      const double2 w0 = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rv, 8u * ev, 0, 0));
+      const double2 w1 = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rv, 8u * ev + 16u, 0, 0));
+      const u32x4 c = __builtin_amdgcn_raw_buffer_load_b128(rc, 4u * ev, 0, 0);
+      // columns past the row end are valid indices or 0
+      const double p0 = direction(int32_t(c.x)), p1 = direction(int32_t(c.y));
+      const double p2 = direction(int32_t(c.z)), p3 = direction(int32_t(c.w));
+      acc = __builtin_fma(w0.x, p0, acc);
+      if (e + 1 < end) acc = __builtin_fma(w0.y, p1, acc);
+      if (e + 2 < end) acc = __builtin_fma(w1.x, p2, acc);
+      if (e + 3 < end) acc = __builtin_fma(w1.y, p3, acc);
+    }
+    acc += lane_xor<2>(acc);
+    acc += lane_xor<1>(acc);
+    if (lig == 0) own_ap[t >> 2] = acc;
+    if (lig == 1) own_p[t >> 2] = direction(int32_t(r));
+  }
+  __syncthreads();
+  if (t < SV_B) {
+    const int64_t i = int64_t(blockIdx.x) * SV_B + t;
+    double a = 0.0;
+    if (i < n) {
+      a = __builtin_fma(own_p[t], own_ap[t], 0.0);
+      ap[i] = own_ap[t];
+      if (with_direction) p_new[i] = own_p[t];
+    }
+    a = wave_sum(a);
+    if ((t & 63) == 0) w[t >> 6] = {a, 0.0};
+  }
+  __syncthreads();
+  if (t == 0) part_pap[blockIdx.x] = ((w[0].a + w[1].a) + w[2].a) + w[3].a;
+}
+
 // r_b: forces at the k_bb indexes
 __global__ void sv_gather(const double* __restrict__ src, const int64_t* __restrict__ idx, int64_t n,
                           double* __restrict__ dst) {
@@ -1123,9 +1240,6 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
   if (!(e = take(bufs, 8, size_t(2 * SV_PARTS), part)).empty()) return e;
   if (!(e = take(bufs, 9, size_t(S_COUNT), sc)).empty()) return e;
   double *b = vec[0], *x = vec[1], *r = vec[2], *z = vec[3], *p = vec[4], *ap = vec[5], *rr = vec[6], *rb = vec[7];
-  // partials: (r, z), (r, r), and p.Ap in b, which is not read after the start
-  // (it holds n values, at least one per block)
-  double *pa = part, *pb = part + SV_PARTS, *pc = b;
   double* host = bufs.host;
   const int64_t* rp[4];
   const int32_t* ci[4];
@@ -1151,6 +1265,12 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
   const unsigned parts = unsigned(std::min<int64_t>(SV_PARTS, grid_for(na, SV_B)));
   const bool quad = wide && size_t(d->sep_nnz[0]) * 8 < (size_t(1) << 32);
   const uint32_t v_bytes = quad ? uint32_t(size_t(d->sep_nnz[0]) * 8) : 0u;
+  // partials: (r, z), (r, r) and p.Ap.  b is not read after the start (it holds n
+  // values, at least one per block): it takes the third set, or with two launches
+  // per update, whose three sets fit `part`, the other direction
+  const bool fused = quad && na <= FU_N;
+  constexpr int FU_PARTS = 2 * SV_PARTS / 3;
+  double *pa = part, *pb = part + (fused ? FU_PARTS : SV_PARTS), *pc = fused ? part + 2 * FU_PARTS : b;
   double stop = 0.0;
   int it = 0;
   bool conv = false;
@@ -1238,25 +1358,31 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
       // kernel queued after that returns at once.  The count stays exact and the
       // host waits once per batch, not once per update.
       const unsigned spmv_blocks = grid_for(na * (quad ? SPMV_QUAD_LANES : SPMV_LANES), B);
+      double* p_other = b;
       Slices sl;
-      bool slice = quad && bufs.grows() && d->sep_nnz[0] >= SL_MIN_NNZ && max_iter >= SL_MIN_UPDATES;
+      bool slice = quad && !fused && bufs.grows() && d->sep_nnz[0] >= SL_MIN_NNZ && max_iter >= SL_MIN_UPDATES;
       uint32_t slice_total = 0;
       int queued = 0, batch = 1;
       for (;;) {
         const int nq = std::min(batch, max_iter - queued);
         for (int q = 0; q < nq; ++q) {
           const int turn = (queued + q) & 1;
-          if (sl.data)
+          if (fused) {
+            sv_direction_product<<<parts, FU_T, 0, s>>>(rp[0], ci[0], v[0], v_bytes, z, p, p_other, ap, na, sc, turn,
+                                                        q > 0, pa, pb, stop, pc);
+            if (q > 0) std::swap(p, p_other);
+          } else if (sl.data)
             sv_spmv_slices<<<grid_for(sl.n, 4), 256, 0, s>>>(sl.data, rp[0], sl.rows, sl.pairs, sl.cbase, sl.offset,
                                                              sl.n, p, ap, sc, turn);
           else if (quad) sv_spmv_it_quad<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, turn, v_bytes);
           else sv_spmv_it<<<spmv_blocks, B, 0, s>>>(rp[0], ci[0], v[0], p, ap, na, sc, turn);
-          sv_dot_it<<<parts, B, 0, s>>>(p, ap, na, sc, turn, pc);
+          if (!fused) sv_dot_it<<<parts, B, 0, s>>>(p, ap, na, sc, turn, pc);
           if (precond == 0)
             sv_update_jacobi<<<parts, B, 0, s>>>(diag, p, ap, sc, turn, pc, na, x, r, z, pa, pb);
           else
             sv_update_block<<<parts, B, 0, s>>>(inv, starts, nblk, p, ap, sc, turn, pc, x, r, z, pa, pb);
-          sv_direction<<<parts, B, 0, s>>>(z, sc, turn, pa, pb, stop, double(max_iter), na, p);
+          if (!fused || q + 1 == nq)
+            sv_direction<<<parts, B, 0, s>>>(z, sc, turn, pa, pb, stop, double(max_iter), na, p);
         }
         HIP_TRY(hipGetLastError());
         const bool first = queued == 0;

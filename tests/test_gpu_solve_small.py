@@ -60,6 +60,27 @@ def test_edges_match_the_reference(gpu, n_aa, pre):
     assert len(aa) == n_aa
 
 
+@pytest.mark.parametrize("pre", PRE)
+@pytest.mark.parametrize("n_aa", [2049, 2304, 2305, 30000, 65535, 65536, 65537])
+def test_first_updates_match_the_reference(gpu, n_aa, pre):
+    """Past one workgroup: two launches per update up to 65536 rows (256 per
+    workgroup), four above.  After 1 + 2 + 4 updates (three waits of the host)
+    the iterate agrees with the reference's: seven updates, each of a few sums
+    of at most 65537 products, stay far below 1e-10 of the solution's size."""
+    mesh = meshgen.plate_grid(108, 104, seed=n_aa) if n_aa > 3000 else meshgen.beam_frame(8, 8, 8, seed=1)
+    m = _clamped(mesh, (0, 1, 2, 3, 4, 5), n_aa, seed=n_aa)
+    mats, aa, bb, ra, ub = m.separate_sparse()
+    print("case", n_aa, pre, flush=True)
+    assert len(aa) == n_aa
+    b = find_b_sparse(ra, mats["ab"], ub)
+    for updates in (1, 7):
+        ua, rr, it, conv = m.solve_pcg(pre, updates)
+        x, it_ref, _ = pcg(mats["aa"], b, updates, m.rel_tol, m.abs_tol,
+                           block_starts(aa) if pre == "block_jacobi" else None)
+        assert it == it_ref == updates
+        assert np.linalg.norm(ua - x) <= 1e-10 * np.linalg.norm(x)
+
+
 def test_more_updates_than_one_launch(gpu):
     """A chain of 83 beams needs more Jacobi updates than one launch takes (4096)."""
     mesh = meshgen.beam_frame(84, 1, 1, seed=3)
