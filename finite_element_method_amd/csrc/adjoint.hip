@@ -46,7 +46,8 @@ struct AdjArgs {
   // flat plates, per (element, p): CSR position of row 6 a of corner p's node a,
   // and the block index k of each q (6 bits each) | nb << 24
   const uint2* kpack;
-  const uint32_t* eorder;  // dL/dK of beams and flat plates: the elements in workgroup order
+  const uint32_t* eorder;  // dL/dK: flat plates and beams (the beam, its nodes) in workgroup order
+  const uint4* beams;
   const int64_t* row_ptr;
   const uint4* rec;  // BlockPos records, or null
   double* dparam;  // n x params_per, may be null
@@ -83,12 +84,12 @@ __global__ __launch_bounds__(256) void adjoint_records_kernel(const uint32_t* __
                                                               const uint64_t* __restrict__ bmask,
                                                               const uint16_t* __restrict__ boff,
                                                               const int64_t* __restrict__ row_ptr,
-                                                              const uint32_t* __restrict__ eorder, size_t n_pairs,
+                                                              const uint4* __restrict__ beams, size_t n_pairs,
                                                               int nodes, uint4* __restrict__ rec) {
   const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n_pairs) return;
   const int pairs = nodes * nodes, pq = int(i % pairs);
-  const size_t e = eorder ? eorder[i / pairs] : i / pairs;
+  const size_t e = beams ? beams[i / pairs].x : i / pairs;
   const uint32_t k = bid[e * pairs + pq], a = conn[e * nodes + pq / nodes];
   uint32_t pos[6];
 #pragma unroll
@@ -112,10 +113,10 @@ __device__ inline void gather_block_far(const AdjArgs& A, uint32_t k, uint32_t a
 }
 
 // global-frame 6x6 gradient block at b: the block's entries of row i are
-// contiguous in the CSR row; load the run, then place it by the row mask.
-// With g_bytes set the run is read in 16-byte pairs (and one 8-byte tail) by
-// buffer loads, range-checked against g: half the memory requests of one load
-// per value, and the requests, not the bytes, bound this gather.
+// contiguous in the CSR row.  With g_bytes set they are read by buffer loads,
+// range-checked against g: full blocks in 16-byte pairs, half the requests of
+// one load per value.  (Frames of 512 and 33 k nodes, runs in pairs and then
+// moved to their places: kernels 10.8 and 25.7 us; one load per place: 9.4, 24.5.)
 __device__ inline void gather_block(const AdjArgs& A, const BlockPos& b, double G[36]) {
   const __amdgpu_buffer_rsrc_t rsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(A.g), 0, int(A.g_bytes), 0x00020000);
@@ -132,40 +133,24 @@ __device__ inline void gather_block(const AdjArgs& A, const BlockPos& b, double 
       }
     return;
   }
+  // otherwise one load per place; one that the mask leaves out is sent past the
+  // end of g, where loads return 0: no branches, and nothing to move afterwards
 #pragma unroll
   for (int i = 0; i < 6; ++i) {
     const uint32_t mi = uint32_t(b.mask >> (6 * i)) & 63u;
-    const int n = __builtin_popcount(mi);
-    double v[6];
-    if (A.g_bytes) {
-      const uint32_t byte = b.pos[i] * 8u;
-#pragma unroll
-      for (int c = 0; c < 6; c += 2) {
-        v[c] = 0.0;
-        v[c + 1] = 0.0;
-        if (c + 1 < n) {
-          const double2 w = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rsrc, byte + 8u * c, 0, 0));
-          v[c] = w.x;
-          v[c + 1] = w.y;
-        } else if (c < n) {
-          v[c] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, byte + 8u * c, 0, 0));
-        }
-      }
-    } else {
-      const double* src = A.g + b.pos[i];
-#pragma unroll
-      for (int c = 0; c < 6; ++c) v[c] = c < n ? src[c] : 0.0;
-    }
-    // open the gaps of the mask from the left
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
       const bool on = (mi >> j) & 1u;
-#pragma unroll
-      for (int c = 5; c > j; --c) v[c] = on ? v[c] : v[c - 1];
-      G[i * 6 + j] = on ? v[j] : 0.0;
+      const uint32_t at = b.pos[i] + uint32_t(__builtin_popcount(mi & ((1u << j) - 1u)));
+      if (A.g_bytes)
+        G[6 * i + j] = __builtin_bit_cast(
+            double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, on ? 8u * at : 0xFFFFFFF8u, 0, 0));
+      else
+        G[6 * i + j] = on ? A.g[at] : 0.0;
     }
   }
 }
+
 __device__ inline bool is_identity(const double R[9]) {
   return R[0] == 1.0 && R[4] == 1.0 && R[8] == 1.0 && R[1] == 0.0 && R[2] == 0.0 && R[3] == 0.0 && R[5] == 0.0 &&
          R[6] == 0.0 && R[7] == 0.0;
@@ -781,8 +766,17 @@ __global__ __launch_bounds__(256) void beam_adjoint_kernel(AdjArgs A) {
   const int pq0 = LANES == 4 ? int(threadIdx.x & 3u) : 0;
   if (LANES == 1 && own >= A.n) return;
   const size_t at = own < A.n ? own : A.n - 1;  // spare quads repeat the last beam
-  size_t e = MODE == MODE_DLDK ? A.eorder[at] : at;
-  const uint32_t nd[2] = {A.conn[2 * e], A.conn[2 * e + 1]};
+  size_t e = at;
+  uint32_t nd[2];
+  if (MODE == MODE_DLDK) {
+    const uint4 beam = A.beams[at];
+    e = beam.x;
+    nd[0] = beam.y;
+    nd[1] = beam.z;
+  } else {
+    nd[0] = A.conn[2 * e];
+    nd[1] = A.conn[2 * e + 1];
+  }
   double d[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) d[i] = A.xyz[3 * size_t(nd[1]) + i] - A.xyz[3 * size_t(nd[0]) + i];
@@ -828,7 +822,7 @@ __global__ __launch_bounds__(256) void beam_adjoint_kernel(AdjArgs A) {
     }
     __syncthreads();
     if (threadIdx.x >= 64 || first + threadIdx.x >= A.n) return;
-    e = A.eorder[first + threadIdx.x];
+    e = A.beams[first + threadIdx.x].x;
 #pragma unroll
     for (int k = 0; k < 6; ++k) S[k] = sums[7 * threadIdx.x + k];
     J = sums[7 * threadIdx.x + 6];
@@ -886,10 +880,10 @@ std::string upload_adjoint_maps(Device* d, const AdjointMaps& am) {
     e = dupload(d->adj_kpack, am.kpack.data(), am.kpack.size());
     if (!e.empty()) return e;
   }
-  for (int t = 0; t < 3; ++t) {
-    e = dupload(d->adj_eorder[t], am.eorder[t].data(), am.eorder[t].size());
-    if (!e.empty()) return e;
-  }
+  e = dupload(d->adj_eorder, am.eorder.data(), am.eorder.size());
+  if (!e.empty()) return e;
+  e = dupload(d->adj_beams, am.beams.data(), am.beams.size());
+  if (!e.empty()) return e;
   // block records of beams, and of plates where the flat kernel does not serve
   for (int t = 0; t < 3; ++t) {
     const size_t pairs = am.bid[t].size();
@@ -901,7 +895,9 @@ std::string upload_adjoint_maps(Device* d, const AdjointMaps& am) {
     }
     if (!d->adj_rec[t]) continue;
     adjoint_records_kernel<<<unsigned((pairs + 255) / 256), 256>>>(d->conn[t], d->adj_bid[t], d->adj_bmask, d->adj_boff,
-                                                                   d->row_ptr, d->adj_eorder[t], pairs, NODES_PER[t],
+                                                                   d->row_ptr,
+                                                                   t == BEAM ? reinterpret_cast<const uint4*>(d->adj_beams) : nullptr,
+                                                                   pairs, NODES_PER[t],
                                                                    d->adj_rec[t]);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipDeviceSynchronize());
@@ -929,7 +925,8 @@ std::string run_adjoint(Device* d, int mode, const double* g, double* const dpar
     A.bmask = d->adj_bmask;
     A.boff = d->adj_boff;
     A.kpack = reinterpret_cast<const uint2*>(d->adj_kpack);
-    A.eorder = d->adj_eorder[t];
+    A.eorder = d->adj_eorder;
+    A.beams = reinterpret_cast<const uint4*>(d->adj_beams);
     A.row_ptr = d->row_ptr;
     A.rec = d->adj_rec[t];
     A.dparam = dparam[t];

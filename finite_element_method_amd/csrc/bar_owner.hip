@@ -27,6 +27,7 @@
 //   row i of T^T (sum_t s_t v_t,p v_t,q^T) T = sum_t s_t (T^T v_t,p)_i (T^T v_t,q)^T.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 
 #include "device_state.hpp"
@@ -396,7 +397,11 @@ __device__ inline void put_entry(TrussLds& L, int sl, const TrussEntry& E) {
 // by their one element).  Staging: two entries per lane, loads of both in
 // flight together.  Off-diagonal rows: one task per (row, entry), so that
 // consecutive lanes write neighbouring blocks of one row.  Diagonal rows: one
-// lane per (owned node, row 0..2).
+// lane per (owned node, row 0..2).  TWO: some range has more entries than lanes
+// (11 x 11 x 11 lattice, whose ranges have not: 15.5 us per call, 14.5 without the
+// second entry; a branch on the range's own count costs the 40 x 40 x 40 lattice
+// 43.4 -> 45.1).
+template <bool TWO>
 __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
   __shared__ TrussLds L;
   const int t = threadIdx.x;
@@ -414,9 +419,9 @@ __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
   if (ne > 0) {
     TrussEntry E0, E1;
     truss_entry(A, A.inc[e0 + min(t, ne - 1)], E0);
-    if (ne > BO_THREADS) truss_entry(A, A.inc[e0 + min(t + BO_THREADS, ne - 1)], E1);
+    if (TWO) truss_entry(A, A.inc[e0 + min(t + BO_THREADS, ne - 1)], E1);
     if (t < ne) put_entry(L, t, E0);
-    if (t + BO_THREADS < ne) put_entry(L, t + BO_THREADS, E1);
+    if (TWO && t + BO_THREADS < ne) put_entry(L, t + BO_THREADS, E1);
   }
   __syncthreads();
   double* __restrict__ val = A.val + base;
@@ -497,6 +502,10 @@ std::string upload_bar_maps(Device* d, const BarMaps& bm) {
   if (!(e = dupload(d->bo_ranges, bm.ranges.data(), bm.ranges.size())).empty()) return e;
   d->bo_n_ranges = bm.n_bar_ranges;
   d->bo_n_truss_ranges = bm.ranges.size() / 2 - bm.n_bar_ranges;
+  d->bo_truss_entries = 0;
+  for (size_t r = bm.n_bar_ranges; r < bm.ranges.size() / 2; ++r)
+    d->bo_truss_entries = std::max(d->bo_truss_entries, int(bm.inc_ptr[bm.ranges[2 * r] + bm.ranges[2 * r + 1]] -
+                                                            bm.inc_ptr[bm.ranges[2 * r]]));
   if (!(e = dupload(d->bo_inc, bm.inc.data(), bm.inc.size())).empty()) return e;
   if (!(e = dupload(d->bo_rec_elem, bm.rec_elem.data(), bm.rec_elem.size())).empty()) return e;
   if (!(e = dupload(d->bo_entry_rec, bm.entry_rec.data(), bm.entry_rec.size())).empty()) return e;
@@ -532,7 +541,8 @@ std::string assemble_bar_owner(Device* d, double* val, void* stream, bool timed)
     }
     if (d->bo_n_truss_ranges) {
       A.ranges += d->bo_n_ranges;
-      truss_owner_kernel<<<unsigned(d->bo_n_truss_ranges), BO_THREADS, 0, s>>>(A);
+      auto kernel = d->bo_truss_entries > BO_THREADS ? truss_owner_kernel<true> : truss_owner_kernel<false>;
+      kernel<<<unsigned(d->bo_n_truss_ranges), BO_THREADS, 0, s>>>(A);
       HIP_TRY(hipGetLastError());
     }
   }

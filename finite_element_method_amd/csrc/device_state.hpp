@@ -64,6 +64,7 @@ struct Device {
   uint16_t* bo_boff = nullptr;
   uint32_t *bo_inc_ptr = nullptr, *bo_inc = nullptr, *bo_ranges = nullptr;
   size_t bo_n_ranges = 0, bo_n_truss_ranges = 0;  // bar-kernel ranges, then truss-kernel ranges
+  int bo_truss_entries = 0;    // most entries of a truss-kernel range
   uint32_t *bo_rec_elem = nullptr, *bo_entry_rec = nullptr, *bo_entry_ptr = nullptr;
   double* bo_rec = nullptr;    // element constants of the bar-kernel ranges
   uint4 *bo_entry = nullptr, *bo_self = nullptr;  // masks and row offsets: off-diagonal per entry, diagonal per node
@@ -74,7 +75,8 @@ struct Device {
   uint64_t* adj_bmask = nullptr;
   uint16_t* adj_boff = nullptr;
   uint32_t *adj_inc_ptr = nullptr, *adj_xpos = nullptr, *adj_kpack = nullptr;
-  uint32_t* adj_eorder[3] = {nullptr, nullptr, nullptr};  // beams, flat plates: elements in Morton order
+  uint32_t* adj_eorder = nullptr;  // flat plates: elements in Morton order
+  uint32_t* adj_beams = nullptr;   // beams likewise, four words each: the beam, its nodes, 0
   uint4* adj_rec[3] = {nullptr, nullptr, nullptr};  // per (element, node pair): its block's CSR positions and mask
   double* adj_xs = nullptr;
   int64_t adj_xoff[3] = {0, 0, 0};

@@ -58,7 +58,8 @@ void destroy_device(Device* d) {
   f(d->derived); f(d->truss_dir); f(d->row_ptr); f(d->col_idx); f(d->val); f(d->class_mask); f(d->class_off); f(d->contrib);
   f(d->slot_ptr); f(d->slot_src); f(d->pf_hdr); f(d->pf_conn); f(d->pf_eid); f(d->pf_rows); f(d->pf_oinfo);
   f(d->pf_oboff); f(d->pf_oooff); f(d->pf_blk); f(d->pf_obase);
-  for (int t = 0; t < 3; ++t) { f(d->adj_bid[t]); f(d->adj_rec[t]); f(d->adj_eorder[t]); }
+  for (int t = 0; t < 3; ++t) { f(d->adj_bid[t]); f(d->adj_rec[t]); }
+  f(d->adj_eorder); f(d->adj_beams);
   for (int t = 0; t < 2; ++t) f(d->bo_bid[t]);
   f(d->bo_bmask); f(d->bo_boff); f(d->bo_inc_ptr); f(d->bo_inc); f(d->bo_ranges);
   f(d->bo_rec_elem); f(d->bo_entry_rec); f(d->bo_entry_ptr); f(d->bo_rec); f(d->bo_entry); f(d->bo_self);

@@ -254,10 +254,10 @@ struct AdjointMaps {
   // flat: per (element, p) two words: the CSR position of row 6 a of corner
   // p's node a; the block index within a's rows of each q (6 bits each) | nb << 24
   std::vector<uint32_t> kpack;
-  // beams, flat plates: the elements in the order in which the dL/dK kernels
-  // take them (Morton order of the centroids: compact tiles, whose lanes'
-  // gathers share cache lines)
-  std::vector<uint32_t> eorder[3];
+  // flat plates: the elements in the order in which the dL/dK kernel takes them
+  // (Morton order of the centroids: compact tiles, whose lanes' gathers share
+  // cache lines); beams likewise, four words each: the beam, its nodes, 0
+  std::vector<uint32_t> eorder, beams;
 };
 std::string upload_adjoint_maps(Device* d, const AdjointMaps& am);
 // mode 0: g = dL/dK (nnz values, CSR order); mode 1: g = nodal displacements

@@ -1569,8 +1569,8 @@ int ensure_adjoint(fem_model* m) {
       std::vector<std::pair<uint64_t, uint32_t>> ord(n);
       for (size_t e = 0; e < n; ++e) ord[e] = {code(PLATE, e, 2097152.0), uint32_t(e)};
       std::sort(ord.begin(), ord.end());
-      am.eorder[PLATE].resize(n);
-      for (size_t i = 0; i < n; ++i) am.eorder[PLATE][i] = ord[i].second;
+      am.eorder.resize(n);
+      for (size_t i = 0; i < n; ++i) am.eorder[i] = ord[i].second;
     }
     if (const size_t n = m->set[BEAM].size()) {
       // on a 2^10 grid, by three counting passes over ten bits each
@@ -1586,7 +1586,13 @@ int ensure_adjoint(fem_model* m) {
         for (size_t i = 0; i < n; ++i) next[at[(key[to[i]] >> shift) & 1023u]++] = to[i];
         to.swap(next);
       }
-      am.eorder[BEAM] = std::move(to);
+      am.beams.resize(4 * n);
+      for (size_t i = 0; i < n; ++i) {
+        const uint32_t* c = &m->set[BEAM].conn[2 * size_t(to[i])];
+        am.beams[4 * i] = to[i];
+        am.beams[4 * i + 1] = c[0];
+        am.beams[4 * i + 2] = c[1];
+      }
     }
   }
   am.bmask = m->pat_bmask;
