@@ -69,7 +69,7 @@ __device__ inline unsigned xcd_block(unsigned b, unsigned nb) {
 // runs and its union mask, in one 32-byte record per (element, pair).  Looked up
 // through the pattern (pair -> block -> mask and row offsets -> row pointers)
 // the same costs four loads that wait for each other and 72 gathered bytes.
-// Frame of 33 x 33 x 33 nodes: 38.6 -> 34.1 us.
+// Frame of 32 x 32 x 32 nodes: 36.0 -> 34.1 us.
 struct BlockPos {
   uint32_t pos[6];
   uint64_t mask;
@@ -115,7 +115,7 @@ __device__ inline void gather_block_far(const AdjArgs& A, uint32_t k, uint32_t a
 // global-frame 6x6 gradient block at b: the block's entries of row i are
 // contiguous in the CSR row.  With g_bytes set they are read by buffer loads,
 // range-checked against g: full blocks in 16-byte pairs, half the requests of
-// one load per value.  (Frames of 512 and 33 k nodes, runs in pairs and then
+// one load per value.  (Frames of 2744 and 33 k nodes, runs in pairs and then
 // moved to their places: kernels 10.8 and 25.7 us; one load per place: 9.4, 24.5.)
 __device__ inline void gather_block(const AdjArgs& A, const BlockPos& b, double G[36]) {
   const __amdgpu_buffer_rsrc_t rsrc =
@@ -751,7 +751,7 @@ __global__ __launch_bounds__(256) void truss_adjoint_kernel(AdjArgs A) {
 // scattered gathers run in parallel; the term sums are added in block order
 // (pq = 0, 1, 2, 3).  The parameter derivatives (angle, sines, divisions: about
 // half of the instructions) are then taken by the block's first wave, a lane per
-// beam, where every wave had one lane in four at it (frame of 26 k nodes: 28.4 ->
+// beam, where every wave had one lane in four at it (frame of 37 k nodes: 28.4 ->
 // 24.8 us).  Compliance: one lane per beam (its two nodal displacements serve all
 // four blocks).
 template <int MODE>

@@ -138,7 +138,8 @@ struct fem_model {
 
 // A batch of independent meshes assembled together (no counterpart in the
 // crate).  Meshes are copied into per-group disjoint-union models: flat
-// plate-only meshes (fused plate kernel) and all others (generic path).  A
+// plate-only meshes, plates with frames of their own, trusses, models with
+// beams, and all others (summed through contributions).  A
 // mesh's nodes are a contiguous index range of its group, so its CSR rows and
 // values are contiguous slices of the group CSR and its values are summed in
 // its own element-insertion order, exactly as when it is assembled alone.

@@ -286,8 +286,8 @@ int fem_global_result(fem_model* m, uint32_t* node_numbers, int32_t* dofs, doubl
  * Many independent meshes assembled by one hipGraph launch.  The meshes'
  * nodes and elements are copied (at create) into per-group disjoint-union
  * models: flat plate-only meshes (fused plate kernel), truss and beam meshes
- * (node-owner kernels) and all others (generic path); the input handles are
- * not modified and may be destroyed afterwards.  Each mesh keeps its own CSR:
+ * (node-owner kernels), plates with frames of their own and all others (both
+ * "generic"); the input handles are not modified and may be destroyed afterwards.  Each mesh keeps its own CSR:
  * its rows and values are contiguous slices of its group's CSR, and every
  * value is summed in the mesh's own element order by the same value path as
  * when the mesh is assembled alone, so the results are identical.  All
@@ -337,18 +337,19 @@ int fem_batch_mesh_csr_to_host(fem_batch* b, size_t mesh, int64_t* row_ptr, int3
  *   "plate_wg_per_cu"    resident workgroups per CU of the fused plate kernels,
  *                        looping over the patches: 0..64 (0 = one workgroup
  *                        per patch; default 0 for plate_blocks, 2 for plate_fused)
- *   "force_generic"      1 = always use the generic value path
- *   "separate_lanes"     0 (default) = fem_separate's four-entry kernels where
- *                        the values span under 4 GiB (count 4 and fill 8 lanes
- *                        per CSR row), else one entry per lane with 4 or 8
- *                        lanes per row from the mean row length; 4, 8, 16, 32 =
- *                        the one-entry kernels with that many lanes.  The
- *                        separated matrices are bitwise equal either way
+ *   "force_generic"      1 = always sum element contributions through a buffer
+ *                        (the way of models that no other kernel takes)
+ *   "separate_lanes"     0 (default) = fem_separate's kernels that copy runs of
+ *                        entries where the values span under 4 GiB, else one
+ *                        entry per lane with 4 or 8 lanes per row from the mean
+ *                        row length; 4, 8, 16, 32 = the one-entry kernels with
+ *                        that many lanes.  The separated matrices are bitwise
+ *                        equal either way
  *   "wide_loads"         1 (default) = where the values span under 4 GiB,
- *                        the backward reads each row run of a dL/dK block, and
- *                        the PCG's SpMV four values per lane, with 16-byte
- *                        range-checked loads; 0 = one 8-byte load per value
- *                        (the paths taken above 4 GiB).  Gradients are bitwise
+ *                        the backward reads dL/dK blocks, and the PCG's SpMV
+ *                        four values per lane, with range-checked (16-byte)
+ *                        loads; 0 = one plain 8-byte load per value (the
+ *                        paths taken above 4 GiB).  Gradients are bitwise
  *                        equal either way; PCG iterates differ by rounding (the
  *                        SpMV sums a row in another order)
  *   "time_assembly"      1 (default) = events around every assembly launch
@@ -359,7 +360,8 @@ int fem_batch_mesh_csr_to_host(fem_batch* b, size_t mesh, int64_t* row_ptr, int3
 int fem_set_option(fem_model* m, const char* key, int64_t value);
 
 /* Name of the value path of the last assembly: "plate_lanes", "plate_blocks",
- * "plate_fused", "plate_corners", "bar_owner" or "generic". */
+ * "plate_fused", "plate_corners", "bar_owner" or "generic" (plates with frames
+ * of their own, and everything that is summed through contributions). */
 const char* fem_assembly_path(fem_model* m);
 
 #ifdef __cplusplus
