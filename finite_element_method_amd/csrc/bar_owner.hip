@@ -44,6 +44,7 @@ constexpr int BO_THREADS = 256;
 constexpr int BO_NODES = 40;     // owned nodes per workgroup (10 per wave, 6 row lanes each)
 constexpr int BO_ENTRIES = 256;  // (owned node, incident element) entries per workgroup
 constexpr int BO_REC = 16;       // doubles per element record
+constexpr int TO_REC = 6;        // truss kernel: doubles per element record (r, k_pp, k_pq, 0)
 constexpr int BO_VALUES = 5120;  // CSR values of the owned rows per workgroup
 constexpr int TO_NODES = 85;     // truss kernel: owned nodes per workgroup (3 row lanes each)
 constexpr int TO_ENTRIES = 512;  // truss kernel: entries per workgroup
@@ -85,12 +86,11 @@ static_assert(BO_NODES == BAR_WG_NODES && BO_ENTRIES == BAR_WG_ENTRIES && BO_VAL
 // so the layout is compact (four workgroups per CU) and a range holds twice
 // the entries.
 struct TrussLds {
-  double data[TO_ENTRIES][5];      // r (3), kpp, kpq
-  uint64_t mask[TO_ENTRIES][2];    // masks of the entry's blocks (p, p) and (p, 1 - p)
-  uint16_t off[TO_ENTRIES][2][3];  // offsets of rows 0..2 of those blocks
-  uint8_t node[TO_ENTRIES];        // owned node of the entry
+  double data[TO_ENTRIES][5];  // r (3), kpp, kpq
+  uint4 block[TO_ENTRIES];     // the entry's off-diagonal block
+  uint8_t node[TO_ENTRIES];    // owned node of the entry
   uint32_t first[TO_NODES + 1];
-  uint32_t row[TO_NODES][3];       // start of rows 0..2 of each owned node, from the range's first value
+  uint32_t row[TO_NODES][3];   // start of rows 0..2 of each owned node, from the range's first value
 };
 static_assert(4 * sizeof(TrussLds) <= 160 * 1024, "four workgroups per CU");
 static_assert(TO_NODES == TRUSS_WG_NODES && TO_ENTRIES == TRUSS_WG_ENTRIES && 3 * TO_NODES <= BO_THREADS, "range cut");
@@ -162,10 +162,23 @@ __device__ inline void form_record(const BarArgs& A, uint32_t u, double* __restr
   for (int k = 0; k < BO_REC / 2; ++k) dst[k] = make_double2(o[2 * k], o[2 * k + 1]);
 }
 
+// trusses of the truss kernel's ranges, formed in the same launch (blocks after the first n)
+__device__ inline void form_truss_record(const BarArgs& A, uint32_t u, double* __restrict__ rec) {
+  double o[TO_REC];
+  o[5] = 0.0;
+  truss_constants(A, (u >> 1) & 0x3FFFFFFFu, 0, o);
+  double2* dst = reinterpret_cast<double2*>(rec);
+#pragma unroll
+  for (int k = 0; k < TO_REC / 2; ++k) dst[k] = make_double2(o[2 * k], o[2 * k + 1]);
+}
+
 __global__ __launch_bounds__(256) void bar_record_kernel(BarArgs A, const uint32_t* __restrict__ elem, size_t n,
-                                                         double* __restrict__ rec) {
+                                                         double* __restrict__ rec,
+                                                         const uint32_t* __restrict__ truss_elem, size_t n_truss,
+                                                         double* __restrict__ truss_rec) {
   const size_t s = blockIdx.x * size_t(blockDim.x) + threadIdx.x;
   if (s < n) form_record(A, elem[s], rec + BO_REC * s);
+  else if (s - n < n_truss) form_truss_record(A, truss_elem[s - n], truss_rec + TO_REC * (s - n));
 }
 
 // a block's mask (36 bits) and the offsets of its rows within the owned node's
@@ -351,45 +364,32 @@ __global__ __launch_bounds__(BO_THREADS) void bar_owner_kernel(BarArgs A) {
 }
 
 // row i < 3 of a truss block (columns 0..2) straight to the CSR
-__device__ inline void write_row3(double* val, uint64_t mask, int off, int i, int64_t r0, const double v[3]) {
-  const uint32_t mi = uint32_t(mask >> (6 * i)) & 7u;
-  double* dst = val + (r0 + off);
+__device__ inline void write_row3(double* val, const uint4& w, int i, int64_t r0, const double v[3]) {
+  const uint32_t mi = word_mask(w, i) & 7u;
+  double* dst = val + (r0 + word_off(w, i));
 #pragma unroll
   for (int j = 0; j < 3; ++j)
     if ((mi >> j) & 1u) dst[__builtin_popcount(mi & ((1u << j) - 1u))] = v[j];
 }
 
-// one truss entry's constants, masks and row offsets (registers)
+// one truss entry (registers)
 struct TrussEntry {
-  double o[5];
-  uint64_t m[2];
-  uint16_t off[2][3];
+  double2 o[TO_REC / 2];
+  uint4 block;
 };
-
-__device__ inline void truss_entry(const BarArgs& A, uint32_t u, TrussEntry& E) {
-  const int p = int(u & 1u);
-  const size_t e = (u >> 1) & 0x3FFFFFFFu;
-  truss_constants(A, e, p, E.o);
-  const uint32_t ks = A.bid[0][4 * e + 3 * p], kn = A.bid[0][4 * e + 2 * p + (1 - p)];
-  E.m[0] = A.bmask[ks];
-  E.m[1] = A.bmask[kn];
+__device__ inline void truss_entry(const BarArgs& A, uint32_t k, TrussEntry& E) {
+  const double2* r = reinterpret_cast<const double2*>(A.rec) + (TO_REC / 2) * size_t(A.entry_rec[k] >> 1);
+  E.block = A.entry[k];
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    E.off[0][i] = A.boff[6 * size_t(ks) + i];
-    E.off[1][i] = A.boff[6 * size_t(kn) + i];
-  }
+  for (int m = 0; m < TO_REC / 2; ++m) E.o[m] = r[m];
 }
-
 __device__ inline void put_entry(TrussLds& L, int sl, const TrussEntry& E) {
-#pragma unroll
-  for (int k = 0; k < 5; ++k) L.data[sl][k] = E.o[k];
-  L.mask[sl][0] = E.m[0];
-  L.mask[sl][1] = E.m[1];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    L.off[sl][0][i] = E.off[0][i];
-    L.off[sl][1][i] = E.off[1][i];
-  }
+  L.data[sl][0] = E.o[0].x;
+  L.data[sl][1] = E.o[0].y;
+  L.data[sl][2] = E.o[1].x;
+  L.data[sl][3] = E.o[1].y;
+  L.data[sl][4] = E.o[2].x;
+  L.block[sl] = E.block;
 }
 
 // Truss-only ranges: the same sums as bar_owner_kernel (diagonal block summed
@@ -409,6 +409,7 @@ __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
   const uint32_t a0 = rg.x, na = rg.y;
   const uint32_t e0 = A.inc_ptr[a0];
   const int ne = int(A.inc_ptr[a0 + na] - e0);  // <= TO_ENTRIES (cut on the host)
+  const uint32_t k0 = A.entry_ptr[blockIdx.x];
   const int64_t base = A.row_ptr[6 * size_t(a0)];
   if (t <= int(na)) L.first[t] = A.inc_ptr[a0 + t] - e0;
   if (t < int(na)) {
@@ -418,8 +419,8 @@ __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
   if (t < 3 * int(na)) L.row[t / 3][t % 3] = uint32_t(A.row_ptr[6 * size_t(a0 + t / 3) + t % 3] - base);
   if (ne > 0) {
     TrussEntry E0, E1;
-    truss_entry(A, A.inc[e0 + min(t, ne - 1)], E0);
-    if (TWO) truss_entry(A, A.inc[e0 + min(t + BO_THREADS, ne - 1)], E1);
+    truss_entry(A, k0 + min(t, ne - 1), E0);
+    if (TWO) truss_entry(A, k0 + min(t + BO_THREADS, ne - 1), E1);
     if (t < ne) put_entry(L, t, E0);
     if (TWO && t + BO_THREADS < ne) put_entry(L, t + BO_THREADS, E1);
   }
@@ -432,7 +433,7 @@ __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
     double nb[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) nb[q] = s * o[q];
-    write_row3(val, L.mask[sl][1], L.off[sl][1][i], i, L.row[L.node[sl]][i], nb);
+    write_row3(val, L.block[sl], i, L.row[L.node[sl]][i], nb);
   }
   const int j = t / 3, i = t % 3;
   if (j >= int(na)) return;
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
 #pragma unroll
     for (int q = 0; q < 3; ++q) acc[q] = sl == s0 ? s * o[q] : acc[q] + s * o[q];
   }
-  write_row3(val, L.mask[s0][0], L.off[s0][0][i], i, L.row[j][i], acc);
+  write_row3(val, A.self[a0 + j], i, L.row[j][i], acc);
 }
 
 }  // namespace
@@ -481,9 +482,10 @@ BarArgs bar_args(Device* d, double* val) {
 // (re)forms the bar kernel's element records from the current coordinates,
 // frames and parameters
 std::string fill_bar_records(Device* d, hipStream_t s) {
-  if (d->bo_n_recs) {
+  if (d->bo_n_recs + d->to_n_recs) {
     BarArgs A = bar_args(d, nullptr);
-    bar_record_kernel<<<unsigned((d->bo_n_recs + 255) / 256), 256, 0, s>>>(A, d->bo_rec_elem, d->bo_n_recs, d->bo_rec);
+    bar_record_kernel<<<unsigned((d->bo_n_recs + d->to_n_recs + 255) / 256), 256, 0, s>>>(
+        A, d->bo_rec_elem, d->bo_n_recs, d->bo_rec, d->to_rec_elem, d->to_n_recs, d->to_rec);
     HIP_TRY(hipGetLastError());
   }
   d->bo_rec_dirty = false;
@@ -511,14 +513,25 @@ std::string upload_bar_maps(Device* d, const BarMaps& bm) {
   if (!(e = dupload(d->bo_entry_rec, bm.entry_rec.data(), bm.entry_rec.size())).empty()) return e;
   if (!(e = dupload(d->bo_entry_ptr, bm.entry_ptr.data(), bm.entry_ptr.size())).empty()) return e;
   d->bo_n_recs = bm.rec_elem.size();
-  const size_t ne = bm.entry_rec.size(), nn = ne ? bm.inc_ptr.size() - 1 : 0;
+  if (!(e = dupload(d->to_rec_elem, bm.truss_elem.data(), bm.truss_elem.size())).empty()) return e;
+  if (!(e = dupload(d->to_entry_rec, bm.truss_entry.data(), bm.truss_entry.size())).empty()) return e;
+  if (!(e = dupload(d->to_entry_ptr, bm.truss_ptr.data(), bm.truss_ptr.size())).empty()) return e;
+  d->to_n_recs = bm.truss_elem.size();
+  const size_t ne = bm.entry_rec.size(), nt = bm.truss_entry.size(), nn = ne + nt ? bm.inc_ptr.size() - 1 : 0;
   if (!(e = dalloc(d->bo_rec, size_t(BO_REC) * d->bo_n_recs)).empty()) return e;
   if (!(e = dalloc(d->bo_entry, ne)).empty()) return e;
   if (!(e = dalloc(d->bo_self, nn)).empty()) return e;
-  if (ne) {
+  if (!(e = dalloc(d->to_rec, size_t(TO_REC) * d->to_n_recs)).empty()) return e;
+  if (!(e = dalloc(d->to_entry, nt)).empty()) return e;
+  if (nn) {
     BarArgs A = bar_args(d, nullptr);
     bar_block_kernel<<<unsigned((ne + nn + 255) / 256), 256>>>(A, d->bo_rec_elem, ne, nn, d->bo_entry, d->bo_self);
     HIP_TRY(hipGetLastError());
+    if (nt) {
+      A.entry_rec = d->to_entry_rec;
+      bar_block_kernel<<<unsigned((nt + 255) / 256), 256>>>(A, d->to_rec_elem, nt, 0, d->to_entry, d->bo_self);
+      HIP_TRY(hipGetLastError());
+    }
   }
   e = fill_bar_records(d, nullptr);
   if (!e.empty()) return e;
@@ -541,6 +554,10 @@ std::string assemble_bar_owner(Device* d, double* val, void* stream, bool timed)
     }
     if (d->bo_n_truss_ranges) {
       A.ranges += d->bo_n_ranges;
+      A.rec = d->to_rec;
+      A.entry = d->to_entry;
+      A.entry_rec = d->to_entry_rec;
+      A.entry_ptr = d->to_entry_ptr;
       auto kernel = d->bo_truss_entries > BO_THREADS ? truss_owner_kernel<true> : truss_owner_kernel<false>;
       kernel<<<unsigned(d->bo_n_truss_ranges), BO_THREADS, 0, s>>>(A);
       HIP_TRY(hipGetLastError());

@@ -69,6 +69,10 @@ struct Device {
   double* bo_rec = nullptr;    // element constants of the bar-kernel ranges
   uint4 *bo_entry = nullptr, *bo_self = nullptr;  // masks and row offsets: off-diagonal per entry, diagonal per node
   size_t bo_n_recs = 0;
+  uint32_t *to_rec_elem = nullptr, *to_entry_rec = nullptr, *to_entry_ptr = nullptr;  // the truss kernel's
+  double* to_rec = nullptr;
+  uint4* to_entry = nullptr;
+  size_t to_n_recs = 0;
   bool bo_rec_dirty = false;   // coordinates or bar parameters changed since bo_rec was filled
   // adjoint maps
   uint32_t* adj_bid[3] = {nullptr, nullptr, nullptr};

@@ -197,6 +197,7 @@ struct BarMaps {
   // their elements (type << 31 | element << 1), and the entries in range order
   // (type << 31 | record << 1 | p); range r owns entries entry_ptr[r] ..
   std::vector<uint32_t> rec_elem, entry_rec, entry_ptr;
+  std::vector<uint32_t> truss_elem, truss_entry, truss_ptr;  // the truss kernel's, the same way
 };
 constexpr int BAR_WG_NODES = 40, BAR_WG_ENTRIES = 256, BAR_WG_VALUES = 5120;
 constexpr int TRUSS_WG_NODES = 85, TRUSS_WG_ENTRIES = 512;

@@ -1394,6 +1394,24 @@ std::string build_pattern(fem_model* m) {
         }
         bm.entry_ptr.push_back(uint32_t(bm.entry_rec.size()));
       }
+      // the truss kernel's records and entries likewise
+      if (!truss_ranges.empty()) {
+        std::vector<uint32_t> at(m->set[TRUSS].size(), 0xFFFFFFFFu);
+        for (size_t r = 0; r < truss_ranges.size() / 2; ++r) {
+          const uint32_t r0 = truss_ranges[2 * r], rn = truss_ranges[2 * r + 1];
+          bm.truss_ptr.push_back(uint32_t(bm.truss_entry.size()));
+          for (uint32_t k = bm.inc_ptr[r0]; k < bm.inc_ptr[r0 + rn]; ++k) {
+            const uint32_t u = bm.inc[k];
+            uint32_t& rec = at[(u >> 1) & 0x3FFFFFFFu];
+            if (rec == 0xFFFFFFFFu) {
+              rec = uint32_t(bm.truss_elem.size());
+              bm.truss_elem.push_back(u & ~1u);
+            }
+            bm.truss_entry.push_back(rec << 1 | (u & 1u));
+          }
+        }
+        bm.truss_ptr.push_back(uint32_t(bm.truss_entry.size()));
+      }
       bm.ranges.insert(bm.ranges.end(), truss_ranges.begin(), truss_ranges.end());
     }
     if (ok && blocks.size() < (size_t(1) << 32)) {
