@@ -82,17 +82,21 @@ static_assert(3 * sizeof(BarLds) <= 160 * 1024, "three workgroups per CU");
 
 static_assert(BO_NODES == BAR_WG_NODES && BO_ENTRIES == BAR_WG_ENTRIES && BO_VALUES == BAR_WG_VALUES, "range cut");
 
-// Truss-only ranges: rows 3..5 are empty and an entry needs five constants,
-// so the layout is compact (four workgroups per CU) and a range holds twice
-// the entries.
+// Truss-only ranges: rows 3..5 are empty and an entry needs five constants, so
+// the layout is compact and a range holds up to twice the entries.
+template <int ENTRIES, int VALUES>
 struct TrussLds {
-  double data[TO_ENTRIES][5];  // r (3), kpp, kpq
-  uint4 block[TO_ENTRIES];     // the entry's off-diagonal block
-  uint8_t node[TO_ENTRIES];    // owned node of the entry
+  double out[VALUES];          // the owned rows, one place in where their CSR position is odd
+  double data[ENTRIES][5];     // r (3), kpp, kpq
+  uint4 block[ENTRIES];        // the entry's off-diagonal block
+  uint8_t node[ENTRIES];       // owned node of the entry
   uint32_t first[TO_NODES + 1];
   uint32_t row[TO_NODES][3];   // start of rows 0..2 of each owned node, from the range's first value
 };
-static_assert(4 * sizeof(TrussLds) <= 160 * 1024, "four workgroups per CU");
+constexpr int TO_STAGED = TRUSS_WG_STAGED;
+static_assert(4 * sizeof(TrussLds<TO_STAGED, TRUSS_WG_VALUES + 2>) <= 160 * 1024, "four workgroups per CU");
+static_assert(5 * sizeof(TrussLds<TO_ENTRIES, 2>) <= 160 * 1024, "five workgroups per CU");
+static_assert(TO_STAGED <= BO_THREADS, "an entry per lane");
 static_assert(TO_NODES == TRUSS_WG_NODES && TO_ENTRIES == TRUSS_WG_ENTRIES && 3 * TO_NODES <= BO_THREADS, "range cut");
 
 // Jacobian of element e of `type` and the nodal shape derivatives b_p, b_q
@@ -383,7 +387,8 @@ __device__ inline void truss_entry(const BarArgs& A, uint32_t k, TrussEntry& E) 
 #pragma unroll
   for (int m = 0; m < TO_REC / 2; ++m) E.o[m] = r[m];
 }
-__device__ inline void put_entry(TrussLds& L, int sl, const TrussEntry& E) {
+template <class Lds>
+__device__ inline void put_entry(Lds& L, int sl, const TrussEntry& E) {
   L.data[sl][0] = E.o[0].x;
   L.data[sl][1] = E.o[0].y;
   L.data[sl][2] = E.o[1].x;
@@ -394,16 +399,19 @@ __device__ inline void put_entry(TrussLds& L, int sl, const TrussEntry& E) {
 
 // Truss-only ranges: the same sums as bar_owner_kernel (diagonal block summed
 // in insertion order from the first contribution, off-diagonal blocks written
-// by their one element).  Staging: two entries per lane, loads of both in
-// flight together.  Off-diagonal rows: one task per (row, entry), so that
-// consecutive lanes write neighbouring blocks of one row.  Diagonal rows: one
-// lane per (owned node, row 0..2).  TWO: some range has more entries than lanes
-// (11 x 11 x 11 lattice, whose ranges have not: 15.5 us per call, 14.5 without the
-// second entry; a branch on the range's own count costs the 40 x 40 x 40 lattice
-// 43.4 -> 45.1).
-template <bool TWO>
+// by their one element).  Entries come through 48-byte element records and the
+// pattern's words, as the bar kernel's (a chain of look-ups per entry and 37 loads
+// per wave before: 40 x 40 x 40 lattice 43.9 -> 39.5 us per call).  Off-diagonal
+// rows: one task per (row, entry), so that consecutive lanes write neighbouring
+// blocks of one row.  Diagonal rows: one lane per (owned node, row 0..2).
+//   STAGED: an entry per lane at most, rows staged in LDS and written as
+//   16-byte chunks; four workgroups per CU.  Latency-bound meshes gain (11 x 11 x
+//   11 lattice 14.2 -> 12.9 us per call, 26 x 26 x 26 18.1 -> 16.8).
+//   Otherwise rows straight to the CSR, five workgroups per CU; TWO: some range
+//   has more entries than lanes, the loads of a lane's two in flight together.
+template <bool TWO, bool STAGED>
 __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
-  __shared__ TrussLds L;
+  __shared__ TrussLds<STAGED ? TO_STAGED : TO_ENTRIES, STAGED ? TRUSS_WG_VALUES + 2 : 2> L;
   const int t = threadIdx.x;
   const uint2 rg = A.ranges[blockIdx.x];
   const uint32_t a0 = rg.x, na = rg.y;
@@ -425,28 +433,50 @@ __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
     if (TWO && t + BO_THREADS < ne) put_entry(L, t + BO_THREADS, E1);
   }
   __syncthreads();
-  double* __restrict__ val = A.val + base;
-  for (int k = t; k < 3 * ne; k += BO_THREADS) {
-    const int i = k / ne, sl = k - i * ne;
-    const double* o = L.data[sl];
-    const double s = o[i] * o[4];
-    double nb[3];
+  auto rows = [&](double* __restrict__ val) {
+    for (int k = t; k < 3 * ne; k += BO_THREADS) {
+      const int i = k / ne, sl = k - i * ne;
+      const double* o = L.data[sl];
+      const double s = o[i] * o[4];
+      double nb[3];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) nb[q] = s * o[q];
-    write_row3(val, L.block[sl], i, L.row[L.node[sl]][i], nb);
-  }
-  const int j = t / 3, i = t % 3;
-  if (j >= int(na)) return;
-  const int s0 = int(L.first[j]), s1 = int(L.first[j + 1]);
-  if (s1 == s0) return;
-  double acc[3];
-  for (int sl = s0; sl < s1; ++sl) {
-    const double* o = L.data[sl];
-    const double s = o[i] * o[3];
+      for (int q = 0; q < 3; ++q) nb[q] = s * o[q];
+      write_row3(val, L.block[sl], i, L.row[L.node[sl]][i], nb);
+    }
+    const int j = t / 3, i = t % 3;
+    if (j >= int(na)) return;
+    const int s0 = int(L.first[j]), s1 = int(L.first[j + 1]);
+    if (s1 == s0) return;
+    double acc[3];
+    for (int sl = s0; sl < s1; ++sl) {
+      const double* o = L.data[sl];
+      const double s = o[i] * o[3];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) acc[q] = sl == s0 ? s * o[q] : acc[q] + s * o[q];
+      for (int q = 0; q < 3; ++q) acc[q] = sl == s0 ? s * o[q] : acc[q] + s * o[q];
+    }
+    write_row3(val, A.self[a0 + j], i, L.row[j][i], acc);
+  };
+  double* __restrict__ dst = A.val + base;
+  if (!STAGED) {
+    rows(dst);
+    return;
   }
-  write_row3(val, A.self[a0 + j], i, L.row[j][i], acc);
+  // staged from the parity of the CSR position: pairs of values leave as aligned
+  // 16-byte chunks, the odd values at either end alone
+  const int nv = int(A.row_ptr[6 * size_t(a0 + na)] - base);  // <= TRUSS_WG_VALUES (cut on the host)
+  const int head = int(base & 1), npair = (nv - head) >> 1;
+  double* const out = L.out + head;
+  rows(out);
+  __syncthreads();
+  for (int k = t; k < npair; k += BO_THREADS) {
+    const int o = head + 2 * k;
+    bo_d2 v;
+    v.x = out[o];
+    v.y = out[o + 1];
+    *reinterpret_cast<bo_d2*>(dst + o) = v;
+  }
+  if (t == 0 && head && nv > 0) dst[0] = out[0];
+  if (t == BO_THREADS - 1 && nv > head && ((nv - head) & 1)) dst[nv - 1] = out[nv - 1];
 }
 
 }  // namespace
@@ -505,6 +535,7 @@ std::string upload_bar_maps(Device* d, const BarMaps& bm) {
   d->bo_n_ranges = bm.n_bar_ranges;
   d->bo_n_truss_ranges = bm.ranges.size() / 2 - bm.n_bar_ranges;
   d->bo_truss_entries = 0;
+  d->to_staged = bm.truss_staged;
   for (size_t r = bm.n_bar_ranges; r < bm.ranges.size() / 2; ++r)
     d->bo_truss_entries = std::max(d->bo_truss_entries, int(bm.inc_ptr[bm.ranges[2 * r] + bm.ranges[2 * r + 1]] -
                                                             bm.inc_ptr[bm.ranges[2 * r]]));
@@ -558,7 +589,9 @@ std::string assemble_bar_owner(Device* d, double* val, void* stream, bool timed)
       A.entry = d->to_entry;
       A.entry_rec = d->to_entry_rec;
       A.entry_ptr = d->to_entry_ptr;
-      auto kernel = d->bo_truss_entries > BO_THREADS ? truss_owner_kernel<true> : truss_owner_kernel<false>;
+      auto kernel = d->to_staged                      ? truss_owner_kernel<false, true>
+                    : d->bo_truss_entries > BO_THREADS ? truss_owner_kernel<true, false>
+                                                       : truss_owner_kernel<false, false>;
       kernel<<<unsigned(d->bo_n_truss_ranges), BO_THREADS, 0, s>>>(A);
       HIP_TRY(hipGetLastError());
     }

@@ -65,6 +65,7 @@ struct Device {
   uint32_t *bo_inc_ptr = nullptr, *bo_inc = nullptr, *bo_ranges = nullptr;
   size_t bo_n_ranges = 0, bo_n_truss_ranges = 0;  // bar-kernel ranges, then truss-kernel ranges
   int bo_truss_entries = 0;    // most entries of a truss-kernel range
+  bool to_staged = false;      // truss ranges cut for the kernel that stages its rows
   uint32_t *bo_rec_elem = nullptr, *bo_entry_rec = nullptr, *bo_entry_ptr = nullptr;
   double* bo_rec = nullptr;    // element constants of the bar-kernel ranges
   uint4 *bo_entry = nullptr, *bo_self = nullptr;  // masks and row offsets: off-diagonal per entry, diagonal per node

@@ -190,7 +190,8 @@ struct BarMaps {
   std::vector<uint32_t> inc;      // per node, insertion order: type << 31 | element << 1 | p
   // per workgroup: first node, node count.  The first n_bar_ranges go to the
   // bar kernel (<= 40 nodes, <= 256 entries, <= 5120 values), the rest, whose
-  // nodes touch trusses only, to the truss kernel (<= 85 nodes, <= 512 entries)
+  // nodes touch trusses only, to the truss kernel (<= 85 nodes, <= 512 entries, or
+  // where its rows are staged <= 256 entries and <= 2560 values)
   std::vector<uint32_t> ranges;
   size_t n_bar_ranges = 0;
   // bar kernel: element records, in the order in which the ranges first meet
@@ -198,9 +199,11 @@ struct BarMaps {
   // (type << 31 | record << 1 | p); range r owns entries entry_ptr[r] ..
   std::vector<uint32_t> rec_elem, entry_rec, entry_ptr;
   std::vector<uint32_t> truss_elem, truss_entry, truss_ptr;  // the truss kernel's, the same way
+  bool truss_staged = false;  // its ranges hold at most TRUSS_WG_STAGED entries and TRUSS_WG_VALUES values
 };
 constexpr int BAR_WG_NODES = 40, BAR_WG_ENTRIES = 256, BAR_WG_VALUES = 5120;
 constexpr int TRUSS_WG_NODES = 85, TRUSS_WG_ENTRIES = 512;
+constexpr int TRUSS_WG_STAGED = 256, TRUSS_WG_VALUES = 2560, TRUSS_STAGED_RANGES = 1024;  // with rows staged in LDS
 std::string upload_bar_maps(Device* d, const BarMaps& bm);
 std::string assemble_bar_owner(Device* d, double* val, void* stream, bool timed = true);
 

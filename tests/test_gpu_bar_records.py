@@ -41,7 +41,7 @@ def _chain(n, seed, along_axes, trusses):
     return xyz, conn.astype(np.uint32) + 1, props, (braces.astype(np.uint32) + 1 if trusses else None)
 
 
-@pytest.mark.parametrize("kind,size", [("truss", (2,)), ("truss", (3,)), ("truss", (12,)), ("truss", (13,)),
+@pytest.mark.parametrize("kind,size", [("truss", (2,)), ("truss", (3,)), ("truss", (12,)), ("truss", (13,)), ("truss", (28,)),
                                        ("beam", (3, 3, 1)), ("beam", (10, 10, 10)), ("beam", (11, 10, 10))])
 def test_small_lattices_match_oracle(gpu, kind, size):
     """Ranges of a small mesh: the least nodes per range and one more range, and
