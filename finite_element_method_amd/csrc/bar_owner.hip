@@ -86,7 +86,7 @@ static_assert(BO_NODES == BAR_WG_NODES && BO_ENTRIES == BAR_WG_ENTRIES && BO_VAL
 // the layout is compact and a range holds up to twice the entries.
 template <int ENTRIES, int VALUES>
 struct TrussLds {
-  double out[VALUES];          // the owned rows, one place in where their CSR position is odd
+  double out[VALUES];          // the owned rows, one place in where their address is odd
   double data[ENTRIES][5];     // r (3), kpp, kpq
   uint4 block[ENTRIES];        // the entry's off-diagonal block
   uint8_t node[ENTRIES];       // owned node of the entry
@@ -461,10 +461,11 @@ __global__ __launch_bounds__(BO_THREADS) void truss_owner_kernel(BarArgs A) {
     rows(dst);
     return;
   }
-  // staged from the parity of the CSR position: pairs of values leave as aligned
-  // 16-byte chunks, the odd values at either end alone
+  // staged from the parity of the address: pairs of values leave as aligned
+  // 16-byte chunks wherever the caller's array starts, the odd values at either
+  // end alone
   const int nv = int(A.row_ptr[6 * size_t(a0 + na)] - base);  // <= TRUSS_WG_VALUES (cut on the host)
-  const int head = int(base & 1), npair = (nv - head) >> 1;
+  const int head = int((reinterpret_cast<uintptr_t>(dst) >> 3) & 1), npair = (nv - head) >> 1;
   double* const out = L.out + head;
   rows(out);
   __syncthreads();

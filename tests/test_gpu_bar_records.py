@@ -54,6 +54,21 @@ def test_small_lattices_match_oracle(gpu, kind, size):
     assert m.assembly_path() == "bar_owner" and r["pattern_equal"] and r["max_ratio"] <= 1.0, r
 
 
+@pytest.mark.parametrize("n", [2, 3, 12, 28])
+def test_trusses_into_an_array_at_any_place(gpu, n):
+    """The caller's values may start at an odd multiple of 8 bytes; nothing beside them is written."""
+    m = FEM.from_mesh(meshgen.truss_lattice(n, seed=n))
+    want = m.stiffness_csr()[2]
+    print("case", n, len(want), flush=True)
+    for first in (0, 1):
+        room = torch.full((len(want) + 3,), 7.0, dtype=torch.float64, device="cuda")
+        m.assemble_into(room[first:first + len(want)])
+        torch.cuda.synchronize()
+        got = room.cpu().numpy()
+        assert np.array_equal(got[first:first + len(want)].view(np.uint64), want.view(np.uint64))
+        assert np.all(got[:first] == 7.0) and np.all(got[first + len(want):] == 7.0)
+
+
 def _load(model, xyz, conn, props, braces):
     n, ne = len(xyz), len(conn)
     model.add_nodes(np.arange(1, n + 1, dtype=np.uint32), xyz)
