@@ -120,27 +120,29 @@ __host__ __device__ inline void plate_frame_adjoint(const double o[13], double d
 }
 
 // dL/d(E, nu, t, k) from the constitutive partials: cm = E t/(1-nu^2),
-// cb = E t^3/(12 (1-nu^2)), cs = E t k/(2 (1+nu)).  The constants' reciprocals
-// come from two divisions.
+// cb = E t^3/(12 (1-nu^2)), cs = E t k/(2 (1+nu)).  The derivatives by E, t and k are
+// the products of the other factors: no parameter divides, so that a zero one
+// (the modulus or thickness of a void) leaves every derivative finite.
 __host__ __device__ inline void plate_adjoint_params(const double P[7], double E, double nu, double t, double k,
                                                      double grad_param[4]) {
   const double inv_n = 1.0 / ((1.0 - nu) * (1.0 + nu));  // 1 / (1 - nu^2)
-  const double inv_etk = 1.0 / ((E * t) * k);
   const double cm = E * t * inv_n;
   const double cb = E * (t * t * t) * (1.0 / 12.0) * inv_n;
   const double inv_1pn = (1.0 - nu) * inv_n;  // 1 / (1 + nu)
   const double cs = E * t * k * 0.5 * inv_1pn;
   const double h = (1.0 - nu) / 2.0;
-  const double Lm = cm * ((P[0] + nu * P[1]) + h * P[2]);
-  const double Lb = cb * ((P[3] + nu * P[4]) + h * P[5]);
-  const double Ls = cs * P[6];
+  // membrane, bending and shear per unit of E t, E t^3 and E t k
+  const double Lm = ((P[0] + nu * P[1]) + h * P[2]) * inv_n;
+  const double Lb = ((P[3] + nu * P[4]) + h * P[5]) * ((1.0 / 12.0) * inv_n);
+  const double Ls = P[6] * (0.5 * inv_1pn);
+  const double tb = t * t * Lb, ks = k * Ls;
   const double dcm = cm * 2.0 * nu * inv_n, dcb = cb * 2.0 * nu * inv_n;
-  grad_param[0] = ((Lm + Lb) + Ls) * (t * k * inv_etk);
+  grad_param[0] = t * ((Lm + tb) + ks);
   grad_param[1] = (((P[0] * dcm + P[1] * (cm + nu * dcm)) + P[2] * (h * dcm - 0.5 * cm)) +
                    ((P[3] * dcb + P[4] * (cb + nu * dcb)) + P[5] * (h * dcb - 0.5 * cb))) -
                   P[6] * cs * inv_1pn;
-  grad_param[2] = ((Lm + 3.0 * Lb) + Ls) * (E * k * inv_etk);
-  grad_param[3] = Ls * (E * t * inv_etk);
+  grad_param[2] = E * ((Lm + 3.0 * tb) + ks);
+  grad_param[3] = E * t * Ls;
 }
 
 // Element-level finish from the four lanes' sums.
