@@ -510,8 +510,10 @@ BarArgs bar_args(Device* d, double* val) {
   return A;
 }
 
-// (re)forms the bar kernel's element records from the current coordinates,
-// frames and parameters
+}  // namespace
+
+// (re)forms the element records from the current coordinates, frames and
+// parameters
 std::string fill_bar_records(Device* d, hipStream_t s) {
   if (d->bo_n_recs + d->to_n_recs) {
     BarArgs A = bar_args(d, nullptr);
@@ -519,11 +521,8 @@ std::string fill_bar_records(Device* d, hipStream_t s) {
         A, d->bo_rec_elem, d->bo_n_recs, d->bo_rec, d->to_rec_elem, d->to_n_recs, d->to_rec);
     HIP_TRY(hipGetLastError());
   }
-  d->bo_rec_dirty = false;
   return "";
 }
-
-}  // namespace
 
 std::string upload_bar_maps(Device* d, const BarMaps& bm) {
   std::string e;
@@ -567,16 +566,13 @@ std::string upload_bar_maps(Device* d, const BarMaps& bm) {
   }
   e = fill_bar_records(d, nullptr);
   if (!e.empty()) return e;
+  d->kept = Kept::BAR_RECORDS;
   HIP_TRY(hipDeviceSynchronize());
   return "";
 }
 
 std::string assemble_bar_owner(Device* d, double* val, void* stream, bool timed) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (d->bo_rec_dirty) {  // coordinates or parameters changed since the records were formed
-    auto e = fill_bar_records(d, s);
-    if (!e.empty()) return e;
-  }
   if (timed) HIP_TRY(hipEventRecord(d->ev0, s));
   if (d->bo_n_ranges + d->bo_n_truss_ranges) {
     BarArgs A = bar_args(d, val);

@@ -9,6 +9,10 @@ namespace femdev {
 
 struct UpdateReport;
 
+// what the value path of the current pattern keeps of coordinates, frames and
+// parameters in a form of its own: formed with its maps and by every update
+enum class Kept { NONE, PLATE_SLOTS, FRAME_SLOTS, BAR_RECORDS };
+
 struct Device {
   hipStream_t stream = nullptr;
   int dev = 0;
@@ -26,6 +30,7 @@ struct Device {
   int32_t* col_idx = nullptr;
   double* val = nullptr;
   int64_t n_rows = 0, nnz = 0;
+  Kept kept = Kept::NONE;
   // generic maps
   uint64_t* class_mask = nullptr;
   uint32_t* class_off = nullptr;
@@ -47,7 +52,6 @@ struct Device {
   int pl_waves = 0;
   uint32_t *pl_nodes = nullptr, *pl_lanes = nullptr, *pl_lane_set = nullptr;
   double* pl_geo = nullptr;   // per wave element slot: local coordinates and parameters
-  bool pl_geo_dirty = false;  // node coordinates or plate parameters changed since pl_geo was filled
   // every plate has the same E, nu and k (bitwise): the slots hold t only and
   // the three values go to the kernel as arguments
   bool pl_uniform = false;
@@ -57,7 +61,6 @@ struct Device {
   int pn_waves = 0;
   uint32_t *pn_eid = nullptr, *pn_nodes = nullptr, *pn_wave = nullptr, *pn_lanes = nullptr;
   double* pn_geo = nullptr;   // per wave element slot: local coordinates, parameters, frame
-  bool pn_geo_dirty = false;  // coordinates, frames or parameters changed since pn_geo was filled
   // bar owner maps
   uint32_t* bo_bid[2] = {nullptr, nullptr};
   uint64_t* bo_bmask = nullptr;
@@ -74,7 +77,6 @@ struct Device {
   double* to_rec = nullptr;
   uint4* to_entry = nullptr;
   size_t to_n_recs = 0;
-  bool bo_rec_dirty = false;   // coordinates or bar parameters changed since bo_rec was filled
   // adjoint maps
   uint32_t* adj_bid[3] = {nullptr, nullptr, nullptr};
   uint64_t* adj_bmask = nullptr;
@@ -139,6 +141,11 @@ struct Device {
     hipError_t _e = (expr);                                                           \
     if (_e != hipSuccess) return std::string(#expr) + ": " + hipGetErrorString(_e);  \
   } while (0)
+
+// form what the path keeps (Kept) from the current coordinates, frames and parameters
+std::string plate_lanes_gather(Device* d, hipStream_t s);   // plate_lanes.hip
+std::string plate_frames_gather(Device* d, hipStream_t s);  // plate_frames.hip
+std::string fill_bar_records(Device* d, hipStream_t s);     // bar_owner.hip
 
 template <class T>
 inline std::string dalloc(T*& p, size_t n) {

@@ -126,9 +126,9 @@ struct PlateLaneMaps {
   std::vector<uint32_t> lane_set;  // per wave: its set in `lanes`
 };
 std::string upload_plate_lane_maps(Device* d, const PlateLaneMaps& pm);
-// E, nu and k shared by every plate (uniform) or per element: sets the slot
-// layout (8 or 10 doubles) and marks the slots for refilling
-std::string set_plate_lane_material(Device* d, bool uniform, const double mat[3]);
+// E, nu and k shared by every plate (uniform) or per element: the slot layout (8
+// or 10 doubles) that the next filling of the slots takes
+void set_plate_lane_material(Device* d, bool uniform, const double mat[3]);
 std::string assemble_plate_lanes(Device* d, double* val, void* stream, bool timed = true);
 
 // Plates with frames of their own (plate_frames.hip): meshes of plates only in

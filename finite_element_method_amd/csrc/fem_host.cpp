@@ -1285,8 +1285,7 @@ std::string build_pattern(fem_model* m) {
       femdev::PlateLaneMaps plm;
       if (m->pf_kernel == 3 && build_plate_lane_maps(m, bptr, blocks, row_ptr, plm)) {
         double mat[3];
-        e = femdev::set_plate_lane_material(m->dev, plate_material_uniform(m, mat), mat);
-        if (!e.empty()) return e;
+        femdev::set_plate_lane_material(m->dev, plate_material_uniform(m, mat), mat);
         e = femdev::upload_plate_lane_maps(m->dev, plm);
         if (!e.empty()) return e;
         m->path = "plate_lanes";
@@ -2444,11 +2443,6 @@ int fem_update_params(fem_model* m, int type, const double* params_device, void*
   m->params_behind[type] = m->set[type].size() != 0;
   auto e = femdev::update_params(m->dev, type, params_device, stream, rep);
   if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
-  if (type == PLATE && m->path == "plate_lanes") {  // the slot layout follows the new parameters
-    const double mat[3] = {rep.plate[0], rep.plate[1], rep.plate[3]};
-    e = femdev::set_plate_lane_material(m->dev, !rep.mixed, mat);
-    if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
-  }
   return apply_report(m, rep);
 }
 

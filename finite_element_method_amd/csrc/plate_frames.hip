@@ -310,6 +310,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
   }
 }
 
+}  // namespace
+
 std::string plate_frames_gather(Device* d, hipStream_t s) {
   const size_t n_slots = size_t(d->pn_waves) * PN_ELEMS;
   if (n_slots) {
@@ -317,11 +319,8 @@ std::string plate_frames_gather(Device* d, hipStream_t s) {
                                                                              d->R[PLATE], d->pn_eid, n_slots, d->pn_geo);
     HIP_TRY(hipGetLastError());
   }
-  d->pn_geo_dirty = false;
   return "";
 }
-
-}  // namespace
 
 std::string upload_plate_frame_maps(Device* d, const PlateFrameMaps& pm) {
   d->pn_waves = 0;
@@ -333,16 +332,13 @@ std::string upload_plate_frame_maps(Device* d, const PlateFrameMaps& pm) {
   if (!(e = dalloc(d->pn_geo, size_t(pm.n_waves) * PN_ELEMS * PN_GEO)).empty()) return e;
   d->pn_waves = pm.n_waves;
   if (!(e = plate_frames_gather(d, nullptr)).empty()) return e;
+  d->kept = Kept::FRAME_SLOTS;
   HIP_TRY(hipDeviceSynchronize());
   return "";
 }
 
 std::string assemble_plate_frames(Device* d, double* val, void* stream, bool timed) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (d->pn_geo_dirty) {  // coordinates or parameters changed since the slots were filled
-    auto e = plate_frames_gather(d, s);
-    if (!e.empty()) return e;
-  }
   if (timed) HIP_TRY(hipEventRecord(d->ev0, s));
   FrameArgs a;
   a.geo = d->pn_geo;

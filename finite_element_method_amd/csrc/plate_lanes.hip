@@ -377,6 +377,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void pl
   }
 }
 
+}  // namespace
+
 std::string plate_lanes_gather(Device* d, hipStream_t s) {
   const size_t n_slots = size_t(d->pl_waves) * PL_ELEMS;
   if (n_slots) {
@@ -385,11 +387,8 @@ std::string plate_lanes_gather(Device* d, hipStream_t s) {
                                                                             d->pl_uniform ? PL_GEO_U : PL_GEO, d->pl_geo);
     HIP_TRY(hipGetLastError());
   }
-  d->pl_geo_dirty = false;
   return "";
 }
-
-}  // namespace
 
 std::string upload_plate_lane_maps(Device* d, const PlateLaneMaps& pm) {
   d->pl_waves = pm.n_waves;
@@ -402,23 +401,18 @@ std::string upload_plate_lane_maps(Device* d, const PlateLaneMaps& pm) {
   if (!(e = dalloc(d->pl_geo, size_t(pm.n_waves) * PL_ELEMS * PL_GEO)).empty()) return e;  // either layout fits
   e = plate_lanes_gather(d, nullptr);
   if (!e.empty()) return e;
+  d->kept = Kept::PLATE_SLOTS;
   HIP_TRY(hipDeviceSynchronize());
   return "";
 }
 
-std::string set_plate_lane_material(Device* d, bool uniform, const double mat[3]) {
+void set_plate_lane_material(Device* d, bool uniform, const double mat[3]) {
   d->pl_uniform = uniform;
   for (int k = 0; k < 3; ++k) d->pl_mat[k] = uniform ? mat[k] : 0.0;
-  d->pl_geo_dirty = true;
-  return "";
 }
 
 std::string assemble_plate_lanes(Device* d, double* val, void* stream, bool timed) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (d->pl_geo_dirty) {  // coordinates or parameters changed since the slots were filled
-    auto e = plate_lanes_gather(d, s);
-    if (!e.empty()) return e;
-  }
   if (timed) HIP_TRY(hipEventRecord(d->ev0, s));
   if (d->pl_waves > 0) {
     LaneArgs a;

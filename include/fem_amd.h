@@ -172,7 +172,12 @@ double fem_last_backward_ms(fem_model* m);
 /* Replace one element type's parameters (device memory, same layout as the
  * fem_add_* props) or all node coordinates (device memory, N x 3).  Values are
  * not re-validated.  Frames are recomputed; if a frame's zero pattern changes
- * the sparsity pattern is rebuilt by the next assembly. */
+ * the sparsity pattern is rebuilt by the next assembly.  The update has finished
+ * when the call returns: calls on any stream then read the new values, and so do
+ * replays of captured ones while the pattern stays.  Exception: a captured
+ * assembly of flat plates ("plate_lanes") with E, nu and k the same for every
+ * plate holds these three as launch arguments; capture it again when an update
+ * changes them or makes them differ. */
 int fem_update_params(fem_model* m, int type, const double* params_device, void* stream);
 int fem_update_nodes(fem_model* m, const double* xyz_device, void* stream);
 

@@ -1,0 +1,144 @@
+"""fem_update_* against work on several streams and in captured graphs, for every
+value path: assemblies on two streams after an update, a captured assembly
+replayed after updates, a capture as the first call after an update."""
+
+import numpy as np
+import pytest
+
+from finite_element_method_amd import BEAM, FEM, PLATE, TRUSS, meshgen
+from tests.test_gpu_bar_records import _chain, _load
+from tests.test_gpu_plate_frames import _turn, _vault
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def _cuda(a):
+    return torch.tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda")
+
+
+class _Meshed:
+    """A mesh of one element type; variant k has other sizes and coordinates."""
+
+    def __init__(self, mesh, etype, column, one_material=False):
+        self.mesh, self.etype, self.column = mesh, etype, column
+        if one_material:
+            mesh.props[:, [0, 1, 3]] = mesh.props[0, [0, 1, 3]]
+
+    def data(self, k):
+        m = self.mesh
+        props = m.props.copy()
+        props[:, self.column] *= np.random.default_rng(k).uniform(0.7, 1.4, len(props))
+        return m.xyz * (1.0 + 0.25 * k), {self.etype: props}
+
+    def model(self, k):
+        m, (xyz, props) = self.mesh, self.data(k)
+        return FEM.from_mesh(meshgen.Mesh(m.kind, m.node_numbers, xyz, m.numbers, m.conn, props[self.etype]))
+
+
+class _Braced:
+    """A chain of beams braced by trusses."""
+
+    def __init__(self, n):
+        self.chain = _chain(n, n, False, True)
+
+    def data(self, k):
+        xyz, conn, props, braces = self.chain
+        props = props.copy()
+        props[:, 2] *= np.random.default_rng(k).uniform(0.7, 1.4, len(props))
+        return xyz * (1.0 + 0.25 * k), {BEAM: props}
+
+    def model(self, k):
+        xyz, conn, props, braces = self.chain
+        x, p = self.data(k)
+        return _load(FEM.create(1e-4, 1e-12, len(xyz)), x, conn, p[BEAM], braces)
+
+
+CASES = {
+    "lattice": lambda: _Meshed(meshgen.truss_lattice(9, seed=1), TRUSS, 1),
+    "frame": lambda: _Meshed(meshgen.beam_frame(6, 7, 5, seed=2), BEAM, 2),
+    "braced_chain": lambda: _Braced(90),
+    "shell": lambda: _Meshed(_vault(19, 14, 3, _turn()), PLATE, 2),
+    "plate": lambda: _Meshed(meshgen.plate_grid(23, 17, seed=4), PLATE, 2),
+    "plate_materials": lambda: _Meshed(_materials(meshgen.plate_grid(23, 17, seed=5)), PLATE, 2),
+}
+
+
+class _Mixing(_Meshed):
+    """Plates of one material in even variants, of several in odd ones."""
+
+    def data(self, k):
+        xyz, props = super().data(k)
+        if k % 2:
+            props[PLATE][3::5, 0] *= 1.5
+        return xyz, props
+
+
+def _materials(mesh):
+    mesh.props[:, 0] *= np.random.default_rng(6).uniform(0.5, 2.0, mesh.n_elements)
+    return mesh
+
+
+def _update(m, case, k, stream=None):
+    xyz, props = case.data(k)
+    for t, p in props.items():
+        m.update_params(t, _cuda(p), stream=stream)
+    m.update_nodes(_cuda(xyz), stream=stream)
+
+
+def _want(case, k):
+    return torch.tensor(case.model(k).stiffness_csr()[2], device="cuda")
+
+
+def _same(a, b):
+    return torch.equal(a.view(torch.int64), b.view(torch.int64))
+
+
+@pytest.mark.parametrize("name", sorted(CASES) + ["plate_mixing"])
+def test_two_streams_after_an_update(gpu, name):
+    """The update has finished when it returns: assemblies on any stream see it."""
+    case = CASES[name]() if name in CASES else _Mixing(meshgen.plate_grid(23, 17, seed=7), PLATE, 2)
+    print("case", name, flush=True)
+    m = case.model(0)
+    m.stiffness_csr()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    out = [torch.empty(m.csr_info()[1], dtype=torch.float64, device="cuda") for _ in streams]
+    torch.cuda.synchronize()
+    for k in (1, 2, 3):
+        _update(m, case, k, stream=streams[k % 3])
+        for s, o in zip(streams, out):
+            m.assemble_into(o, stream=s)
+        torch.cuda.synchronize()
+        want = _want(case, k)
+        assert all(_same(o, want) for o in out), k
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_captured_assembly_after_updates(gpu, name):
+    """A captured assembly replays with the values of the last update (E, nu and k
+    of flat plates apart, which stay here as they were); a capture as the first
+    call after an update leaves the eager calls as they are."""
+    case = CASES[name]()
+    print("case", name, flush=True)
+    m = case.model(0)
+    m.stiffness_csr()
+    m.set_option("time_assembly", 0)
+    eager, out = (torch.zeros(m.csr_info()[1], dtype=torch.float64, device="cuda") for _ in range(2))
+    _update(m, case, 1)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        m.assemble_into(out, stream=torch.cuda.current_stream())
+    m.assemble_into(eager)
+    torch.cuda.synchronize()
+    assert _same(eager, _want(case, 1))
+    for k in (1, 2, 3, 4):
+        _update(m, case, k)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = _want(case, k)
+        assert _same(out, want), k
+        m.assemble_into(eager)
+        torch.cuda.synchronize()
+        assert _same(eager, want), k
