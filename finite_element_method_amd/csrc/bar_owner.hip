@@ -353,9 +353,10 @@ __global__ __launch_bounds__(BO_THREADS) void bar_owner_kernel(BarArgs A) {
   }
   __syncthreads();
   double* __restrict__ dst = A.val + base;
-  // 16-byte stores from the first even CSR position, non-temporal (nothing in
-  // this kernel reads the values again); the odd values at either end alone
-  const int head = int(base & 1), npair = (nv - head) >> 1;
+  // 16-byte stores from the first aligned address wherever the caller's array
+  // starts, non-temporal (nothing in this kernel reads the values again); the odd
+  // values at either end alone
+  const int head = int((reinterpret_cast<uintptr_t>(dst) >> 3) & 1), npair = (nv - head) >> 1;
   for (int k = t; k < npair; k += BO_THREADS) {
     const int o = head + 2 * k;
     bo_d2 v;
