@@ -536,6 +536,15 @@ class FEM:
     def last_backward_ms(self):
         return lib().fem_last_backward_ms(self._h)
 
+    @staticmethod
+    def _update_stream(stream, values):
+        """An update without a stream runs on torch's current one, where its values were made."""
+        if stream is None:
+            import torch
+
+            stream = torch.cuda.current_stream(values.device)
+        return _stream_handle(stream)
+
     def update_params(self, etype, params, stream=None):
         """Replaces one element type's parameters (float64 CUDA tensor, add_* layout)."""
         params = params.detach().contiguous()
@@ -543,7 +552,7 @@ class FEM:
         if params.numel() != n * PARAMS_PER[etype] or not params.is_cuda or params.dtype.itemsize != 8:
             raise ValueError("expected a float64 CUDA tensor of %d x %d" % (n, PARAMS_PER[etype]))
         self._call(lib().fem_update_params(self._h, int(etype), ctypes.c_void_p(params.data_ptr()),
-                                           _stream_handle(stream)))
+                                           self._update_stream(stream, params)))
         self._version = getattr(self, "_version", 0) + 1
 
     def update_nodes(self, xyz, stream=None):
@@ -552,7 +561,7 @@ class FEM:
         n = self.model_size()[0]
         if xyz.numel() != 3 * n or not xyz.is_cuda or xyz.dtype.itemsize != 8:
             raise ValueError("expected a float64 CUDA tensor of %d x 3" % n)
-        self._call(lib().fem_update_nodes(self._h, ctypes.c_void_p(xyz.data_ptr()), _stream_handle(stream)))
+        self._call(lib().fem_update_nodes(self._h, ctypes.c_void_p(xyz.data_ptr()), self._update_stream(stream, xyz)))
         self._version = getattr(self, "_version", 0) + 1
 
     # ----------------------------------------------------------- convenience

@@ -126,6 +126,12 @@ struct Device {
   double sol_ms = 0.0;
   double* u_glob = nullptr;  // global displacements of the last solve (6 per node)
   size_t ucap = 0;
+  // streams that were given work since the last update that reads what an update
+  // rewrites (note_use; of more than two, two say enough); captured: such work is
+  // in a graph, whose replays may run on any stream
+  hipStream_t used[2] = {nullptr, nullptr};
+  int n_used = 0;
+  bool captured = false;
   // updates in place (fem_device.hip): report words, their copy in pinned host
   // memory, and the number of the last update
   uint32_t* upd_words = nullptr;

@@ -214,8 +214,12 @@ std::string run_setup(Device* d, int type, size_t n, double rel_tol, double abs_
 // them and what the value path keeps, and reports to the host in a few words; the
 // host's own copies stay behind and are fetched when the host reads them
 // (fetch_nodes, fetch_params).  When it returns, all of that is written: later
-// calls on any stream, and replays of captured ones, read the new values.  It waits
-// for the device first: work in flight on any stream may read what it rewrites.
+// calls on any stream, and replays of captured ones, read the new values.
+// Work of this model may be in flight and read what the update rewrites.  On the
+// update's own stream it comes first anyway; only where the model was used on
+// another stream since the last update, or captured into a graph, does the update
+// wait for the device, so that models on streams of their own do not wait for each
+// other.
 // Frame codes are compared on the device.  New coordinates and parameters,
 // assembly and backward of a 257 x 191 plate: 4.3 -> 0.21 ms; copying both
 // arrays to the host, rebuilding its table of coordinates and comparing the
@@ -248,16 +252,20 @@ __global__ void report_kernel(const uint32_t* __restrict__ words, const double* 
 
 namespace {
 
-std::string begin_update(Device* d) {
+std::string begin_update(Device* d, hipStream_t s) {
   if (!d->upd_words) {
     auto e = dalloc(d->upd_words, size_t(UPD_WORDS));
     if (!e.empty()) return e;
     const uint32_t zero[UPD_WORDS] = {};
     HIP_TRY(hipMemcpy(d->upd_words, zero, sizeof(zero), hipMemcpyHostToDevice));
+    HIP_TRY(hipStreamSynchronize(nullptr));
   }
   if (!d->upd_report) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&d->upd_report), sizeof(UpdateReport)));
   d->upd_number = d->upd_number + 1 ? d->upd_number + 1 : 1;
-  HIP_TRY(hipDeviceSynchronize());
+  bool elsewhere = d->captured;
+  // hipStreamPerThread is another stream in each thread
+  for (int k = 0; k < d->n_used; ++k) elsewhere = elsewhere || d->used[k] != s || s == hipStreamPerThread;
+  if (elsewhere) HIP_TRY(hipDeviceSynchronize());
   return "";
 }
 
@@ -265,6 +273,7 @@ std::string end_update(Device* d, hipStream_t s, UpdateReport& out) {
   report_kernel<<<1, 64, 0, s>>>(d->upd_words, d->n_elem[PLATE] ? d->params[PLATE] : nullptr, d->upd_report, d->upd_number);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(s));
+  d->n_used = 0;
   out = *d->upd_report;
   return "";
 }
@@ -283,12 +292,24 @@ std::string refresh_kept(Device* d, hipStream_t s) {
 
 }  // namespace
 
+void note_use(Device* d, void* stream) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (s && hipStreamIsCapturing(s, &status) == hipSuccess && status != hipStreamCaptureStatusNone) {
+    d->captured = true;
+    return;
+  }
+  for (int k = 0; k < d->n_used; ++k)
+    if (d->used[k] == s) return;
+  if (d->n_used < 2) d->used[d->n_used++] = s;
+}
+
 std::string update_params(Device* d, int type, const double* src, void* stream, UpdateReport& out) {
   out = UpdateReport();
   const size_t n = d->n_elem[type];
   if (!n) return "";
   hipStream_t s = static_cast<hipStream_t>(stream);
-  auto e = begin_update(d);
+  auto e = begin_update(d, s);
   if (!e.empty()) return e;
   const size_t count = n * PARAMS_PER[type];
   if (type == PLATE) {
@@ -317,7 +338,7 @@ std::string update_nodes(Device* d, const double* src, void* stream, UpdateRepor
   const size_t n = 3 * d->n_nodes;
   if (!n) return "";
   hipStream_t s = static_cast<hipStream_t>(stream);
-  auto e = begin_update(d);
+  auto e = begin_update(d, s);
   if (!e.empty()) return e;
   copy_kernel<<<blocks_of(n), 256, 0, s>>>(src, n, d->xyz);
   HIP_TRY(hipGetLastError());

@@ -281,6 +281,9 @@ struct UpdateReport {
   uint32_t mixed = 0;
   double plate[4] = {0.0, 0.0, 0.0, 0.0};  // the first plate's parameters
 };
+// note_use: `stream` is given work that reads coordinates, parameters, frames or
+// what the value path keeps of them; updates wait for such work.
+void note_use(Device* d, void* stream);
 std::string update_params(Device* d, int type, const double* src, void* stream, UpdateReport& out);
 std::string update_nodes(Device* d, const double* src, void* stream, UpdateReport& out);
 std::string fetch_nodes(Device* d, double* host);

@@ -1668,8 +1668,9 @@ int ensure_adjoint(fem_model* m) {
   return FEM_OK;
 }
 
+// on `stream`, for a call on the caller's stream `called`
 int run_backward(fem_model* m, int mode, const double* g, double* dp_truss, double* dp_beam, double* dp_plate,
-                 double* dxyz, void* stream) {
+                 double* dxyz, void* stream, void* called) {
   if (!m) return FEM_ERR_ARGUMENT;
   if (!g) return fail(m, FEM_ERR_ARGUMENT, mode == 0 ? "dL/dK values are required" : "displacements are required");
   if (dxyz && m->set[BEAM].size())
@@ -1679,6 +1680,7 @@ int run_backward(fem_model* m, int mode, const double* g, double* dp_truss, doub
   int rc = ensure_adjoint(m);
   if (rc) return rc;
   double* dp[3] = {dp_truss, dp_beam, dp_plate};
+  femdev::note_use(m->dev, called);
   auto e = femdev::run_adjoint(m->dev, mode, g, dp, dxyz, stream, m->wide_loads);
   return e.empty() ? FEM_OK : fail(m, FEM_ERR_DEVICE, e);
 }
@@ -2347,6 +2349,7 @@ int fem_assemble_into(fem_model* m, double* val_device, void* stream) {
   int rc = ensure_ready(m);
   if (rc) return rc;
   const bool t = m->time_assembly;
+  femdev::note_use(m->dev, stream);
   std::string e = m->path == "plate_fused" ? femdev::assemble_plate_fused(m->dev, val_device, stream, t)
                   : m->path == "plate_lanes" ? femdev::assemble_plate_lanes(m->dev, val_device, stream, t)
                   : m->path == "plate_blocks" ? femdev::assemble_plate_blocks(m->dev, val_device, stream, t)
@@ -2393,12 +2396,12 @@ double fem_last_assembly_ms(fem_model* m) { return m && m->dev ? femdev::last_ms
 
 int fem_backward(fem_model* m, const double* dl_dk, double* dl_dparam_truss, double* dl_dparam_beam,
                  double* dl_dparam_plate, double* dl_dxyz, void* stream) {
-  return run_backward(m, 0, dl_dk, dl_dparam_truss, dl_dparam_beam, dl_dparam_plate, dl_dxyz, stream);
+  return run_backward(m, 0, dl_dk, dl_dparam_truss, dl_dparam_beam, dl_dparam_plate, dl_dxyz, stream, stream);
 }
 
 int fem_compliance_sensitivity(fem_model* m, const double* u, double* s_truss, double* s_beam, double* s_plate,
                                double* s_xyz, void* stream) {
-  return run_backward(m, 1, u, s_truss, s_beam, s_plate, s_xyz, stream);
+  return run_backward(m, 1, u, s_truss, s_beam, s_plate, s_xyz, stream, stream);
 }
 
 int fem_forward_backward(fem_model* m, double* val_device, const double* dl_dk, double* dl_dparam_truss,
@@ -2415,12 +2418,14 @@ int fem_forward_backward(fem_model* m, double* val_device, const double* dl_dk, 
   // the backward does not read the forward's values: both passes run at once
   auto e = femdev::stream_wait(m->side_stream, stream, m->fork_ev);
   if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
-  rc = run_backward(m, 0, dl_dk, dl_dparam_truss, dl_dparam_beam, dl_dparam_plate, dl_dxyz, m->side_stream);
-  if (rc) return rc;
-  rc = fem_assemble_into(m, val_device, stream);
-  if (rc) return rc;
-  e = femdev::stream_wait(stream, m->side_stream, m->join_ev);
-  return e.empty() ? FEM_OK : fail(m, FEM_ERR_DEVICE, e);
+  rc = run_backward(m, 0, dl_dk, dl_dparam_truss, dl_dparam_beam, dl_dparam_plate, dl_dxyz, m->side_stream, stream);
+  if (!rc) rc = fem_assemble_into(m, val_device, stream);
+  if (!rc) {
+    e = femdev::stream_wait(stream, m->side_stream, m->join_ev);
+    if (!e.empty()) rc = fail(m, FEM_ERR_DEVICE, e);
+  }
+  if (rc) femdev::note_use(m->dev, m->side_stream);  // not joined
+  return rc;
 }
 
 int fem_model_size(const fem_model* m, size_t* n_nodes, size_t* n_truss, size_t* n_beam, size_t* n_plate) {
@@ -2662,6 +2667,7 @@ int fem_element_forces(fem_model* m, const double* u_device, double* truss_out, 
   int rc = ensure_ready(m);
   if (rc) return rc;
   double* const out[3] = {truss_out, beam_out, plate_out};
+  femdev::note_use(m->dev, stream);
   auto e = femdev::element_forces(m->dev, u_device, out, stream);
   return e.empty() ? FEM_OK : fail(m, FEM_ERR_DEVICE, e);
 }

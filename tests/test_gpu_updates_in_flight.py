@@ -142,3 +142,69 @@ def test_captured_assembly_after_updates(gpu, name):
         m.assemble_into(eager)
         torch.cuda.synchronize()
         assert _same(eager, want), k
+
+
+def _keep_busy(stream, room):
+    """Queues some hundred milliseconds of copies on `stream`; the event after them."""
+    with torch.cuda.stream(stream):
+        for _ in range(120):
+            room.mul_(1.0)
+        return stream.record_event()
+
+
+def test_update_does_not_wait_for_other_work(gpu):
+    """An update waits for its own model's work, not for what other programs of the
+    process have queued.  Streams may share a hardware queue, in whose order
+    they then run: one of several streams has to be passed."""
+    case = CASES["lattice"]()
+    m = case.model(0)
+    m.stiffness_csr()
+    mine = torch.cuda.Stream()
+    out = torch.empty(m.csr_info()[1], dtype=torch.float64, device="cuda")
+    _update(m, case, 1, stream=mine)
+    xyz, props = case.data(2)
+    xyz, props = _cuda(xyz), _cuda(props[TRUSS])
+    room = torch.ones(1 << 29, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    passed = []
+    for _ in range(3):
+        other = torch.cuda.Stream()
+        m.assemble_into(out, stream=mine)
+        end = _keep_busy(other, room)
+        m.update_params(TRUSS, props, stream=mine)
+        m.update_nodes(xyz, stream=mine)
+        passed.append(not end.query())
+        torch.cuda.synchronize()
+    print("passed", passed, flush=True)
+    assert any(passed)
+
+
+@pytest.mark.parametrize("name", ["lattice", "frame", "shell", "plate"])
+def test_update_waits_for_its_own_model(gpu, name):
+    """An assembly still queued on another stream, eager or as a captured graph's
+    replay, has the values of before the update."""
+    case = CASES[name]()
+    print("case", name, flush=True)
+    m = case.model(0)
+    m.stiffness_csr()
+    m.set_option("time_assembly", 0)
+    mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+    out, replayed = (torch.zeros(m.csr_info()[1], dtype=torch.float64, device="cuda") for _ in range(2))
+    room = torch.ones(1 << 28, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    for k in (1, 2):
+        _keep_busy(other, room)
+        m.assemble_into(out, stream=other)
+        _update(m, case, k, stream=mine)
+        torch.cuda.synchronize()
+        assert _same(out, _want(case, k - 1)), k
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        m.assemble_into(replayed, stream=torch.cuda.current_stream())
+    for k in (3, 4):
+        _keep_busy(other, room)
+        with torch.cuda.stream(other):
+            graph.replay()
+        _update(m, case, k, stream=mine)
+        torch.cuda.synchronize()
+        assert _same(replayed, _want(case, k - 1)), k
