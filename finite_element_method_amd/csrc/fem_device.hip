@@ -292,10 +292,19 @@ std::string refresh_kept(Device* d, hipStream_t s) {
 
 }  // namespace
 
+bool capturing(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (!stream) return false;  // the null stream never is
+  if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess) {
+    (void)hipGetLastError();  // what is wrong with the stream shows at its first use
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 void note_use(Device* d, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (s && hipStreamIsCapturing(s, &status) == hipSuccess && status != hipStreamCaptureStatusNone) {
+  if (capturing(stream)) {
     d->captured = true;
     return;
   }

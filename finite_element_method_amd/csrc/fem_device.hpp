@@ -281,6 +281,7 @@ struct UpdateReport {
   uint32_t mixed = 0;
   double plate[4] = {0.0, 0.0, 0.0, 0.0};  // the first plate's parameters
 };
+bool capturing(void* stream);  // `stream` is being captured into a graph
 // note_use: `stream` is given work that reads coordinates, parameters, frames or
 // what the value path keeps of them; updates wait for such work.
 void note_use(Device* d, void* stream);

@@ -92,6 +92,7 @@ struct fem_model {
   // an update in place rewrites the device's coordinates or parameters: xyz,
   // params and coord_hash here are then behind until refresh_host
   bool xyz_behind = false, hash_behind = false, params_behind[3] = {false, false, false};
+  bool codes_behind = false;  // an update failed half way: so may rzero be
   ElementSet set[3];
   std::unordered_map<uint64_t, uint32_t> truss_pairs, beam_pairs;
   std::vector<std::vector<uint32_t>> node_plates;
@@ -180,6 +181,7 @@ void clear_model(fem_model* m, uint32_t nodes_number) {
   m->coord_hash.clear();
   m->xyz_behind = m->hash_behind = false;
   for (bool& b : m->params_behind) b = false;
+  m->codes_behind = false;
   for (auto& s : m->set) s = ElementSet();
   m->truss_pairs.clear();
   m->beam_pairs.clear();
@@ -1509,8 +1511,16 @@ int ensure_ready(fem_model* m) {
     }
     if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
     m->dirty = false;
+    m->codes_behind = false;
     m->pattern_valid = false;
     m->own_vals = false;
+  }
+  if (m->codes_behind) {
+    for (int t = 0; t < 3; ++t) {
+      auto e = femdev::fetch_codes(m->dev, t, m->rzero[t]);
+      if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
+    }
+    m->codes_behind = false;
   }
   if (!m->pattern_valid) {
     // a new pattern comes with a new (unwritten) values buffer
@@ -1685,16 +1695,23 @@ int run_backward(fem_model* m, int mode, const double* g, double* dp_truss, doub
   return e.empty() ? FEM_OK : fail(m, FEM_ERR_DEVICE, e);
 }
 
-// a frame code that an update changed changes the sparsity pattern
-int apply_report(fem_model* m, const femdev::UpdateReport& r) {
-  for (int t = 0; t < 3; ++t)
-    if (r.changed[t]) {
-      m->pattern_valid = false;
-      m->adj_valid = false;
-      auto e = femdev::fetch_codes(m->dev, t, m->rzero[t]);
-      if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
-    }
-  return FEM_OK;
+// After an update (e: its error, if any): a frame code that it changed changes the
+// sparsity pattern.  After an error the device may hold new codes that no later
+// update would report, so the codes are read again and the pattern is built anew.
+int apply_report(fem_model* m, const std::string& e, const femdev::UpdateReport& r) {
+  if (e.empty() && !r.changed[0] && !r.changed[1] && !r.changed[2]) return FEM_OK;
+  m->pattern_valid = false;
+  m->adj_valid = false;
+  m->codes_behind = true;
+  return e.empty() ? FEM_OK : fail(m, FEM_ERR_DEVICE, e);
+}
+
+// false (with a message): a captured update could not report, and the host could
+// not follow it
+bool update_allowed(fem_model* m, void* stream) {
+  if (!femdev::capturing(stream)) return true;
+  m->err = "an update cannot be captured into a graph: it reports to the host";
+  return false;
 }
 
 // ------------------------------------------------------------------ batches
@@ -2441,25 +2458,24 @@ double fem_last_backward_ms(fem_model* m) { return m && m->dev ? femdev::last_ba
 
 int fem_update_params(fem_model* m, int type, const double* params_device, void* stream) {
   if (!m || type < 0 || type > 2 || (!params_device && m->set[type].size())) return FEM_ERR_ARGUMENT;
+  if (!update_allowed(m, stream)) return FEM_ERR_DEVICE;
   int rc = ensure_ready(m);
   if (rc) return rc;
   femdev::UpdateReport rep;
   m->own_vals = false;
   m->params_behind[type] = m->set[type].size() != 0;
-  auto e = femdev::update_params(m->dev, type, params_device, stream, rep);
-  if (!e.empty()) return fail(m, FEM_ERR_DEVICE, e);
-  return apply_report(m, rep);
+  return apply_report(m, femdev::update_params(m->dev, type, params_device, stream, rep), rep);
 }
 
 int fem_update_nodes(fem_model* m, const double* xyz_device, void* stream) {
   if (!m || (!xyz_device && m->node_number.size())) return FEM_ERR_ARGUMENT;
+  if (!update_allowed(m, stream)) return FEM_ERR_DEVICE;
   int rc = ensure_ready(m);
   if (rc) return rc;
   femdev::UpdateReport rep;
   m->own_vals = false;
   m->xyz_behind = m->hash_behind = m->node_number.size() != 0;
-  auto e = femdev::update_nodes(m->dev, xyz_device, stream, rep);
-  return e.empty() ? apply_report(m, rep) : fail(m, FEM_ERR_DEVICE, e);
+  return apply_report(m, femdev::update_nodes(m->dev, xyz_device, stream, rep), rep);
 }
 
 int fem_add_displacements(fem_model* m, size_t n, const uint32_t* numbers, const int32_t* dofs, const double* values,

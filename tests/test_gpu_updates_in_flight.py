@@ -5,7 +5,7 @@ replayed after updates, a capture as the first call after an update."""
 import numpy as np
 import pytest
 
-from finite_element_method_amd import BEAM, FEM, PLATE, TRUSS, meshgen
+from finite_element_method_amd import BEAM, DeviceError, FEM, PLATE, TRUSS, meshgen
 from tests.test_gpu_bar_records import _chain, _load
 from tests.test_gpu_plate_frames import _turn, _vault
 
@@ -208,3 +208,38 @@ def test_update_waits_for_its_own_model(gpu, name):
         _update(m, case, k, stream=mine)
         torch.cuda.synchronize()
         assert _same(replayed, _want(case, k - 1)), k
+
+
+@pytest.mark.parametrize("name", ["frame", "shell", "plate"])
+def test_update_in_a_capture_is_refused(gpu, name):
+    """It changes nothing: the capture goes on, and the model is as it was, its
+    pattern included, until the next update."""
+    case = CASES[name]()
+    print("case", name, flush=True)
+    m = case.model(0)
+    m.stiffness_csr()
+    m.set_option("time_assembly", 0)
+    xyz, props = case.data(1)
+    xyz, props = _cuda(xyz), {t: _cuda(p) for t, p in props.items()}
+    eager, out = (torch.zeros(m.csr_info()[1], dtype=torch.float64, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(DeviceError, match="captured"):
+            m.update_nodes(xyz)
+        for t, p in props.items():
+            with pytest.raises(DeviceError, match="captured"):
+                m.update_params(t, p)
+        m.assemble_into(out, stream=torch.cuda.current_stream())
+    want = _want(case, 0)
+    for _ in range(2):
+        graph.replay()
+        m.assemble_into(eager)
+        torch.cuda.synchronize()
+        assert _same(out, want) and _same(eager, want)
+    _update(m, case, 1)
+    graph.replay()
+    m.assemble_into(eager)
+    torch.cuda.synchronize()
+    want = _want(case, 1)
+    assert _same(out, want) and _same(eager, want)
