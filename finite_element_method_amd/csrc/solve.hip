@@ -159,6 +159,12 @@ constexpr int SL_WINDOW = 1024;  // rows sorted together, by one workgroup
 // updates 4.47 vs 4.88; 7.7 M entries: 1.22 vs 1.16 ms, 50 updates 2.66 vs 2.64).
 constexpr int64_t SL_MIN_NNZ = 10000000;    // K_aa entries
 constexpr int SL_MIN_UPDATES = 16;          // updates asked for
+// Bytes per entry up to which the slices are taken.  A slice is as wide as its
+// longest row: a few long rows per window (hubs) cost all 64 lanes their length.
+// 10.3 bytes take 78 us where the CSR product takes 106, so the gain ends at
+// 14; a lattice with a hub of 400 bars among every 341 nodes would take some 50 bytes,
+// in time and in memory that the handle then keeps.
+constexpr size_t SL_MAX_BYTES = 14;
 constexpr uint32_t SL_NONE = 0xFFFFFFFFu;   // no row in this lane
 constexpr uint32_t SL_UNITS16 = 5, SL_UNITS32 = 6;  // 256-byte units of a pair of 64 lanes
 
@@ -1397,7 +1403,8 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
         if (host[S_DONE] != 0.0 || host[S_DONE + 1] != 0.0 || queued >= max_iter) break;
         if (slice && first) {
           std::memcpy(&slice_total, host + S_COUNT, sizeof(uint32_t));
-          if (!slices_fill(bufs, rp[0], ci[0], v[0], v_bytes, slice_total, s, sl)) sl.data = nullptr;
+          slice = size_t(slice_total) * 256 <= SL_MAX_BYTES * size_t(d->sep_nnz[0]);
+          if (slice && !slices_fill(bufs, rp[0], ci[0], v[0], v_bytes, slice_total, s, sl)) sl.data = nullptr;
         }
         batch = std::min(batch * 2, 64);
       }
