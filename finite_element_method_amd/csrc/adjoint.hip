@@ -99,7 +99,8 @@ __global__ __launch_bounds__(256) void adjoint_records_kernel(const uint32_t* __
   rec[2 * i + 1] = make_uint4(pos[4], pos[5], uint32_t(m), uint32_t(m >> 32));
 }
 
-// the same from the pattern's arrays (values past 32-bit positions have no records)
+// the same from the pattern's arrays, where there are no records (make_records;
+// values past 32-bit positions)
 __device__ inline void gather_block_far(const AdjArgs& A, uint32_t k, uint32_t a, double G[36]) {
   const uint64_t um = A.bmask[k];
 #pragma unroll
@@ -884,31 +885,46 @@ std::string upload_adjoint_maps(Device* d, const AdjointMaps& am) {
   if (!e.empty()) return e;
   e = dupload(d->adj_beams, am.beams.data(), am.beams.size());
   if (!e.empty()) return e;
-  // block records of beams, and of plates where the flat kernel does not serve
-  for (int t = 0; t < 3; ++t) {
-    const size_t pairs = am.bid[t].size();
-    const bool want = pairs && t != TRUSS && !(t == PLATE && am.flat) && uint64_t(d->nnz) < (uint64_t(1) << 32);
-    // without room for the records the kernels look blocks up in the pattern
-    if (!dalloc(d->adj_rec[t], want ? 2 * pairs : 0).empty()) {
-      (void)hipGetLastError();
-      d->adj_rec[t] = nullptr;
-    }
-    if (!d->adj_rec[t]) continue;
-    adjoint_records_kernel<<<unsigned((pairs + 255) / 256), 256>>>(d->conn[t], d->adj_bid[t], d->adj_bmask, d->adj_boff,
-                                                                   d->row_ptr,
-                                                                   t == BEAM ? reinterpret_cast<const uint4*>(d->adj_beams) : nullptr,
-                                                                   pairs, NODES_PER[t],
-                                                                   d->adj_rec[t]);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipDeviceSynchronize());
-  }
+  for (int t = 0; t < 3; ++t) (void)dalloc(d->adj_rec[t], 0);
+  d->adj_rec_made = false;
   d->adj_nxs = am.n_xs_rows;
   return dalloc(d->adj_xs, size_t(3 * am.n_xs_rows));
 }
 
+namespace {
+
+// Block records of beams, and of plates where the flat kernel does not serve, by
+// the first backward (compliance does not read them).  Without room for them, and
+// while the caller's stream is captured, the kernels look blocks up in the pattern.
+std::string make_records(Device* d, void* stream) {
+  if (d->adj_rec_made || capturing(stream)) return "";
+  for (int t : {BEAM, PLATE}) {
+    const size_t pairs = d->n_elem[t] * size_t(NODES_PER[t] * NODES_PER[t]);
+    if (!pairs || (t == PLATE && d->adj_flat) || uint64_t(d->nnz) >= (uint64_t(1) << 32)) continue;
+    if (!dalloc(d->adj_rec[t], 2 * pairs).empty()) {
+      (void)hipGetLastError();
+      d->adj_rec[t] = nullptr;
+      continue;
+    }
+    adjoint_records_kernel<<<unsigned((pairs + 255) / 256), 256>>>(
+        d->conn[t], d->adj_bid[t], d->adj_bmask, d->adj_boff, d->row_ptr,
+        t == BEAM ? reinterpret_cast<const uint4*>(d->adj_beams) : nullptr, pairs, NODES_PER[t], d->adj_rec[t]);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(nullptr));
+  }
+  d->adj_rec_made = true;
+  return "";
+}
+
+}  // namespace
+
 std::string run_adjoint(Device* d, int mode, const double* g, double* const dparam[3], double* dxyz, void* stream,
                         bool wide) {
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (mode == MODE_DLDK) {
+    auto e = make_records(d, stream);
+    if (!e.empty()) return e;
+  }
   HIP_TRY(hipEventRecord(d->ev2, s));
   for (int t = 0; t < 3; ++t) {
     const size_t n = d->n_elem[t];

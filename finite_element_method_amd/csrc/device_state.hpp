@@ -85,6 +85,7 @@ struct Device {
   uint32_t* adj_eorder = nullptr;  // flat plates: elements in Morton order
   uint32_t* adj_beams = nullptr;   // beams likewise, four words each: the beam, its nodes, 0
   uint4* adj_rec[3] = {nullptr, nullptr, nullptr};  // per (element, node pair): its block's CSR positions and mask
+  bool adj_rec_made = false;       // made (or left out for want of room) for these maps
   double* adj_xs = nullptr;
   int64_t adj_xoff[3] = {0, 0, 0};
   int64_t adj_nxs = 0;

@@ -46,3 +46,27 @@ def test_compliance_makes_no_records(gpu, kind):
     assert records >= record - slack and maps <= both - record + slack
     assert all(torch.equal(a, b) for a, b in zip(_bits(second), _bits(models[1].backward(g, xyz=xyz))))
     assert all(torch.equal(a, b) for a, b in zip(_bits(first), _bits(models[1].compliance_sensitivity(u, xyz=xyz))))
+
+
+@pytest.mark.parametrize("kind", ["shell", "frame", "plate"])
+def test_first_backward_in_a_capture(gpu, kind):
+    """After a compliance call the first backward may be captured: it makes no
+    records then (nothing is allocated), and its replays have the eager call's bits."""
+    mesh = {"shell": lambda: _vault(11, 6, 3, _turn()), "frame": lambda: meshgen.beam_frame(5, 4, 3, seed=4),
+            "plate": lambda: meshgen.plate_grid(9, 5, seed=5)}[kind]()
+    xyz = kind != "frame"
+    m = FEM.from_mesh(mesh)
+    m.build_pattern()
+    g = torch.randn(m.csr_info()[1], dtype=torch.float64, device="cuda")
+    u = torch.randn(6 * mesh.n_nodes, dtype=torch.float64, device="cuda")
+    m.compliance_sensitivity(u, xyz=xyz)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = m.backward(g, xyz=xyz)
+    for _ in range(3):
+        g.copy_(torch.randn_like(g))
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = [t.clone() for t in _bits(out)]
+        assert all(torch.equal(a, b) for a, b in zip(replayed, _bits(m.backward(g, xyz=xyz))))
