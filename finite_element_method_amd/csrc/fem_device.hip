@@ -532,6 +532,8 @@ std::string upload_generic(Device* d, const GenericMaps& g) {
 
 void set_generic_block(Device* d, int threads) { d->gen_block = threads; }
 
+bool sums_contributions(const Device* d) { return !d->pn_waves; }
+
 std::string assemble_generic(Device* d, double* val, void* stream, bool timed) {
   if (d->pn_waves) return assemble_plate_frames(d, val, stream, timed);
   hipStream_t s = static_cast<hipStream_t>(stream);

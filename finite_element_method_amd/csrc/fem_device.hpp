@@ -216,6 +216,7 @@ double last_ms(Device* d);
 // plate kernel (0 = one per patch); block size of the generic kernels
 std::string set_plate_grid(Device* d, int wg_per_cu);
 void set_generic_block(Device* d, int threads);
+bool sums_contributions(const Device* d);  // "generic" through the contribution kernels, which take that block size
 
 // Batched assembly helpers (batch.hip)
 struct Graph;

@@ -2910,7 +2910,7 @@ int fem_batch_autotune(fem_batch* b) {
             if (rc) return rc;
             if (ms < best_ms) { best_ms = ms; cfg = {pn, wg, 256}; }
           }
-        } else if (g->path == "bar_owner" || g->path == "plate_lanes") {
+        } else if (g->path == "bar_owner" || g->path == "plate_lanes" || !femdev::sums_contributions(g->dev)) {
           cfg = {pn, g->pf_wg_per_cu, 256};  // fixed workgroup shape
         } else {
           for (int bs : {128, 256, 512}) {
@@ -2950,9 +2950,10 @@ int fem_batch_autotune(fem_batch* b) {
       if (!e.empty()) return batch_fail(b, FEM_ERR_DEVICE, e);
       b->config += "group " + std::to_string(k) + ": " + g->path + " wg_per_cu=" + std::to_string(best[k][1]) + "; ";
     } else {
-      if (g->path == "generic") femdev::set_generic_block(g->dev, best[k][2]);
+      const bool block = g->path == "generic" && femdev::sums_contributions(g->dev);
+      if (block) femdev::set_generic_block(g->dev, best[k][2]);
       b->config += "group " + std::to_string(k) + ": " + g->path +
-                   (g->path == "generic" ? " block=" + std::to_string(best[k][2]) : std::string()) + "; ";
+                   (block ? " block=" + std::to_string(best[k][2]) : std::string()) + "; ";
     }
   }
   if (best_schedule < 0) {

@@ -306,7 +306,7 @@ const char* fem_batch_last_error(const fem_batch* b);
 int fem_batch_size(const fem_batch* b, size_t* n_meshes, size_t* n_groups);
 /* Times candidate launch shapes per group (row-staging plate kernel: owned
  * nodes per patch and resident workgroups per CU; block-lane plate kernels:
- * workgroups per CU; generic path: block size) and the schedule of the groups
+ * workgroups per CU; contribution kernels: block size) and the schedule of the groups
  * (concurrent graph branches, or one after another on one stream) on whole
  * graph replays, keeps the fastest and captures the graph.  Results are cached
  * per (gfx architecture, batch signature) for the life of the process and in a
