@@ -323,15 +323,16 @@ struct SolveResult {
   double residual = 0.0, stop = 0.0;
 };
 // wide: the update loop's SpMV reads four values per lane and step with 16-byte range-checked loads
-// when K_aa's values span under 4 GiB
+// when K_aa's values span under 4 GiB.  plain: four launches per update and the CSR product at every size
+// (the same bits)
 std::string solve_pcg(Device* d, int precond, int max_iter, double rel_tol, double abs_tol, void* stream,
-                      SolveResult& res, bool wide = true);
+                      SolveResult& res, bool wide = true, bool plain = false);
 // The same solve with every work buffer in one static device array of
 // STATIC_SCRATCH_BYTES per GPU (no allocation); u_a (n_aa) and r_r (n_bb) are
 // caller device memory.  The model's stored solution is not changed.
 constexpr size_t STATIC_SCRATCH_BYTES = size_t(64) << 20;
 std::string solve_pcg_static(Device* d, int precond, int max_iter, double rel_tol, double abs_tol, void* stream,
-                             double* u_a, double* r_r, SolveResult& res, bool wide = true);
+                             double* u_a, double* r_r, SolveResult& res, bool wide = true, bool plain = false);
 std::string solution(Device* d, const double** u_a, const double** r_r, int64_t* n_aa, int64_t* n_bb);
 double last_solve_ms(Device* d);
 

@@ -112,6 +112,7 @@ struct fem_model {
                           // 3 = balanced lanes (plate_lanes; falls back to plate_blocks)
   bool force_generic = false;
   bool wide_loads = true;  // backward block gathers and PCG SpMV: 16-byte loads when the values fit 32-bit offsets
+  bool pcg_plain = false;  // PCG: four launches per update and the CSR product at every size
   bool time_assembly = true;  // events around each assembly launch (fem_last_assembly_ms)
   int pl_order = 0;  // balanced-lane plate patches: 0 = automatic, 1 = node-index order, 2 = Morton order
   // node-pair blocks of the pattern (kept for the adjoint maps): node a owns
@@ -2594,7 +2595,8 @@ int fem_solve_pcg(fem_model* m, int preconditioner, uint64_t max_iter, void* str
     return fail(m, FEM_ERR_ARGUMENT, "preconditioner must be 0 (Jacobi) or 1 (node-block Jacobi)");
   if (max_iter > uint64_t(INT32_MAX)) return fail(m, FEM_ERR_ARGUMENT, "max_iter too large");
   femdev::SolveResult r;
-  auto e = femdev::solve_pcg(m->dev, preconditioner, int(max_iter), m->rel_tol, m->abs_tol, stream, r, m->wide_loads);
+  auto e = femdev::solve_pcg(m->dev, preconditioner, int(max_iter), m->rel_tol, m->abs_tol, stream, r, m->wide_loads,
+                             m->pcg_plain);
   if (!e.empty()) {
     const bool numeric = e.rfind("PCG", 0) == 0;
     return fail(m, numeric ? FEM_ERR_VALIDATION : FEM_ERR_DEVICE, e);
@@ -2613,7 +2615,7 @@ int fem_solve_pcg_noalloc(fem_model* m, int preconditioner, uint64_t max_iter, d
   if (max_iter > uint64_t(INT32_MAX)) return fail(m, FEM_ERR_ARGUMENT, "max_iter too large");
   femdev::SolveResult r;
   auto e = femdev::solve_pcg_static(m->dev, preconditioner, int(max_iter), m->rel_tol, m->abs_tol, stream, u_a, r_r,
-                                    r, m->wide_loads);
+                                    r, m->wide_loads, m->pcg_plain);
   if (!e.empty()) {
     const bool numeric = e.rfind("PCG", 0) == 0;
     const bool limit = e.find("static scratch") != std::string::npos || e.find("device buffers") != std::string::npos;
@@ -2731,6 +2733,9 @@ int fem_set_option(fem_model* m, const char* key, int64_t value) {
     return FEM_OK;  // speed only; the pattern stays
   } else if (k == "wide_loads") {
     m->wide_loads = value != 0;
+    return FEM_OK;  // speed only
+  } else if (k == "pcg_plain") {
+    m->pcg_plain = value != 0;
     return FEM_OK;  // speed only
   } else if (k == "time_assembly") {
     // 0: no events around the assembly launches (two fewer packets between

@@ -584,8 +584,8 @@ __global__ void sv_start_jacobi(const double* __restrict__ b, const double* __re
     r[i] = bi;
     z[i] = zi;
     p[i] = zi;
-    ra += bi * zi;
-    rb += bi * bi;
+    ra = __builtin_fma(bi, zi, ra);
+    rb = __builtin_fma(bi, bi, rb);
   }
   block_partials(ra, rb, part_a, part_b);
 }
@@ -604,8 +604,8 @@ __global__ void sv_update_jacobi(const double* __restrict__ d, const double* __r
     r[i] = ri;
     const double zi = ri / d[i];
     z[i] = zi;
-    ra += ri * zi;
-    rb += ri * ri;
+    ra = __builtin_fma(ri, zi, ra);
+    rb = __builtin_fma(ri, ri, rb);
   }
   block_partials(ra, rb, part_a, part_b);
 }
@@ -1232,7 +1232,7 @@ bool slices_fill(SolveBuffers& bufs, const int64_t* rp, const int32_t* ci, const
 
 // the solve proper: b, preconditioner, PCG updates, r_r, into `bufs`
 std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, double abs_tol, hipStream_t s,
-                       SolveResult& res, bool wide, SolveBuffers& bufs) {
+                       SolveResult& res, bool wide, bool plain, SolveBuffers& bufs) {
   res = SolveResult();
   const int64_t na = d->sep_rows[0], nb = d->sep_rows[2];
   const size_t una = size_t(std::max<int64_t>(na, 1)), unb = size_t(std::max<int64_t>(nb, 1));
@@ -1274,7 +1274,7 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
   // partials: (r, z), (r, r) and p.Ap.  b is not read after the start (it holds n
   // values, at least one per block): it takes the third set, or with two launches
   // per update, whose three sets fit `part`, the other direction
-  const bool fused = quad && na <= FU_N;
+  const bool fused = quad && !plain && na <= FU_N;
   constexpr int FU_PARTS = 2 * SV_PARTS / 3;
   double *pa = part, *pb = part + (fused ? FU_PARTS : SV_PARTS), *pc = fused ? part + 2 * FU_PARTS : b;
   double stop = 0.0;
@@ -1282,7 +1282,7 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
   bool conv = false;
   // a small system: one block inverse per dof is room enough, so the number of
   // node blocks stays on the device, and so do the tolerance and the updates
-  if (quad && na > 0 && na <= SM_N && d->sep_nnz[0] <= SM_NNZ &&
+  if (quad && !plain && na > 0 && na <= SM_N && d->sep_nnz[0] <= SM_NNZ &&
       bufs.room() >= una * (36 * sizeof(double) + sizeof(int32_t)) + 4096) {
     uint32_t* count = nullptr;
     if (precond == 0) {
@@ -1366,7 +1366,7 @@ std::string solve_core(Device* d, int precond, int max_iter, double rel_tol, dou
       const unsigned spmv_blocks = grid_for(na * (quad ? SPMV_QUAD_LANES : SPMV_LANES), B);
       double* p_other = b;
       Slices sl;
-      bool slice = quad && !fused && bufs.grows() && d->sep_nnz[0] >= SL_MIN_NNZ && max_iter >= SL_MIN_UPDATES;
+      bool slice = quad && !plain && !fused && bufs.grows() && d->sep_nnz[0] >= SL_MIN_NNZ && max_iter >= SL_MIN_UPDATES;
       uint32_t slice_total = 0;
       int queued = 0, batch = 1;
       for (;;) {
@@ -1459,13 +1459,13 @@ struct ModelBuffers : SolveBuffers {
 }  // namespace
 
 std::string solve_pcg(Device* d, int precond, int max_iter, double rel_tol, double abs_tol, void* stream,
-                      SolveResult& res, bool wide) {
+                      SolveResult& res, bool wide, bool plain) {
   d->sol_done = false;
   if (!d->sep_done) return "no separation computed";
   if (!d->sol_host) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&d->sol_host), 16 * sizeof(double)));
   ModelBuffers bufs(d);
   bufs.host = d->sol_host;
-  auto e = solve_core(d, precond, max_iter, rel_tol, abs_tol, static_cast<hipStream_t>(stream), res, wide, bufs);
+  auto e = solve_core(d, precond, max_iter, rel_tol, abs_tol, static_cast<hipStream_t>(stream), res, wide, plain, bufs);
   if (!e.empty()) return e;
   d->sol_na = d->sep_rows[0];
   d->sol_nb = d->sep_rows[2];
@@ -1521,7 +1521,7 @@ struct StaticBuffers : SolveBuffers {
 }  // namespace
 
 std::string solve_pcg_static(Device* d, int precond, int max_iter, double rel_tol, double abs_tol, void* stream,
-                             double* u_a, double* r_r, SolveResult& res, bool wide) {
+                             double* u_a, double* r_r, SolveResult& res, bool wide, bool plain) {
   if (!d->sep_done) return "no separation computed";
   if ((!u_a && d->sep_rows[0]) || (!r_r && d->sep_rows[2])) return "u_a and r_r must be device buffers";
   void* base = nullptr;
@@ -1533,7 +1533,7 @@ std::string solve_pcg_static(Device* d, int precond, int max_iter, double rel_to
   bufs.r_r = r_r;
   double host[S_COUNT + 1];
   bufs.host = host;
-  return solve_core(d, precond, max_iter, rel_tol, abs_tol, static_cast<hipStream_t>(stream), res, wide, bufs);
+  return solve_core(d, precond, max_iter, rel_tol, abs_tol, static_cast<hipStream_t>(stream), res, wide, plain, bufs);
 }
 
 std::string solution(Device* d, const double** u_a, const double** r_r, int64_t* n_aa, int64_t* n_bb) {

@@ -359,6 +359,11 @@ int fem_batch_mesh_csr_to_host(fem_batch* b, size_t mesh, int64_t* row_ptr, int3
  *                        paths taken above 4 GiB).  Gradients are bitwise
  *                        equal either way; PCG iterates differ by rounding (the
  *                        SpMV sums a row in another order)
+ *   "pcg_plain"          0 (default) = fem_solve_pcg takes kernels by the size
+ *                        of K_aa (one workgroup for all updates, two launches per
+ *                        update, four with the product on K_aa in slices); 1 =
+ *                        four launches per update and the CSR product at
+ *                        every size.  Bitwise equal solutions
  *   "time_assembly"      1 (default) = events around every assembly launch
  *                        for fem_last_assembly_ms; 0 = none (two fewer
  *                        packets between back-to-back launches)
