@@ -919,9 +919,9 @@ std::string make_records(Device* d, void* stream) {
 }  // namespace
 
 std::string run_adjoint(Device* d, int mode, const double* g, double* const dparam[3], double* dxyz, void* stream,
-                        bool wide) {
+                        bool wide, bool records) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (mode == MODE_DLDK) {
+  if (mode == MODE_DLDK && records) {
     auto e = make_records(d, stream);
     if (!e.empty()) return e;
   }
@@ -944,7 +944,7 @@ std::string run_adjoint(Device* d, int mode, const double* g, double* const dpar
     A.eorder = d->adj_eorder;
     A.beams = reinterpret_cast<const uint4*>(d->adj_beams);
     A.row_ptr = d->row_ptr;
-    A.rec = d->adj_rec[t];
+    A.rec = records ? d->adj_rec[t] : nullptr;
     A.dparam = dparam[t];
     A.xs = (dxyz && t != BEAM) ? d->adj_xs : nullptr;
     A.xpos = d->adj_xpos + d->adj_xoff[t];

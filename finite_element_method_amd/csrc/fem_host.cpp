@@ -112,6 +112,7 @@ struct fem_model {
                           // 3 = balanced lanes (plate_lanes; falls back to plate_blocks)
   bool force_generic = false;
   bool wide_loads = true;  // backward block gathers and PCG SpMV: 16-byte loads when the values fit 32-bit offsets
+  bool adjoint_records = true;  // backward: gradient blocks through their records
   bool pcg_plain = false;  // PCG: four launches per update and the CSR product at every size
   bool time_assembly = true;  // events around each assembly launch (fem_last_assembly_ms)
   int pl_order = 0;  // balanced-lane plate patches: 0 = automatic, 1 = node-index order, 2 = Morton order
@@ -1692,7 +1693,7 @@ int run_backward(fem_model* m, int mode, const double* g, double* dp_truss, doub
   if (rc) return rc;
   double* dp[3] = {dp_truss, dp_beam, dp_plate};
   femdev::note_use(m->dev, called);
-  auto e = femdev::run_adjoint(m->dev, mode, g, dp, dxyz, stream, m->wide_loads);
+  auto e = femdev::run_adjoint(m->dev, mode, g, dp, dxyz, stream, m->wide_loads, m->adjoint_records);
   return e.empty() ? FEM_OK : fail(m, FEM_ERR_DEVICE, e);
 }
 
@@ -2733,6 +2734,9 @@ int fem_set_option(fem_model* m, const char* key, int64_t value) {
     return FEM_OK;  // speed only; the pattern stays
   } else if (k == "wide_loads") {
     m->wide_loads = value != 0;
+    return FEM_OK;  // speed only
+  } else if (k == "adjoint_records") {
+    m->adjoint_records = value != 0;
     return FEM_OK;  // speed only
   } else if (k == "pcg_plain") {
     m->pcg_plain = value != 0;

@@ -359,6 +359,12 @@ int fem_batch_mesh_csr_to_host(fem_batch* b, size_t mesh, int64_t* row_ptr, int3
  *                        paths taken above 4 GiB).  Gradients are bitwise
  *                        equal either way; PCG iterates differ by rounding (the
  *                        SpMV sums a row in another order)
+ *   "adjoint_records"    1 (default) = the backward of beams, and of plates in
+ *                        frames of their own, reads gradient blocks through
+ *                        records; 0 = through the pattern's arrays (the way taken
+ *                        past 2^32 values, without room for the records, and
+ *                        where the first backward is captured).  Bitwise equal
+ *                        gradients
  *   "pcg_plain"          0 (default) = fem_solve_pcg takes kernels by the size
  *                        of K_aa (one workgroup for all updates, two launches per
  *                        update, four with the product on K_aa in slices); 1 =

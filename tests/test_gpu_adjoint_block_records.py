@@ -70,3 +70,19 @@ def test_first_backward_in_a_capture(gpu, kind):
         torch.cuda.synchronize()
         replayed = [t.clone() for t in _bits(out)]
         assert all(torch.equal(a, b) for a, b in zip(replayed, _bits(m.backward(g, xyz=xyz))))
+
+
+@pytest.mark.parametrize("kind,size", [("shell", (1, 1)), ("shell", (5, 3)), ("shell", (17, 4)), ("vault", (5, 3)),
+                                       ("vault", (8, 2)), ("frame", (2, 1, 1)), ("frame", (5, 4, 3)),
+                                       ("frame", (9, 7, 8))])
+def test_without_records(gpu, kind, size):
+    """Blocks through the pattern's arrays (full and partial masks): the bits of those through the records."""
+    mesh = meshgen.beam_frame(*size, seed=6) if kind == "frame" else _vault(*size, 7, _turn() if kind == "shell" else None)
+    xyz = kind != "frame"
+    print("case", kind, size, flush=True)
+    m = FEM.from_mesh(mesh)
+    m.build_pattern()
+    g = torch.randn(m.csr_info()[1], dtype=torch.float64, device="cuda")
+    want = _bits(m.backward(g, xyz=xyz))
+    m.set_option("adjoint_records", 0)
+    assert all(torch.equal(a, b) for a, b in zip(_bits(m.backward(g, xyz=xyz)), want))
