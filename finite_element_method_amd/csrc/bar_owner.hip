@@ -132,7 +132,7 @@ __device__ inline void truss_constants(const BarArgs& A, size_t e, int p, double
 // An element's constants (beam: R (9), the scales of the rank-one terms u, v and
 // w, tu, tv, tw, and |b_p|; truss: r (3), k_pp, k_pq; truss.rs:132-189,
 // beam.rs:495-605).  One record serves both ends: with a copy per end (and the
-// pattern's words in it, 160 bytes) the 64 x 64 x 64 frame read 248 MB of
+// pattern's words in it, 160 bytes) the 64 x 64 x 64 frame holds 248 MB of
 // constants, here 99 MB and 31 MB of entries.
 __device__ inline void form_record(const BarArgs& A, uint32_t u, double* __restrict__ rec) {
   const int type = int(u >> 31);
@@ -274,10 +274,12 @@ __device__ inline void write_row(BarLds& L, const uint4& w, int i, int r0, const
 
 // One workgroup per range of owned nodes: one lane per (owned node, row) forms
 // the rows in LDS, element records loaded two entries ahead; then consecutive
-// lanes write the range out.  Bound: latency and LDS traffic at the three
-// workgroups per CU that the staged rows leave room for, close to the bytes
-// (64 x 64 x 64 frame: 86 us; 261 MB out and 130 MB in take 66 us at fill and
-// read rate).
+// lanes write the range out.  Bound: memory.  The 64 x 64 x 64 frame writes its
+// 261 MB of values and reads 222 MB, of which 130 MB are records and entries
+// once; the rest are those of elements whose other end lies in a range far away,
+// read again.  98 us, 4.9 TB/s, the rate of a large copy (the compulsory bytes
+// alone would take 66); called over and over on the same buffers, whose second
+// reads the last-level cache then serves, 75 us.  LDS is busy 54 %, VALU 44 %.
 __global__ __launch_bounds__(BO_THREADS) void bar_owner_kernel(BarArgs A) {
   __shared__ BarLds L;
   const int t = threadIdx.x;
@@ -402,12 +404,16 @@ __device__ inline void put_entry(Lds& L, int sl, const TrussEntry& E) {
 // in insertion order from the first contribution, off-diagonal blocks written
 // by their one element).  Entries come through 48-byte element records and the
 // pattern's words, as the bar kernel's (a chain of look-ups per entry and 37 loads
-// per wave before: 40 x 40 x 40 lattice 43.9 -> 39.5 us per call).  Off-diagonal
+// per wave before; launches back to back in a graph: 11 x 11 x 11 lattice 8.6 ->
+// 4.95 us with the smaller ranges, 40 x 40 x 40 36.1 -> 29.5).  Whole calls of small
+// meshes are bound by the host's part, 12.5 to 18 us from process to process.  An
+// update of the areas forms the records anew, and with its assembly takes 32 us for
+// the small lattice (49 before there were any) and 68 for the large.  Off-diagonal
 // rows: one task per (row, entry), so that consecutive lanes write neighbouring
 // blocks of one row.  Diagonal rows: one lane per (owned node, row 0..2).
 //   STAGED: an entry per lane at most, rows staged in LDS and written as
-//   16-byte chunks; four workgroups per CU.  Latency-bound meshes gain (11 x 11 x
-//   11 lattice 14.2 -> 12.9 us per call, 26 x 26 x 26 18.1 -> 16.8).
+//   16-byte chunks; four workgroups per CU (26 x 26 x 26 lattice 9.5 -> 8.7 us back
+//   to back; 11 x 11 x 11 4.85 -> 4.95).
 //   Otherwise rows straight to the CSR, five workgroups per CU; TWO: some range
 //   has more entries than lanes, the loads of a lane's two in flight together.
 template <bool TWO, bool STAGED>

@@ -1355,16 +1355,18 @@ std::string build_pattern(fem_model* m) {
       };
       // A small mesh is cut into more ranges than these limits ask for, so that
       // its chain of loads has fewer entries per lane: truss lattices up to 512
-      // ranges of 4 nodes or more (64 nodes: 16.4 -> 13.7 us per call, 2744: 17.0
-      // -> 15.0, 8000: 17.2 -> 16.6; with 1000 ranges the larger ones lose, 17576
-      // nodes 20.2 -> 21.4), frames up to 128 of 8 or more (512 nodes: 14.6 ->
-      // 13.7; at 8000 and more the full ranges are as fast).
+      // ranges of 4 nodes or more (launches back to back in a graph, 64 nodes: 5.2
+      // -> 4.4 us, 1331: 5.35 -> 4.95, 4913: 5.85 -> 5.6, 8000: as fast; with 1000
+      // ranges the larger ones lose, 4913 nodes 6.0, 17576 9.6 against 8.7), frames
+      // up to 128 of 8 or more (64 nodes: 6.5 -> 5.95, 1000: 6.9 -> 6.1; from 2744
+      // on the full ranges are as fast).
       auto few = [&](uint32_t least, size_t ranges) { return std::max(least, uint32_t((N + ranges - 1) / ranges)); };
       std::vector<uint32_t> truss_ranges;
       // Truss ranges are cut for the kernel that stages its rows (half the
       // entries) where that leaves no more than fit the chip at once, four per
-      // CU; else to the full limits for the one that does not (24389 nodes, 1219
-      // half ranges: 22.2 us against 19.5; 17576 nodes: 16.8 against 18.1).
+      // CU; else to the full limits for the one that does not (back to back, 24389
+      // nodes in 1388 half ranges: 15.0 us against 11.1; 17576 nodes: 8.7 against
+      // 9.5; up to 8000 nodes, cut alike either way, staging costs 0.1 to 0.2).
       auto cut = [&](bool staged) {
         bm.ranges.clear();
         truss_ranges.clear();

@@ -336,7 +336,8 @@ int fem_batch_mesh_csr_to_host(fem_batch* b, size_t mesh, int64_t* row_ptr, int3
  *                        per owned node-pair block (plate_blocks), 0 = row
  *                        staging (plate_fused), 2 = one lane per element
  *                        corner (plate_corners); bitwise equal values
- *   "plate_patch_order"  patches of the balanced-lane kernel: 0 = automatic
+ *   "plate_patch_order"  patches of the balanced-lane kernel and of the kernel
+ *                        for plates in frames of their own: 0 = automatic
  *                        (node-index order unless it scatters the patches'
  *                        elements, then Morton order), 1 = node-index order,
  *                        2 = Morton order; bitwise equal values
