@@ -538,12 +538,19 @@ class FEM:
 
     @staticmethod
     def _update_stream(stream, values):
-        """An update without a stream runs on torch's current one, where its values were made."""
-        if stream is None:
-            import torch
+        """The update's stream: torch's current one, where its values were made, or the
+        given one, which then waits for them."""
+        import torch
 
-            stream = torch.cuda.current_stream(values.device)
-        return _stream_handle(stream)
+        current = torch.cuda.current_stream(values.device)
+        if stream is None:
+            return _stream_handle(current)
+        handle = _stream_handle(stream)
+        if (handle.value or 0) != current.cuda_stream:
+            other = torch.cuda.ExternalStream(handle.value, device=values.device) if handle.value else \
+                torch.cuda.default_stream(values.device)
+            other.wait_stream(current)
+        return handle
 
     def update_params(self, etype, params, stream=None):
         """Replaces one element type's parameters (float64 CUDA tensor, add_* layout)."""

@@ -243,3 +243,30 @@ def test_update_in_a_capture_is_refused(gpu, name):
     torch.cuda.synchronize()
     want = _want(case, 1)
     assert _same(out, want) and _same(eager, want)
+
+
+@pytest.mark.parametrize("name", ["lattice", "shell", "plate"])
+def test_update_waits_for_its_values(gpu, name):
+    """Values made on torch's current stream, as the last of much other work, and
+    the copy that a transposed tensor needs: the update's own stream waits for both."""
+    case = CASES[name]()
+    print("case", name, flush=True)
+    m = case.model(0)
+    m.stiffness_csr()
+    maker, mine = torch.cuda.Stream(), torch.cuda.Stream()
+    out = torch.zeros(m.csr_info()[1], dtype=torch.float64, device="cuda")
+    room = torch.ones(1 << 28, dtype=torch.float64, device="cuda")
+    for k, stream in ((1, mine), (2, None), (3, mine.cuda_stream), (4, 0)):
+        xyz, props = case.data(k)
+        xyz, props = _cuda(xyz), {t: _cuda(p.T) for t, p in props.items()}
+        torch.cuda.synchronize()
+        _keep_busy(maker, room)
+        with torch.cuda.stream(maker):
+            made = {t: p * 1.0 for t, p in props.items()}
+            for t, p in made.items():
+                m.update_params(t, p.t(), stream=stream)
+            _keep_busy(maker, room)
+            m.update_nodes(xyz * 1.0, stream=stream)
+        m.assemble_into(out)
+        torch.cuda.synchronize()
+        assert _same(out, _want(case, k)), k
