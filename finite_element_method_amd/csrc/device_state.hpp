@@ -13,6 +13,12 @@ struct UpdateReport;
 // parameters in a form of its own: formed with its maps and by every update
 enum class Kept { NONE, PLATE_SLOTS, FRAME_SLOTS, BAR_RECORDS };
 
+// balanced-lane plate slots: their stride in doubles, and E, nu, k where every plate's are the same
+struct PlateLaneHead {
+  double mat[3];
+  uint32_t stride;
+};
+
 struct Device {
   hipStream_t stream = nullptr;
   int dev = 0;
@@ -53,9 +59,9 @@ struct Device {
   uint32_t *pl_nodes = nullptr, *pl_lanes = nullptr, *pl_lane_set = nullptr;
   double* pl_geo = nullptr;   // per wave element slot: local coordinates and parameters
   // every plate has the same E, nu and k (bitwise): the slots hold t only and
-  // the three values go to the kernel as arguments
+  // the three values sit in the head
   bool pl_uniform = false;
-  double pl_mat[3] = {0.0, 0.0, 0.0};
+  PlateLaneHead* pl_head = nullptr;
   // maps of plates in frames of their own (generic path of plate-only meshes);
   // pn_waves == 0: the generic path sums element contributions
   int pn_waves = 0;

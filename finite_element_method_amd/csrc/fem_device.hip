@@ -72,7 +72,7 @@ void destroy_device(Device* d) {
   f(d->sep_rp); f(d->sep_sum); f(d->sep_ci); f(d->sep_dpos);
   f(d->pb_hdr); f(d->pb_conn); f(d->pb_eid); f(d->pb_blk);
   f(d->pn_eid); f(d->pn_nodes); f(d->pn_wave); f(d->pn_lanes); f(d->pn_geo);
-  f(d->pl_nodes); f(d->pl_lanes); f(d->pl_lane_set); f(d->pl_geo);
+  f(d->pl_nodes); f(d->pl_lanes); f(d->pl_lane_set); f(d->pl_geo); f(d->pl_head);
   for (int k = 0; k < 6; ++k) f(d->sol_vec[k]);
   f(d->sol_rr); f(d->sol_rb); f(d->sol_part); f(d->sol_s); f(d->sol_diag); f(d->sol_inv); f(d->sol_flag);
   f(d->sol_bid); f(d->sol_starts); f(d->sol_tmp); f(d->u_glob);
@@ -242,13 +242,11 @@ __global__ void copy_plate_params_kernel(const double* __restrict__ src, size_t 
   if (k != 2 && __double_as_longlong(v) != __double_as_longlong(src[k])) words[UPD_MIXED] = number;
 }
 
-// the words, and the first plate's parameters, to pinned host memory
-__global__ void report_kernel(const uint32_t* __restrict__ words, const double* __restrict__ plate, UpdateReport* out,
-                              uint32_t number) {
+// the words to pinned host memory
+__global__ void report_kernel(const uint32_t* __restrict__ words, UpdateReport* out, uint32_t number) {
   const int t = threadIdx.x;
   if (t < 3) out->changed[t] = words[UPD_CHANGED + t] == number;
   if (t == 3) out->mixed = words[UPD_MIXED] == number;
-  if (t >= 4 && t < 8 && plate) out->plate[t - 4] = plate[t - 4];
 }
 
 namespace {
@@ -271,7 +269,7 @@ std::string begin_update(Device* d, hipStream_t s) {
 }
 
 std::string end_update(Device* d, hipStream_t s, UpdateReport& out) {
-  report_kernel<<<1, 64, 0, s>>>(d->upd_words, d->n_elem[PLATE] ? d->params[PLATE] : nullptr, d->upd_report, d->upd_number);
+  report_kernel<<<1, 64, 0, s>>>(d->upd_words, d->upd_report, d->upd_number);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(s));
   d->n_used = 0;
@@ -335,8 +333,7 @@ std::string update_params(Device* d, int type, const double* src, void* stream, 
   // flat plates: the slots' layout follows the parameters; they were filled in
   // the layout of before, which as a rule stays
   const bool same = d->pl_uniform == !out.mixed;
-  const double mat[3] = {out.plate[0], out.plate[1], out.plate[3]};
-  set_plate_lane_material(d, !out.mixed, mat);
+  set_plate_lane_material(d, !out.mixed);
   if (same) return "";
   if (!(e = plate_lanes_gather(d, s)).empty()) return e;
   HIP_TRY(hipStreamSynchronize(s));

@@ -128,7 +128,7 @@ struct PlateLaneMaps {
 std::string upload_plate_lane_maps(Device* d, const PlateLaneMaps& pm);
 // E, nu and k shared by every plate (uniform) or per element: the slot layout (8
 // or 10 doubles) that the next filling of the slots takes
-void set_plate_lane_material(Device* d, bool uniform, const double mat[3]);
+void set_plate_lane_material(Device* d, bool uniform);
 std::string assemble_plate_lanes(Device* d, double* val, void* stream, bool timed = true);
 
 // Plates with frames of their own (plate_frames.hip): meshes of plates only in
@@ -281,7 +281,6 @@ double last_backward_ms(Device* d);
 struct UpdateReport {
   uint32_t changed[3] = {0, 0, 0};
   uint32_t mixed = 0;
-  double plate[4] = {0.0, 0.0, 0.0, 0.0};  // the first plate's parameters
 };
 bool capturing(void* stream);  // `stream` is being captured into a graph
 // note_use: `stream` is given work that reads coordinates, parameters, frames or

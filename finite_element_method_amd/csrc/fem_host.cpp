@@ -698,9 +698,9 @@ bool build_plate_block_maps(fem_model* m, const std::vector<uint64_t>& bptr, con
   return flush();
 }
 
-// true when every plate has the same E, nu and k, bit for bit (into mat); the
-// balanced-lane slots then hold t only
-bool plate_material_uniform(const fem_model* m, double mat[3]) {
+// true when every plate has the same E, nu and k, bit for bit; the balanced-lane
+// slots then hold t only
+bool plate_material_uniform(const fem_model* m) {
   const auto& S = m->set[PLATE];
   if (!S.size()) return false;
   const double* P = S.params.data();
@@ -709,7 +709,6 @@ bool plate_material_uniform(const fem_model* m, double mat[3]) {
     const double v[3] = {P[4 * e], P[4 * e + 1], P[4 * e + 3]};
     if (std::memcmp(v, first, sizeof(v)) != 0) return false;
   }
-  for (int k = 0; k < 3; ++k) mat[k] = first[k];
   return true;
 }
 
@@ -1288,8 +1287,7 @@ std::string build_pattern(fem_model* m) {
       femdev::PlateBlockMaps pbm;
       femdev::PlateLaneMaps plm;
       if (m->pf_kernel == 3 && build_plate_lane_maps(m, bptr, blocks, row_ptr, plm)) {
-        double mat[3];
-        femdev::set_plate_lane_material(m->dev, plate_material_uniform(m, mat), mat);
+        femdev::set_plate_lane_material(m->dev, plate_material_uniform(m));
         e = femdev::upload_plate_lane_maps(m->dev, plm);
         if (!e.empty()) return e;
         m->path = "plate_lanes";

@@ -53,7 +53,9 @@ constexpr int PL_LDS = PL_ELEMS * PL_REC > PL_STAGE_VALUES ? PL_ELEMS * PL_REC :
 static_assert(PL_STAGE_VALUES % 2 == 0 && PL_STAGE_VALUES >= PL_NODES * (13 * PL_MAX_NB + 2), "staging");
 
 // Everything a wave reads sits at fixed offsets from its index, so all its
-// loads issue at once: no load waits for another's result.
+// loads issue at once: no load waits for another's result (but the slots' for
+// the head, a scalar load that the whole chip shares; as launch arguments stride and
+// material would stay, in a captured launch, what they were when it was captured).
 struct LaneArgs {
   const double* __restrict__ geo;    // per wave PL_ELEMS slots of PL_GEO doubles
   // per wave PL_NODES: CSR position of row 6a of owned node s,
@@ -62,9 +64,8 @@ struct LaneArgs {
   const uint2* __restrict__ lanes;   // 64 lane descriptors per distinct set
   const uint32_t* __restrict__ lane_set;  // per wave: its descriptor set
   double* __restrict__ val;
+  const PlateLaneHead* __restrict__ head;  // the slots' stride, and E, nu, k when they are uniform
   uint32_t val_bytes;
-  uint32_t geo_stride;  // PL_GEO, or PL_GEO_U when E, nu, k are uniform (then in mat)
-  double mat[3];
 };
 
 // inputs of wave patch w: the lane's descriptor, owned node (l mod 16) and
@@ -73,13 +74,14 @@ __device__ inline void load_patch(const LaneArgs& A, uint32_t w, int l, int le, 
                                   double2& g1, double2& g2, double2& g3, double2& g4) {
   desc = A.lanes[size_t(A.lane_set[w]) * 64 + l];
   nd = A.nodes[size_t(w) * PL_NODES + (l & (PL_NODES - 1))];
-  const double2* gs = reinterpret_cast<const double2*>(A.geo + (size_t(w) * PL_ELEMS + le) * A.geo_stride);
+  const uint32_t stride = A.head->stride;
+  const double2* gs = reinterpret_cast<const double2*>(A.geo + (size_t(w) * PL_ELEMS + le) * stride);
   g0 = gs[0];
   g1 = gs[1];
   g2 = gs[2];
-  if (A.geo_stride == PL_GEO_U) {  // (E, nu) and (t, k) from the uniform values
-    g3 = make_double2(A.mat[0], A.mat[1]);
-    g4 = make_double2(gs[3].x, A.mat[2]);
+  if (stride == PL_GEO_U) {  // (E, nu) and (t, k) from the uniform values
+    g3 = make_double2(A.head->mat[0], A.head->mat[1]);
+    g4 = make_double2(gs[3].x, A.head->mat[2]);
   } else {
     g3 = gs[3];
     g4 = gs[4];
@@ -89,13 +91,18 @@ __device__ inline void load_patch(const LaneArgs& A, uint32_t w, int l, int le, 
 // Fills the wave slots' geometry: local coordinates of nodes 1, 2, 4 about
 // node 3 (the same differences the crate's plate frame takes, quad:340-378,
 // with an identity frame) and the element parameters (t only when E, nu and k
-// are uniform: stride PL_GEO_U).
+// are uniform: stride PL_GEO_U); and the head.
 __global__ __launch_bounds__(256) void plate_lanes_gather_kernel(const double* __restrict__ xyz,
                                                                  const double* __restrict__ params,
                                                                  const uint32_t* __restrict__ sconn,
                                                                  const uint32_t* __restrict__ seid, size_t n_slots,
-                                                                 int stride, double* __restrict__ geo) {
+                                                                 int stride, double* __restrict__ geo,
+                                                                 PlateLaneHead* __restrict__ head) {
   const size_t i = blockIdx.x * size_t(blockDim.x) + threadIdx.x;
+  if (i == 0) {
+    head->stride = uint32_t(stride);
+    for (int k = 0; k < 3; ++k) head->mat[k] = params[k < 2 ? k : 3];
+  }
   if (i >= n_slots) return;
   const uint32_t eid = seid[i];
   double* g = geo + i * stride;
@@ -384,7 +391,8 @@ std::string plate_lanes_gather(Device* d, hipStream_t s) {
   if (n_slots) {
     plate_lanes_gather_kernel<<<unsigned((n_slots + 255) / 256), 256, 0, s>>>(d->xyz, d->params[PLATE], d->pb_conn,
                                                                             d->pb_eid, n_slots,
-                                                                            d->pl_uniform ? PL_GEO_U : PL_GEO, d->pl_geo);
+                                                                            d->pl_uniform ? PL_GEO_U : PL_GEO, d->pl_geo,
+                                                                            d->pl_head);
     HIP_TRY(hipGetLastError());
   }
   return "";
@@ -399,6 +407,7 @@ std::string upload_plate_lane_maps(Device* d, const PlateLaneMaps& pm) {
   if (!(e = dupload(d->pl_lanes, pm.lanes.data(), pm.lanes.size())).empty()) return e;
   if (!(e = dupload(d->pl_lane_set, pm.lane_set.data(), pm.lane_set.size())).empty()) return e;
   if (!(e = dalloc(d->pl_geo, size_t(pm.n_waves) * PL_ELEMS * PL_GEO)).empty()) return e;  // either layout fits
+  if (!(e = dalloc(d->pl_head, 1)).empty()) return e;
   e = plate_lanes_gather(d, nullptr);
   if (!e.empty()) return e;
   d->kept = Kept::PLATE_SLOTS;
@@ -406,10 +415,7 @@ std::string upload_plate_lane_maps(Device* d, const PlateLaneMaps& pm) {
   return "";
 }
 
-void set_plate_lane_material(Device* d, bool uniform, const double mat[3]) {
-  d->pl_uniform = uniform;
-  for (int k = 0; k < 3; ++k) d->pl_mat[k] = uniform ? mat[k] : 0.0;
-}
+void set_plate_lane_material(Device* d, bool uniform) { d->pl_uniform = uniform; }
 
 std::string assemble_plate_lanes(Device* d, double* val, void* stream, bool timed) {
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -420,8 +426,7 @@ std::string assemble_plate_lanes(Device* d, double* val, void* stream, bool time
     a.nodes = reinterpret_cast<const uint2*>(d->pl_nodes);
     a.lanes = reinterpret_cast<const uint2*>(d->pl_lanes);
     a.lane_set = d->pl_lane_set;
-    a.geo_stride = uint32_t(d->pl_uniform ? PL_GEO_U : PL_GEO);
-    for (int k = 0; k < 3; ++k) a.mat[k] = d->pl_mat[k];
+    a.head = d->pl_head;
     a.val = val;
     a.val_bytes = uint32_t(d->nnz * 8);
     plate_lanes_kernel<<<d->pl_waves, 64, 0, s>>>(a);

@@ -174,10 +174,7 @@ double fem_last_backward_ms(fem_model* m);
  * not re-validated.  Frames are recomputed; if a frame's zero pattern changes
  * the sparsity pattern is rebuilt by the next assembly.  The update has finished
  * when the call returns: calls on any stream then read the new values, and so do
- * replays of captured ones while the pattern stays.  Exception: a captured
- * assembly of flat plates ("plate_lanes") with E, nu and k the same for every
- * plate holds these three as launch arguments; capture it again when an update
- * changes them or makes them differ.  The update reads the caller's values on
+ * replays of captured ones while the pattern stays.  The update reads the caller's values on
  * `stream` and waits for it; where the model was used on another stream since its last update, or in a
  * captured call, it waits for the device first.  Not to be captured. */
 int fem_update_params(fem_model* m, int type, const double* params_device, void* stream);

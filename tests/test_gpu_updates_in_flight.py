@@ -66,10 +66,11 @@ CASES = {
 
 
 class _Mixing(_Meshed):
-    """Plates of one material in even variants, of several in odd ones."""
+    """Plates of one material in even variants, another in each, and of several in odd ones."""
 
     def data(self, k):
         xyz, props = super().data(k)
+        props[PLATE][:, [0, 1]] *= [1.0 + 0.5 * k, 1.0 + 0.1 * k]
         if k % 2:
             props[PLATE][3::5, 0] *= 1.5
         return xyz, props
@@ -78,6 +79,10 @@ class _Mixing(_Meshed):
 def _materials(mesh):
     mesh.props[:, 0] *= np.random.default_rng(6).uniform(0.5, 2.0, mesh.n_elements)
     return mesh
+
+
+def _case(name):
+    return CASES[name]() if name in CASES else _Mixing(meshgen.plate_grid(23, 17, seed=7), PLATE, 2)
 
 
 def _update(m, case, k, stream=None):
@@ -98,7 +103,7 @@ def _same(a, b):
 @pytest.mark.parametrize("name", sorted(CASES) + ["plate_mixing"])
 def test_two_streams_after_an_update(gpu, name):
     """The update has finished when it returns: assemblies on any stream see it."""
-    case = CASES[name]() if name in CASES else _Mixing(meshgen.plate_grid(23, 17, seed=7), PLATE, 2)
+    case = _case(name)
     print("case", name, flush=True)
     m = case.model(0)
     m.stiffness_csr()
@@ -114,12 +119,11 @@ def test_two_streams_after_an_update(gpu, name):
         assert all(_same(o, want) for o in out), k
 
 
-@pytest.mark.parametrize("name", sorted(CASES))
+@pytest.mark.parametrize("name", sorted(CASES) + ["plate_mixing"])
 def test_captured_assembly_after_updates(gpu, name):
-    """A captured assembly replays with the values of the last update (E, nu and k
-    of flat plates apart, which stay here as they were); a capture as the first
-    call after an update leaves the eager calls as they are."""
-    case = CASES[name]()
+    """A captured assembly replays with the values of the last update; a capture as
+    the first call after an update leaves the eager calls as they are."""
+    case = _case(name)
     print("case", name, flush=True)
     m = case.model(0)
     m.stiffness_csr()
